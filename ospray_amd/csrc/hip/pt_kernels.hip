@@ -337,14 +337,13 @@ __global__ __launch_bounds__(256) void k_generate(DFrame F, DPaths P)
 }
 
 // Work distribution of the traversal kernels: each wave takes batches of
-// `size` (64 unless the queue is short) consecutive queue entries
-// (neighbouring pixels' rays, which share node fetches) with one atomic
-// per batch, until the queue is exhausted.
-__device__ __forceinline__ int nextBatch(int32_t *counter, int size = 64)
+// 64 consecutive queue entries (neighbouring pixels' rays, which share node
+// fetches) with one atomic per batch, until the queue is exhausted.
+__device__ __forceinline__ int nextBatch(int32_t *counter)
 {
   int base = 0;
   if (laneId() == 0)
-    base = atomicAdd(counter, size);
+    base = atomicAdd(counter, 64);
   return __shfl(base, 0);
 }
 
@@ -373,11 +372,15 @@ constexpr int kExtendRefill = HPT_EXTEND_REFILL, kShadowRefill = HPT_SHADOW_REFI
 // finish(ended, entry, best, occluded, state) runs on every lane of the
 // wave (`ended` on the lanes whose ray ended), so it may use wave-wide
 // appends.  A queue shorter than 64 entries per wave of the grid (the
-// last bounces' few paths) is spread over every wave instead: each wave
-// takes one batch of ceil(n / waves) entries and no more, so the few rays
+// last bounces' few paths) is spread over every wave instead: wave w owns
+// the ceil(n / waves) entries from w * ceil(n / waves) on, so the few rays
 // run in many waves side by side rather than 64 to a wave (where each
 // round waits for the slowest of 64 node fetches and the longest of 64
-// rays sets the wave's time).  Each ray's traversal is the one traceRay
+// rays sets the wave's time).  Their place follows from the wave's index,
+// not from a fetch: the atomics of one address are served one by one (10 ns
+// each between the XCDs), so the 6144 waves of the default grid fetching one
+// batch each held every launch back by 61 us, whatever its ray count (a
+// 64x64 frame 1385 -> 650 us, 641x359 at 2 spp and 21 bounces 7.1 -> 4.7 ms).  Each ray's traversal is the one traceRay
 // runs: the result does not depend on which rays share a wave.
 template <int MODE, bool STATS, bool RECORD, int TIES, int REFILL, class Load, class Finish>
 __device__ __forceinline__ void traceQueue(const DScene &S, const uint32_t *queue, int n, int32_t *fetch, uint32_t *lds,
@@ -388,7 +391,8 @@ __device__ __forceinline__ void traceQueue(const DScene &S, const uint32_t *queu
   const int waves = (int)((gridDim.x * blockDim.x) >> 6);
   const bool spread = HPT_SPREAD_SHORT_QUEUES && n < 64 * waves;
   const int bCap = spread ? (n + waves - 1) / waves : 64; // entries per batch, 1..64
-  int bBase = nextBatch(fetch, bCap), bNext = 0; // wave-uniform batch cursor
+  // wave-uniform batch cursor; a spread queue's batches are the waves' own
+  int bBase = spread ? (globalId() >> 6) * bCap : nextBatch(fetch), bNext = 0;
   uint32_t bEntry = wl < bCap && bBase + wl < n ? queue[bBase + wl] : 0u;
   TraceState s;
   s.cur = kTraceDone;
@@ -1156,9 +1160,15 @@ __global__ __launch_bounds__(kTraceBlock) void k_shadow_trans(DScene S, DFrame F
   uint32_t *ovf = P.overflow + (size_t)globalId() * kThreadRow;
   TraceStats st = {0, 0};
   uint32_t rays = 0;
-  for (int base = nextBatch(&P.counters[kCntFetchTrans]); base < n; base = nextBatch(&P.counters[kCntFetchTrans])) {
+  // Wave w owns the entries from w * per on, `per` <= 64 of them at a time:
+  // most bounces queue fewer records than there are waves, and a fetch by
+  // every wave serialises (see traceQueue).  641x359 at 2 spp, 21 launches:
+  // 1263 us with a fetch, 4.7 -> 4.0 ms per frame.
+  const int waves = gridStride() >> 6;
+  const int per = min((n + waves - 1) / waves, 64);
+  for (int base = (globalId() >> 6) * per; base < n; base += waves * per) {
     const int i = base + laneId();
-    if (i >= n)
+    if (laneId() >= per || i >= n)
       continue;
     const uint32_t r = P.transQueue[i];
     const float4 o4 = ld4(P.recOrg + 4 * (size_t)r);
@@ -1605,11 +1615,10 @@ inline int gridFor(size_t n, int block, int maxBlocks)
 extern "C" {
 
 namespace {
-// counter masks: the shadow side of a bounce (records, transparency queue and
-// their work fetch) and the extension side of the bounce reading queue q
+// counter masks: the shadow side of a bounce (records, their work fetch and
+// the transparency queue) and the extension side of the bounce reading queue q
 // (the next queue's pair, the extension work fetch, the near-tie queue)
-constexpr uint32_t kShadowSideMask =
-    (1u << kCntShadow) | (1u << kCntFetchShadow) | (1u << kCntTrans) | (1u << kCntFetchTrans);
+constexpr uint32_t kShadowSideMask = (1u << kCntShadow) | (1u << kCntFetchShadow) | (1u << kCntTrans);
 inline uint32_t extensionSideMask(int q)
 {
   return (3u << (2 * (q ^ 1))) | (1u << kCntFetchExtend) | (1u << kCntTies);

@@ -274,12 +274,11 @@ constexpr int kCntShadow = 4; // shadow-ray records
 constexpr int kCntFetchExtend = 5; // work fetch of the extension traversal
 constexpr int kCntFetchShadow = 6; // work fetch of the shadow traversal
 constexpr int kCntTrans = 7; // records for the transparency pass
-constexpr int kCntFetchTrans = 8; // work fetch of the transparency pass
-constexpr int kCntTies = 9; // extension rays whose closest hit has a near-tie
-constexpr int kNumBounceCounters = 10; // the counters above are reset every bounce
-constexpr int kCntNrcQuery = 10; // radiance-cache queries of the pass
-constexpr int kCntNrcTrain = 11; // radiance-cache training records of the pass
-constexpr int kNumCounters = 12;
+constexpr int kCntTies = 8; // extension rays whose closest hit has a near-tie
+constexpr int kNumBounceCounters = 9; // the counters above are reset every bounce
+constexpr int kCntNrcQuery = 9; // radiance-cache queries of the pass
+constexpr int kCntNrcTrain = 10; // radiance-cache training records of the pass
+constexpr int kNumCounters = 11;
 
 // path flags in ld[3]
 constexpr uint32_t FLAG_DEPTH_MASK = 0xffu; // bits 0-7

@@ -57,3 +57,35 @@ def test_queue_batching_renders_the_same_frame(hip_device):
     assert np.array_equal(base[0], ofb.channel(K.OSP_FB_COLOR))
     for arr, ch in zip(base[1:], (K.OSP_FB_DEPTH, K.OSP_FB_ID_PRIMITIVE, K.OSP_FB_ID_INSTANCE)):
         assert np.array_equal(arr, ofb.channel(ch), equal_nan=True), ch
+
+
+def _glass_scene():
+    # every instance glass, so that shadow rays through them fill the
+    # transparency queue: more than 64 entries per wave with one traversal
+    # block per CU (512 waves), fewer than one per wave with 64
+    sc = scenes.c1(width=256, height=144, spp=4, grid=97, instances=160)
+    for i in range(1, len(sc.materials)):
+        sc.materials[i] = {"type": "glass", "eta": 1.5}
+    return sc
+
+
+@pytest.mark.parametrize("bpc", [1, 12, 64])
+def test_transparency_queue_of_any_length(hip_device, bpc):
+    """Wave w of the transparency pass owns the entries from w * per on, in
+    strides of waves * per: the frame equals the oracle's whatever the number
+    of waves (no recorded hit is skipped or replayed twice)."""
+    L = K.lib()
+    dev = L.ospGetCurrentDevice()
+    A.set_device_param(dev, "traceBlocksPerCU", bpc)
+    L.ospDeviceCommit(dev)
+    try:
+        sc = _glass_scene()
+        s = scenes.to_ospray(sc)
+        fb = A.framebuffer(sc.width, sc.height, K.OSP_FB_RGBA32F, CH)
+        A.render(fb, s.renderer, s.camera, s.world)
+        got = A.map_color(fb, sc.width, sc.height, K.OSP_FB_RGBA32F)
+    finally:
+        A.set_device_param(dev, "traceBlocksPerCU", 12)
+        L.ospDeviceCommit(dev)
+    ofb, _, _ = orc.render_scene(sc, frames=1, fmt=K.OSP_FB_RGBA32F, channels=CH)
+    assert np.array_equal(got, ofb.channel(K.OSP_FB_COLOR))
