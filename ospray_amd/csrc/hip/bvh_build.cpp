@@ -1,4 +1,4 @@
-// Binned-SAH BVH builder (host) producing 4-wide hpt::DNode4 nodes.
+// Binned-SAH BVH builder (host) producing 4-wide hpt::BNode4 nodes.
 #include "bvh_build.h"
 
 #include <algorithm>
@@ -193,7 +193,7 @@ BuildResult buildBVH(const std::vector<BuildBox> &boxes, int maxLeaf, int nthrea
   R.order.resize(boxes.size());
   for (size_t i = 0; i < boxes.size(); i++)
     R.order[i] = (uint32_t)i;
-  DNode4 emptyNode;
+  BNode4 emptyNode;
   for (int c = 0; c < 4; c++) {
     emptyNode.lox[c] = emptyNode.hix[c] = kInfF;
     emptyNode.loy[c] = emptyNode.hiy[c] = kInfF;
@@ -283,7 +283,7 @@ BuildResult buildBVH(const std::vector<BuildBox> &boxes, int maxLeaf, int nthrea
   const auto root = resolve(-1, 0);
   R.bounds = get(root.first, root.second).box;
   using Ref = std::pair<int, int32_t>;
-  auto setChild = [&](DNode4 &n, int c, const TNode &t) {
+  auto setChild = [&](BNode4 &n, int c, const TNode &t) {
     n.lox[c] = t.box.lo[0];
     n.loy[c] = t.box.lo[1];
     n.loz[c] = t.box.lo[2];
@@ -300,7 +300,7 @@ BuildResult buildBVH(const std::vector<BuildBox> &boxes, int maxLeaf, int nthrea
   };
   const TNode &r0 = get(root.first, root.second);
   if (r0.left < 0) {
-    DNode4 n = emptyNode;
+    BNode4 n = emptyNode;
     setChild(n, 0, r0);
     n.child[0] = leafCode(r0.first, r0.count);
     R.nodes.push_back(n);
@@ -342,7 +342,7 @@ BuildResult buildBVH(const std::vector<BuildBox> &boxes, int maxLeaf, int nthrea
     }
     const int need = e.need + (nk - 1);
     R.stackNeed = std::max(R.stackNeed, need);
-    DNode4 n = emptyNode;
+    BNode4 n = emptyNode;
     int32_t slot[4] = {-1, -1, -1, -1};
     for (int c = 0; c < nk; c++) {
       const TNode &ch = get(kids[c].first, kids[c].second);

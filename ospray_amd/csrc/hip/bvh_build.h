@@ -1,5 +1,5 @@
 // Host-side BVH construction for the hip device: a binned-SAH binary tree
-// over primitive boxes, collapsed into 4-wide nodes (hpt::DNode4, 128 B) by
+// over primitive boxes, collapsed into 4-wide nodes (hpt::BNode4, 128 B) by
 // repeatedly opening the child of largest surface area, emitted in
 // depth-first order so a subtree is contiguous in HBM.  The reference gets its BVHs from
 // Embree (rtcCommitScene, modules/cpu/common/Group.cpp:129-142,
@@ -21,7 +21,7 @@ struct BuildBox
 
 struct BuildResult
 {
-  std::vector<DNode4> nodes; // node 0 is the root
+  std::vector<BNode4> nodes; // node 0 is the root
   std::vector<uint32_t> order; // item ids in leaf order
   BuildBox bounds;
   int maxDepth = 0; // depth of the binary tree

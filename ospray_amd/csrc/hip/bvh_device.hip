@@ -34,6 +34,7 @@
 
 namespace {
 
+using hpt::BNode4;
 using hpt::DNode4;
 using hpt::DPrim;
 
@@ -497,7 +498,7 @@ struct CollapseArgs
   uint32_t n;
   const Geo *geos;
   int ng;
-  DNode4 *nodes;
+  BNode4 *nodes;
   DPrim *prims;
   uint32_t *counters; // [0] next-level entries, [1] nodes allocated, [2] largest stack need
 };
@@ -535,7 +536,7 @@ __global__ __launch_bounds__(kBlock) void k_collapse(CollapseArgs A, const Entry
   }
   const int need = E.need + nk - 1;
   atomicMax(&A.counters[2], (uint32_t)need);
-  DNode4 N;
+  BNode4 N;
   for (int c = 0; c < 4; c++) {
     N.lox[c] = N.hix[c] = N.loy[c] = N.hiy[c] = N.loz[c] = N.hiz[c] = kInfF;
     N.child[c] = (int32_t)~0u;
@@ -565,24 +566,70 @@ __global__ __launch_bounds__(kBlock) void k_collapse(CollapseArgs A, const Entry
   A.nodes[E.out] = N;
 }
 
-__global__ __launch_bounds__(kBlock) void k_relocate(DNode4 *dst, const DNode4 *src, size_t n, int32_t nodeOff,
-    uint32_t primOff)
+// the largest q with p + q s <= lo, the smallest with p + q s >= hi (both
+// exist in 0..255); the products and sums are exact in double for any floats
+// of comparable size, and within 2^-53 otherwise
+__device__ __forceinline__ uint32_t gridBelow(double p, double s, double lo)
+{
+  int q = s > 0.0 ? min(255, max(0, (int)floor((lo - p) / s))) : 0;
+  while (q > 0 && p + q * s > lo)
+    q--;
+  return (uint32_t)q;
+}
+__device__ __forceinline__ uint32_t gridAbove(double p, double s, double hi)
+{
+  int q = s > 0.0 ? min(255, max(0, (int)ceil((hi - p) / s))) : 0;
+  while (q < 255 && p + q * s < hi)
+    q++;
+  return (uint32_t)q;
+}
+
+// One axis of a node: the grid over the children's bounds and their planes.
+__device__ __forceinline__ void gridAxis(const float lo[4], const float hi[4], const bool used[4], float &p, float &s,
+    uint32_t &qlo, uint32_t &qhi)
+{
+  float a = kInfF, b = -kInfF;
+  for (int c = 0; c < 4; c++)
+    if (used[c]) {
+      a = fminf(a, lo[c]);
+      b = fmaxf(b, hi[c]);
+    }
+  p = a <= b ? a : 0.f;
+  s = a <= b ? (float)(((double)b - a) / 255.0) : 0.f;
+  if (a <= b && (double)p + 255.0 * (double)s < (double)b) // rounded down
+    s = fmaxf(s * 1.0000002f, 1.17549435e-38f);
+  qlo = qhi = 0;
+  for (int c = 0; c < 4; c++)
+    if (used[c]) {
+      qlo |= gridBelow(p, s, lo[c]) << (8 * c);
+      qhi |= gridAbove(p, s, hi[c]) << (8 * c);
+    }
+}
+
+__global__ __launch_bounds__(kBlock) void k_relocate(DNode4 *dst, const BNode4 *src, size_t n, int32_t nodeOff,
+    uint32_t primOff, int32_t unusedRef)
 {
   const size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x;
   if (i >= n)
     return;
-  DNode4 N = src[i];
+  const BNode4 B = src[i];
+  DNode4 N;
+  bool used[4];
   for (int c = 0; c < 4; c++) {
-    if (N.lox[c] == kInfF) // unused slot: never entered
-      continue;
-    const int32_t ch = N.child[c];
-    if (ch >= 0) {
+    used[c] = B.lox[c] != kInfF;
+    const int32_t ch = B.child[c];
+    if (!used[c]) {
+      N.child[c] = unusedRef;
+    } else if (ch >= 0) {
       N.child[c] = ch + nodeOff;
     } else {
       const uint32_t enc = ~(uint32_t)ch;
       N.child[c] = (int32_t) ~((((enc >> 3) + primOff) << 3) | (enc & 7u));
     }
   }
+  gridAxis(B.lox, B.hix, used, N.p[0], N.s[0], N.lox, N.hix);
+  gridAxis(B.loy, B.hiy, used, N.p[1], N.s[1], N.loy, N.hiy);
+  gridAxis(B.loz, B.hiz, used, N.p[2], N.s[2], N.loz, N.hiz);
   dst[i] = N;
 }
 
@@ -752,7 +799,7 @@ HPT_API hipError_t hpt_bvh_build(const HptBvhGeometry *geoms, int numGeoms, int 
   HPT_TRY(hipMemcpyAsync(qa, &rootEntry, sizeof(Entry), hipMemcpyHostToDevice, s));
   const uint32_t initCounters[4] = {0u, 1u, 0u, 0u};
   HPT_TRY(hipMemcpyAsync(counters, initCounters, 16, hipMemcpyHostToDevice, s));
-  CollapseArgs A = {lo, hi, left, right, count, vals, n, dgeo, numGeoms, (DNode4 *)outNodes, (DPrim *)outPrims,
+  CollapseArgs A = {lo, hi, left, right, count, vals, n, dgeo, numGeoms, (BNode4 *)outNodes, (DPrim *)outPrims,
       counters};
   uint32_t nin = 1;
   int levels = 0;
@@ -780,12 +827,12 @@ HPT_API hipError_t hpt_bvh_build(const HptBvhGeometry *geoms, int numGeoms, int 
 }
 
 HPT_API hipError_t hpt_bvh_relocate(void *dst, const void *src, size_t n, int32_t nodeOffset, uint32_t primOffset,
-    hipStream_t s)
+    int32_t unusedRef, hipStream_t s)
 {
   if (n == 0)
     return hipSuccess;
-  k_relocate<<<(unsigned)((n + kBlock - 1) / kBlock), kBlock, 0, s>>>((DNode4 *)dst, (const DNode4 *)src, n,
-      nodeOffset, primOffset);
+  k_relocate<<<(unsigned)((n + kBlock - 1) / kBlock), kBlock, 0, s>>>((DNode4 *)dst, (const BNode4 *)src, n,
+      nodeOffset, primOffset, unusedRef);
   return hipGetLastError();
 }
 

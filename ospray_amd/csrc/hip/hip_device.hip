@@ -749,11 +749,11 @@ struct Light : public ManagedObject
 };
 
 // BLAS of one list of geometries (shared by groups with the same list):
-// built on the device (nodes and records in dNodes/dPrims) or, as the
-// fallback, on the host (nodes/prims)
+// built on the device or on the host, the build nodes and primitive records
+// in dNodes/dPrims (of a host build from nodes/prims, once a world needs it)
 struct Blas
 {
-  std::vector<hpt::DNode4> nodes;
+  std::vector<hpt::BNode4> nodes;
   std::vector<hpt::DPrim> prims;
   DevBuf dNodes, dPrims;
   bool onDevice = false;
@@ -1962,15 +1962,15 @@ static std::shared_ptr<Blas> buildBlasDevice(HipDevice &D, const std::vector<Geo
   auto B = std::make_shared<Blas>();
   DevBuf ws, nodes;
   ws.ensure(hpt_bvh_workspace_bytes(n));
-  nodes.ensure(n * sizeof(hpt::DNode4));
+  nodes.ensure(n * sizeof(hpt::BNode4));
   B->dPrims.ensure(n * sizeof(hpt::DPrim));
   HptBvhResult r;
   HIP_CHECK(hpt_bvh_build(hg.data(), (int)hg.size(), D.bvhRadius, ws.ptr, ws.bytes, nodes.ptr, B->dPrims.ptr,
       D.bvhHostWords(), &r, D.stream));
   if (r.stackNeed > kDeviceBlasStackLimit)
     return nullptr;
-  B->dNodes.ensure((size_t)r.numNodes * sizeof(hpt::DNode4));
-  HIP_CHECK(hipMemcpyAsync(B->dNodes.ptr, nodes.ptr, (size_t)r.numNodes * sizeof(hpt::DNode4), hipMemcpyDeviceToDevice,
+  B->dNodes.ensure((size_t)r.numNodes * sizeof(hpt::BNode4));
+  HIP_CHECK(hipMemcpyAsync(B->dNodes.ptr, nodes.ptr, (size_t)r.numNodes * sizeof(hpt::BNode4), hipMemcpyDeviceToDevice,
       D.stream));
   HIP_CHECK(hipStreamSynchronize(D.stream));
   B->onDevice = true;
@@ -2053,6 +2053,16 @@ static std::shared_ptr<Blas> buildBlasHost(const std::vector<Geometry *> &geoms)
     throw std::runtime_error("too many geometric models in one group");
   B->buildMs = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
   return B;
+}
+
+// largest |coordinate| of a box, 0 of an empty one
+static float boxExtent(const hpt::BuildBox &b)
+{
+  float e = 0.f;
+  if (b.lo[0] <= b.hi[0])
+    for (int k = 0; k < 3; k++)
+      e = std::max(e, std::max(std::fabs(b.lo[k]), std::fabs(b.hi[k])));
+  return e;
 }
 
 void World::commit() // World.cpp:70-188 plus the Group BLAS builds (Group.cpp:93-143)
@@ -2164,9 +2174,11 @@ void World::commit() // World.cpp:70-188 plus the Group BLAS builds (Group.cpp:9
   if (media.size() >= (1u << 12))
     throw std::runtime_error("too many glass materials in one world");
 
-  // concatenate BLAS nodes and primitives
+  // concatenate BLAS nodes and primitives; record 0 is a degenerate triangle
+  // that no ray hits, the leaf of the nodes' unused slots
   std::vector<int> blasNodeOff(uniqueBlas.size()), blasPrimOff(uniqueBlas.size());
-  size_t nNodes = 0, nPrims = 0;
+  size_t nNodes = 0, nPrims = 1;
+  constexpr int32_t kNoPrim = ~0; // ~(0 << 3 | 1 - 1)
   maxDepth = 0;
   int blasStackNeed = 0;
   for (size_t k = 0; k < uniqueBlas.size(); k++) {
@@ -2195,6 +2207,7 @@ void World::commit() // World.cpp:70-188 plus the Group BLAS builds (Group.cpp:9
     di.blasRoot = blasNodeOff[blasSlot[&B]];
     di.modelOffset = groupModelOffset[gi];
     di.userID = I.userID;
+    di.extent = boxExtent(B.bounds);
     di.epsScale = hpt::maxf(std::fabs(x[0]), hpt::maxf(std::fabs(x[4]), std::fabs(x[8])));
     hpt::BuildBox wb;
     for (int k = 0; k < 3; k++) {
@@ -2232,58 +2245,52 @@ void World::commit() // World.cpp:70-188 plus the Group BLAS builds (Group.cpp:9
   for (size_t k = 0; k < T.order.size(); k++)
     tlasOrder[k] = tlasInst[T.order[k]];
   const int tlasOff = (int)nNodes;
-  auto remap = [](hpt::DNode4 n, int nodeOff, int primOff, const std::vector<uint32_t> *order) {
-    for (int c = 0; c < 4; c++) {
-      // an unused slot (box at +inf) is never entered: leave it alone
-      if (n.lox[c] == hpt::kInf)
-        continue;
-      int32_t ch = n.child[c];
-      if (ch >= 0) {
-        n.child[c] = ch + nodeOff;
-      } else {
-        const uint32_t enc = ~(uint32_t)ch;
-        uint32_t first = enc >> 3;
-        const uint32_t cnt = enc & 7u;
-        first = order ? (*order)[first] : first + (uint32_t)primOff;
-        n.child[c] = (int32_t) ~((first << 3) | cnt);
+  // the leaf of the TLAS's unused slots: an instance of that triangle, after
+  // the world's own
+  const int32_t noInstance = (int32_t) ~((uint32_t)dinst.size() << 3);
+  {
+    hpt::DInstance none;
+    std::memset(&none, 0, sizeof(none));
+    none.rcp[0] = none.rcp[4] = none.rcp[8] = 1.f;
+    none.xfm[0] = none.xfm[4] = none.xfm[8] = 1.f;
+    none.blasRoot = kNoPrim;
+    none.userID = hpt::kInvalidID;
+    dinst.push_back(none);
+  }
+  for (auto &n : T.nodes) // TLAS leaves: instance indices
+    for (int c = 0; c < 4; c++)
+      if (n.lox[c] != hpt::kInf && n.child[c] < 0) {
+        const uint32_t enc = ~(uint32_t)n.child[c];
+        n.child[c] = (int32_t) ~((tlasOrder[enc >> 3] << 3) | (enc & 7u));
       }
-    }
-    return n;
-  };
-  // the world's node array: every BLAS (relocated on the device for device
-  // builds, on the host otherwise), then the TLAS; primitive records of
-  // every BLAS in the same order
+  // the world's node array: every BLAS, then the TLAS, put into the
+  // traversal's layout on the device; primitive records of every BLAS in the
+  // same order
   const size_t totalNodeCount = nNodes + T.nodes.size();
   D.gpu();
   HIP_CHECK(hipStreamSynchronize(D.stream)); // frames in flight read the old arrays
-  dNodes.ensure(std::max<size_t>(sizeof(hpt::DNode4) * totalNodeCount, 16));
-  dPrims.ensure(std::max<size_t>(sizeof(hpt::DPrim) * nPrims, 16));
+  dNodes.ensure(sizeof(hpt::DNode4) * totalNodeCount);
+  dPrims.ensure(sizeof(hpt::DPrim) * nPrims);
   hpt::DNode4 *gNodes = dNodes.as<hpt::DNode4>();
   hpt::DPrim *gPrims = dPrims.as<hpt::DPrim>();
+  HIP_CHECK(hipMemsetAsync(gPrims, 0, sizeof(hpt::DPrim), D.stream));
   for (size_t k = 0; k < uniqueBlas.size(); k++) {
-    const Blas &B = *uniqueBlas[k];
-    if (B.onDevice) {
-      HIP_CHECK(hpt_bvh_relocate(gNodes + blasNodeOff[k], B.dNodes.ptr, B.numNodes, blasNodeOff[k],
-          (uint32_t)blasPrimOff[k], D.stream));
+    Blas &B = *uniqueBlas[k];
+    if (!B.nodes.empty()) { // a host build's first world
+      B.dNodes.upload(B.nodes);
+      B.dPrims.upload(B.prims);
+      std::vector<hpt::BNode4>().swap(B.nodes);
+      std::vector<hpt::DPrim>().swap(B.prims);
+    }
+    HIP_CHECK(hpt_bvh_relocate(gNodes + blasNodeOff[k], B.dNodes.ptr, B.numNodes, blasNodeOff[k],
+        (uint32_t)blasPrimOff[k], kNoPrim, D.stream));
+    if (B.numPrims > 0)
       HIP_CHECK(hipMemcpyAsync(gPrims + blasPrimOff[k], B.dPrims.ptr, sizeof(hpt::DPrim) * B.numPrims,
           hipMemcpyDeviceToDevice, D.stream));
-    } else {
-      std::vector<hpt::DNode4> moved(B.nodes.size());
-      for (size_t i = 0; i < B.nodes.size(); i++)
-        moved[i] = remap(B.nodes[i], blasNodeOff[k], blasPrimOff[k], nullptr);
-      HIP_CHECK(hipMemcpy(gNodes + blasNodeOff[k], moved.data(), sizeof(hpt::DNode4) * moved.size(),
-          hipMemcpyHostToDevice));
-      if (!B.prims.empty())
-        HIP_CHECK(hipMemcpy(gPrims + blasPrimOff[k], B.prims.data(), sizeof(hpt::DPrim) * B.prims.size(),
-            hipMemcpyHostToDevice));
-    }
   }
-  {
-    std::vector<hpt::DNode4> tl(T.nodes.size());
-    for (size_t i = 0; i < T.nodes.size(); i++)
-      tl[i] = remap(T.nodes[i], tlasOff, 0, &tlasOrder);
-    HIP_CHECK(hipMemcpy(gNodes + tlasOff, tl.data(), sizeof(hpt::DNode4) * tl.size(), hipMemcpyHostToDevice));
-  }
+  DevBuf tlas;
+  tlas.upload(T.nodes);
+  HIP_CHECK(hpt_bvh_relocate(gNodes + tlasOff, tlas.ptr, T.nodes.size(), tlasOff, 0, noInstance, D.stream));
   HIP_CHECK(hipStreamSynchronize(D.stream));
 
   // lights (PathTracerData.cpp:32-82): [geometry lights, world lights],
@@ -2374,6 +2381,7 @@ void World::commit() // World.cpp:70-188 plus the Group BLAS builds (Group.cpp:9
   scene.lightsCDF = dLightsCDF.as<const float>();
   scene.geoCDF = dGeoCDF.as<const float>();
   scene.tlasRoot = tlasOff;
+  scene.extent = boxExtent(T.bounds);
   scene.numInstances = (int)instances.size();
   scene.numLights = (int)dl.size();
   scene.numMaterials = (int)dmats.size();
@@ -2383,7 +2391,7 @@ void World::commit() // World.cpp:70-188 plus the Group BLAS builds (Group.cpp:9
   scene.volInsts = dVolInsts.as<const hpt::DVolInst>();
   scene.numVolInsts = (int32_t)volInsts.size();
   totalNodes = (int64_t)totalNodeCount;
-  totalPrims = (int64_t)nPrims;
+  totalPrims = (int64_t)nPrims - 1;
   blasBuildMs = 0.0;
   deviceBlas = 0;
   for (auto &b : uniqueBlas) {

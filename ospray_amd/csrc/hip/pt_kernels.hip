@@ -435,8 +435,10 @@ __device__ __forceinline__ void traceQueue(const DScene &S, const uint32_t *queu
       if (idle == ~0ull) // the queue is exhausted and every lane waits
         break;
     }
-    traceDescend<TIES, STATS>(s, S, best, lds, ovf, st);
-    if (busy && (s.post == 0 ? s.cur == kTraceDone : traceLeaf<MODE, STATS, RECORD, TIES>(s, S, best, lds, ovf, st, occluded))) {
+    traceDescend<STATS>(s, S, lds, ovf, st);
+    if (busy
+        && (traceHolds(s) ? traceLeaf<MODE, STATS, RECORD, TIES>(s, S, best, lds, ovf, st, occluded)
+                          : s.cur == kTraceDone)) {
       busy = false;
       ended = true;
       s.cur = kTraceDone;

@@ -3,7 +3,7 @@
 // The reference hands these to Embree (rtcIntersectV,
 // modules/cpu/common/World.ih:29-52, 247-286).  Here:
 //   * two-level 4-wide BVH (TLAS over instances, one BLAS per group) in
-//     128-byte nodes holding four child boxes; one lane per ray, children
+//     64-byte nodes holding four child boxes; one lane per ray, children
 //     visited nearest first, speculative while-while order (Aila and Laine,
 //     "Understanding the efficiency of ray traversal on GPUs", 2009): a
 //     lane holds a leaf it reaches and goes on with inner nodes until no
@@ -29,7 +29,7 @@
 //     compared with the current closest on arrival, hits up to kTieEps
 //     beyond it are still tested, and the flag clears only when a hit
 //     closer than the window's lower end arrives;
-//   * node boxes only cull, conservatively (far plane scaled by 1+4e-7).
+//   * node boxes only cull, conservatively (nodeNear).
 #pragma once
 
 #include "pt_math.h"
@@ -72,10 +72,11 @@ HPT_HD bool better(float t, uint32_t i, uint32_t m, uint32_t p, uint32_t h, cons
   return !b.hit || t < b.t || (t == b.t && keyLess(i, m, p, h, b));
 }
 
-HPT_HD float safeInv(float d)
+// reciprocal of a direction component for the box tests, good to 1 ulp
+__device__ __forceinline__ float boxInv(float d)
 {
   const float ad = fabsf(d);
-  return 1.0f / (ad < 1e-18f ? copysignf(1e-18f, d) : d);
+  return __builtin_amdgcn_rcpf(ad < 1e-18f ? copysignf(1e-18f, d) : d);
 }
 
 struct TriPre
@@ -236,24 +237,44 @@ HPT_HD double fp64SphereT(const double o[3], const double d[3], vec3f center, fl
   return (exitRoot ? (-B + sq) : (-B - sq)) / A;
 }
 
-// one 4-wide node: child boxes as per-axis float4s (lane c = child c)
+// one 4-wide node as its four 16-byte loads (DNode4)
 struct Node4
 {
-  float4 lox, hix, loy, hiy, loz, hiz;
+  float4 a, b; // p, s.x | s.y, s.z, lox, hix
+  uint4 c;     // loy, hiy, loz, hiz
   int4 child;
 };
+
+// What the box test needs of a ray, per axis: 1 / d and -o / d shifted by
+// the padding of the near and far planes (see nodeNear).
+struct BoxRay
+{
+  vec3f inv, kn, kf;
+};
+
+// 10 ulp (of 2^-24) of the largest coordinate difference a box test forms
+constexpr float kBoxPad = 5.96046448e-7f;
+
+__device__ __forceinline__ BoxRay boxRay(vec3f o, vec3f d, float extent)
+{
+  BoxRay r;
+  r.inv = v3(boxInv(d.x), boxInv(d.y), boxInv(d.z));
+  const vec3f k = v3(-o.x * r.inv.x, -o.y * r.inv.y, -o.z * r.inv.z);
+  const vec3f pad = v3(kBoxPad * (fabsf(o.x) + extent) * fabsf(r.inv.x), kBoxPad * (fabsf(o.y) + extent) * fabsf(r.inv.y),
+      kBoxPad * (fabsf(o.z) + extent) * fabsf(r.inv.z));
+  r.kn = k - pad;
+  r.kf = k + pad;
+  return r;
+}
 
 __device__ __forceinline__ Node4 loadNode(const DNode4 *nodes, int idx)
 {
   const float4 *np = reinterpret_cast<const float4 *>(nodes + idx);
   Node4 n;
-  n.lox = np[0];
-  n.hix = np[1];
-  n.loy = np[2];
-  n.hiy = np[3];
-  n.loz = np[4];
-  n.hiz = np[5];
-  n.child = reinterpret_cast<const int4 *>(np)[6];
+  n.a = np[0];
+  n.b = np[1];
+  n.c = reinterpret_cast<const uint4 *>(np)[2];
+  n.child = reinterpret_cast<const int4 *>(np)[3];
   return n;
 }
 
@@ -269,15 +290,52 @@ __device__ __forceinline__ void cswap(float &ta, int &ca, float &tb, int &cb)
   ca = c;
 }
 
-__device__ __forceinline__ float slabNear(float lox, float loy, float loz, float hix, float hiy, float hiz,
-    vec3f o, vec3f inv, float t0, float tb)
+// one axis of a node for a ray: plane q is entered at q * a + near (from
+// the byte of `first`) and left at q * a + far (`last`)
+struct NodeAxis
 {
-  const float x0 = (lox - o.x) * inv.x, x1 = (hix - o.x) * inv.x;
-  const float y0 = (loy - o.y) * inv.y, y1 = (hiy - o.y) * inv.y;
-  const float z0 = (loz - o.z) * inv.z, z1 = (hiz - o.z) * inv.z;
-  const float tn = fmaxf(fmaxf(fminf(x0, x1), fminf(y0, y1)), fmaxf(fminf(z0, z1), t0));
-  const float tf = fminf(fminf(fmaxf(x0, x1), fmaxf(y0, y1)), fminf(fmaxf(z0, z1), tb)) * 1.0000004f;
-  return tn <= tf ? tn : kInf;
+  float a, near, far;
+  uint32_t first, last;
+};
+
+__device__ __forceinline__ NodeAxis nodeAxis(float p, float s, uint32_t lo, uint32_t hi, float inv, float kn, float kf)
+{
+  NodeAxis x;
+  x.a = s * inv;
+  x.near = fmaf(p, inv, kn);
+  x.far = fmaf(p, inv, kf);
+  const bool back = inv < 0.f;
+  x.first = back ? hi : lo;
+  x.last = back ? lo : hi;
+  return x;
+}
+
+// Entry distances t[c] of the four children's boxes over [t0, tb], +inf for
+// a box the ray misses.
+//
+// Conservative: with u = 2^-24, a plane's distance (p + q s - o) / d comes
+// out off by at most 5 u (|o| + extent) / |d| from the roundings of 1 / d (1
+// ulp), -o / d, p / d - o / d, s / d, the product and the sum, extent
+// bounding the tree's coordinates; the near planes are moved down and the
+// far ones up by twice that, which leaves 5 ulp of slack for a primitive's
+// own hit distance, so the closest hit does not depend on the tree.  A NaN
+// (overflow) leaves the axis out of the test.  The near plane of an axis is
+// picked once for the four children, a word at a time: a minimum or maximum
+// costs 4.3 cycles of a SIMD, a select or FMA 2.6 (measured).
+__device__ __forceinline__ void nodeNear(const Node4 &n, const BoxRay &r, float t0, float tb, float t[4])
+{
+  const NodeAxis x = nodeAxis(n.a.x, n.a.w, __float_as_uint(n.b.z), __float_as_uint(n.b.w), r.inv.x, r.kn.x, r.kf.x);
+  const NodeAxis y = nodeAxis(n.a.y, n.b.x, n.c.x, n.c.y, r.inv.y, r.kn.y, r.kf.y);
+  const NodeAxis z = nodeAxis(n.a.z, n.b.y, n.c.z, n.c.w, r.inv.z, r.kn.z, r.kf.z);
+#pragma unroll
+  for (int c = 0; c < 4; c++) {
+    auto q = [c](uint32_t w) { return (float)((w >> (8 * c)) & 0xffu); };
+    const float tn = fmaxf(fmaxf(fmaf(q(x.first), x.a, x.near), fmaf(q(y.first), y.a, y.near)),
+        fmaxf(fmaf(q(z.first), z.a, z.near), t0));
+    const float tf = fminf(fminf(fmaf(q(x.last), x.a, x.far), fmaf(q(y.last), y.a, y.far)),
+        fminf(fmaf(q(z.last), z.a, z.far), tb));
+    t[c] = tn <= tf ? tn : kInf;
+  }
 }
 
 // Traversal modes: MODE_CLOSEST returns the closest hit; MODE_OCCLUSION
@@ -334,7 +392,7 @@ __device__ void resolveNearTie(const DScene &S, vec3f worg, vec3f wdir, float t0
   const float tF = best.t;
   const float tHi = fminf(tF + kTieEps * tF, tfar);
   const float tLo = fmaxf(t0, kTieBoxLow * tF);
-  const vec3f winv = v3(safeInv(wdir.x), safeInv(wdir.y), safeInv(wdir.z));
+  const BoxRay wbox = boxRay(worg, wdir, S.extent);
   Hit w = best;
   double wD = 0.0;
   bool have = false;
@@ -353,14 +411,12 @@ __device__ void resolveNearTie(const DScene &S, vec3f worg, vec3f wdir, float t0
     return (int)ovf[sp - kLdsDepth];
   };
   // children of node `cur` whose boxes the ray enters in (t0, tHi]
-  auto expand = [&](int cur, vec3f o, vec3f inv) -> bool {
+  auto expand = [&](int cur, const BoxRay &r) -> bool {
     const Node4 nd = loadNode(S.nodes, cur);
     if (STATS)
       st.nodes++;
-    const float tc[4] = {slabNear(nd.lox.x, nd.loy.x, nd.loz.x, nd.hix.x, nd.hiy.x, nd.hiz.x, o, inv, tLo, tHi),
-        slabNear(nd.lox.y, nd.loy.y, nd.loz.y, nd.hix.y, nd.hiy.y, nd.hiz.y, o, inv, tLo, tHi),
-        slabNear(nd.lox.z, nd.loy.z, nd.loz.z, nd.hix.z, nd.hiy.z, nd.hiz.z, o, inv, tLo, tHi),
-        slabNear(nd.lox.w, nd.loy.w, nd.loz.w, nd.hix.w, nd.hiy.w, nd.hiz.w, o, inv, tLo, tHi)};
+    float tc[4];
+    nodeNear(nd, r, tLo, tHi, tc);
     const int ch[4] = {nd.child.x, nd.child.y, nd.child.z, nd.child.w};
     for (int c = 0; c < 4; c++)
       if (tc[c] != kInf) {
@@ -374,7 +430,7 @@ __device__ void resolveNearTie(const DScene &S, vec3f worg, vec3f wdir, float t0
   while (sp > 0) {
     const int cur = pop();
     if (cur >= 0) {
-      if (!expand(cur, worg, winv))
+      if (!expand(cur, wbox))
         return;
       continue;
     }
@@ -383,7 +439,7 @@ __device__ void resolveNearTie(const DScene &S, vec3f worg, vec3f wdir, float t0
     const linear3f rl = {{I.rcp[0], I.rcp[1], I.rcp[2]}, {I.rcp[3], I.rcp[4], I.rcp[5]}, {I.rcp[6], I.rcp[7], I.rcp[8]}};
     const vec3f o = mul(rl, worg) + v3(I.rcp[9], I.rcp[10], I.rcp[11]);
     const vec3f d = mul(rl, wdir);
-    const vec3f inv = v3(safeInv(d.x), safeInv(d.y), safeInv(d.z));
+    const BoxRay box = boxRay(o, d, I.extent);
     const TriPre pc = triPrecompute(d);
     double od[3], dd[3];
     fp64ObjectRay(I.rcp, worg, wdir, od, dd);
@@ -392,7 +448,7 @@ __device__ void resolveNearTie(const DScene &S, vec3f worg, vec3f wdir, float t0
     while (sp > base) {
       const int c = pop();
       if (c >= 0) {
-        if (!expand(c, o, inv))
+        if (!expand(c, box))
           return;
         continue;
       }
@@ -469,10 +525,12 @@ constexpr int TIES_OFF = 0, TIES_RESOLVE = 1, TIES_REPORT = 2;
 // the kernels) keeps the lanes of a wave busy with rays from a queue.
 struct TraceState
 {
-  vec3f worg, wdir, winv; // the world ray
-  vec3f o, d, inv;        // the current (world or object) ray
+  vec3f worg, wdir; // the world ray
+  vec3f o, d;       // the current (world or object) ray
+  BoxRay box;       // of the current ray
   TriPre pc;
   float t0, tfar;
+  float tb; // hits beyond it are of no interest: the closest one (with TIES, a near-tie beyond it)
   int inst, modelOffset, sp, cur, post;
   bool tie;            // a near-tie of the current closest hit has been seen (TIES != TIES_OFF)
   bool sawTransparent; // MODE_OCCLUSION: a non-opaque primitive was hit
@@ -492,13 +550,13 @@ __device__ __forceinline__ void traceBegin(
   best.half = 0;
   s.worg = worg;
   s.wdir = wdir;
-  s.winv = v3(safeInv(wdir.x), safeInv(wdir.y), safeInv(wdir.z));
   s.o = worg;
   s.d = wdir;
-  s.inv = s.winv;
+  s.box = boxRay(worg, wdir, S.extent);
   s.pc = {0, 1, 2, 0.f, 0.f, 0.f};
   s.t0 = t0;
   s.tfar = tfar;
+  s.tb = tfar;
   s.inst = -1;
   s.modelOffset = 0;
   s.sp = 0;
@@ -540,26 +598,27 @@ __device__ __forceinline__ int tracePop(TraceState &s, const uint32_t *lds, cons
 // trades some fuller leaf rounds for that.  1920x1080, 4 spp: 26.4 ->
 // 24.9 ms (ratios of searching to holding lanes 1/4, 1/2, 2/3, 1, 3/2, 2, 4:
 // 25.2, 24.7, 24.7, 24.8, 25.1, 25.4, 26.6); never later than that, so a
-// wave with few rays goes on as before.  A held BLAS leaf
-// stops the lane at the instance's exit marker (it needs the object ray); a
+// wave with few rays goes on as before.  The exit of an instance
+// (its marker) stops a lane too: traceLeaf gives it the world ray back.  A
 // held instance leaf is entered from the world level, with the next world
 // node pushed below the marker.  Lanes with cur == kTraceDone and no held
 // leaf (finished or idle) only take part in the wave vote.
-template <int TIES, bool STATS>
+// a lane that needs traceLeaf: it holds a leaf or stands at the exit of an
+// instance
+__device__ __forceinline__ bool traceHolds(const TraceState &s) { return s.post != 0 || s.cur == kMarker; }
+
+template <bool STATS>
 __device__ __forceinline__ void traceDescend(
-    TraceState &s, const DScene &S, const Hit &best, uint32_t *lds, uint32_t *ovf, TraceStats &st)
+    TraceState &s, const DScene &S, uint32_t *lds, uint32_t *ovf, TraceStats &st)
 {
   for (;;) {
     if (s.cur >= 0 && s.cur < kTraceDone) {
       const Node4 nd = loadNode(S.nodes, s.cur);
       if (STATS)
         st.nodes++;
-      // with TIES, boxes up to a near-tie beyond the closest hit stay open
-      const float tb = TIES != TIES_OFF && best.hit ? fminf(best.t + kTieEps * best.t, s.tfar) : best.t;
-      float t0c = slabNear(nd.lox.x, nd.loy.x, nd.loz.x, nd.hix.x, nd.hiy.x, nd.hiz.x, s.o, s.inv, s.t0, tb);
-      float t1c = slabNear(nd.lox.y, nd.loy.y, nd.loz.y, nd.hix.y, nd.hiy.y, nd.hiz.y, s.o, s.inv, s.t0, tb);
-      float t2c = slabNear(nd.lox.z, nd.loy.z, nd.loz.z, nd.hix.z, nd.hiy.z, nd.hiz.z, s.o, s.inv, s.t0, tb);
-      float t3c = slabNear(nd.lox.w, nd.loy.w, nd.loz.w, nd.hix.w, nd.hiy.w, nd.hiz.w, s.o, s.inv, s.t0, tb);
+      float tc[4];
+      nodeNear(nd, s.box, s.t0, s.tb, tc);
+      float t0c = tc[0], t1c = tc[1], t2c = tc[2], t3c = tc[3];
       int c0 = nd.child.x, c1 = nd.child.y, c2 = nd.child.z, c3 = nd.child.w;
       cswap(t0c, c0, t1c, c1);
       cswap(t2c, c2, t3c, c3);
@@ -593,131 +652,134 @@ __device__ __forceinline__ void traceDescend(
           s.cur = c0;
         }
       }
-    } else if (s.cur == kMarker && s.post == 0) {
-      s.o = s.worg;
-      s.d = s.wdir;
-      s.inv = s.winv;
-      s.inst = -1;
-      s.cur = s.sp == 0 ? kTraceDone : tracePop(s, lds, ovf);
     }
     if (s.cur < 0 && s.post == 0) { // hold the leaf, go on
       s.post = s.cur;
       s.cur = s.sp == 0 ? kTraceDone : tracePop(s, lds, ovf);
     }
-    const bool canStep = (s.cur >= 0 && s.cur < kTraceDone) || (s.cur == kMarker && s.post == 0);
-    if (__popcll(__ballot(canStep && s.post == 0)) <= __popcll(__ballot(s.post != 0)))
+    const unsigned long long searching = __ballot(s.cur >= 0 && s.cur < kTraceDone && s.post == 0);
+    if (__popcll(searching) <= __popcll(__ballot(traceHolds(s))))
       break;
   }
 }
 
-// The leaf a lane holds (s.post != 0): an instance leaf enters the
-// instance's BLAS with the object ray; a BLAS leaf tests its primitives.
-// Returns true when the lane's traversal has ended: no node left, an
+// What a lane holds (traceHolds): an instance leaf enters the instance's
+// BLAS with the object ray; a BLAS leaf tests its primitives; the marker
+// leaves the instance.  Returns true when the lane's traversal has ended: no node left, an
 // opaque occluder (MODE_OCCLUSION, `occluded` set) or a full stack.
 template <int MODE, bool STATS, bool RECORD, int TIES>
 __device__ __forceinline__ bool traceLeaf(TraceState &s, const DScene &S, Hit &best, uint32_t *lds, uint32_t *ovf,
     TraceStats &st, bool &occluded)
 {
-  const uint32_t enc = ~(uint32_t)s.post;
-  s.post = 0;
-  const uint32_t first = enc >> 3;
-  const uint32_t count = (enc & 7u) + 1u;
-  if (s.inst < 0) {
-    // world leaf: one instance; continue in its BLAS with the object ray
-    s.inst = (int)first;
-    const DInstance &I = S.instances[s.inst];
-    const linear3f rl = {{I.rcp[0], I.rcp[1], I.rcp[2]}, {I.rcp[3], I.rcp[4], I.rcp[5]}, {I.rcp[6], I.rcp[7], I.rcp[8]}};
-    s.o = mul(rl, s.worg) + v3(I.rcp[9], I.rcp[10], I.rcp[11]);
-    s.d = mul(rl, s.wdir);
-    s.inv = v3(safeInv(s.d.x), safeInv(s.d.y), safeInv(s.d.z));
-    s.pc = triPrecompute(s.d);
-    s.modelOffset = I.modelOffset;
-    if (s.sp + 2 > kLdsDepth + kOverflowDepth)
-      return true;
-    if (s.cur != kTraceDone)
-      tracePush(s, lds, ovf, s.cur);
-    tracePush(s, lds, ovf, kMarker);
-    s.cur = I.blasRoot;
-    return false;
-  }
-  const float t0 = s.t0;
-  for (uint32_t k = 0; k < count; k++) {
-    const DPrim &P = S.prims[first + k];
-    const float4 pa = reinterpret_cast<const float4 *>(&P)[0];
-    const float4 pb = reinterpret_cast<const float4 *>(&P)[1];
-    const float4 pcv = reinterpret_cast<const float4 *>(&P)[2];
-    const uint32_t primID = __float_as_uint(pa.w);
-    const uint32_t mk = __float_as_uint(pb.w);
-    const uint32_t model = mk & 0x0fffffffu;
-    const uint32_t kind = mk >> 28;
-    if (STATS)
-      st.prims++;
-    if (MODE == MODE_OCCLUSION && kind == PRIM_SPHERE) {
-      float tE, tX;
-      vec3f NE, NX;
-      const int roots = sphereRoots(s.o, s.d, t0, v3(pa.x, pa.y, pa.z), pb.x, best.t, tE, NE, tX, NX);
-      if (!roots)
-        continue;
-      if (S.models[s.modelOffset + model].opaque) {
-        occluded = true;
+  if (s.post != 0) {
+    const uint32_t enc = ~(uint32_t)s.post;
+    s.post = 0;
+    const uint32_t first = enc >> 3;
+    const uint32_t count = (enc & 7u) + 1u;
+    if (s.inst < 0) {
+      // world leaf: one instance; continue in its BLAS with the object ray
+      s.inst = (int)first;
+      const DInstance &I = S.instances[s.inst];
+      const linear3f rl = {{I.rcp[0], I.rcp[1], I.rcp[2]}, {I.rcp[3], I.rcp[4], I.rcp[5]}, {I.rcp[6], I.rcp[7], I.rcp[8]}};
+      s.o = mul(rl, s.worg) + v3(I.rcp[9], I.rcp[10], I.rcp[11]);
+      s.d = mul(rl, s.wdir);
+      s.box = boxRay(s.o, s.d, I.extent);
+      s.pc = triPrecompute(s.d);
+      s.modelOffset = I.modelOffset;
+      if (s.sp + 2 > kLdsDepth + kOverflowDepth)
         return true;
-      }
-      s.sawTransparent = true;
-      if (RECORD) {
-        if (roots & 1)
-          recordHit(ovf, tE, (uint32_t)s.inst, first + k, 0);
-        if (roots & 2)
-          recordHit(ovf, tX, (uint32_t)s.inst, first + k, 1);
-      }
-      continue;
+      if (s.cur != kTraceDone)
+        tracePush(s, lds, ovf, s.cur);
+      tracePush(s, lds, ovf, kMarker);
+      s.cur = I.blasRoot;
+      return false;
     }
-    float t, u = 0.f, v = 0.f;
-    vec3f Ng;
-    bool h;
-    uint32_t half = 0;
-    const float tmaxP = TIES != TIES_OFF && best.hit ? fminf(best.t + kTieEps * best.t, s.tfar) : best.t;
-    if (kind == PRIM_SPHERE) {
-      h = intersectSphere(s.o, s.d, t0, v3(pa.x, pa.y, pa.z), pb.x, tmaxP, t, Ng);
-    } else {
-      const vec3f A = v3(pa.x, pa.y, pa.z), B = v3(pb.x, pb.y, pb.z), C = v3(pcv.x, pcv.y, pcv.z);
-      h = intersectTriangle(s.o, t0, s.pc, A, B, C, tmaxP, t, u, v);
-      if (h) {
-        Ng = cross(B - A, C - A);
-        if (kind == PRIM_QUAD1) {
-          half = 1;
-          u = 1.0f - u;
-          v = 1.0f - v;
+    const float t0 = s.t0;
+    for (uint32_t k = 0; k < count; k++) {
+      const DPrim &P = S.prims[first + k];
+      const float4 pa = reinterpret_cast<const float4 *>(&P)[0];
+      const float4 pb = reinterpret_cast<const float4 *>(&P)[1];
+      const float4 pcv = reinterpret_cast<const float4 *>(&P)[2];
+      const uint32_t primID = __float_as_uint(pa.w);
+      const uint32_t mk = __float_as_uint(pb.w);
+      const uint32_t model = mk & 0x0fffffffu;
+      const uint32_t kind = mk >> 28;
+      if (STATS)
+        st.prims++;
+      if (MODE == MODE_OCCLUSION && kind == PRIM_SPHERE) {
+        float tE, tX;
+        vec3f NE, NX;
+        const int roots = sphereRoots(s.o, s.d, t0, v3(pa.x, pa.y, pa.z), pb.x, s.tb, tE, NE, tX, NX);
+        if (!roots)
+          continue;
+        if (S.models[s.modelOffset + model].opaque) {
+          occluded = true;
+          return true;
+        }
+        s.sawTransparent = true;
+        if (RECORD) {
+          if (roots & 1)
+            recordHit(ovf, tE, (uint32_t)s.inst, first + k, 0);
+          if (roots & 2)
+            recordHit(ovf, tX, (uint32_t)s.inst, first + k, 1);
+        }
+        continue;
+      }
+      float t, u = 0.f, v = 0.f;
+      vec3f Ng;
+      bool h;
+      uint32_t half = 0;
+      if (kind == PRIM_SPHERE) {
+        h = intersectSphere(s.o, s.d, t0, v3(pa.x, pa.y, pa.z), pb.x, s.tb, t, Ng);
+      } else {
+        const vec3f A = v3(pa.x, pa.y, pa.z), B = v3(pb.x, pb.y, pb.z), C = v3(pcv.x, pcv.y, pcv.z);
+        h = intersectTriangle(s.o, t0, s.pc, A, B, C, s.tb, t, u, v);
+        if (h) {
+          Ng = cross(B - A, C - A);
+          if (kind == PRIM_QUAD1) {
+            half = 1;
+            u = 1.0f - u;
+            v = 1.0f - v;
+          }
         }
       }
-    }
-    if (!h)
-      continue;
-    if (MODE == MODE_OCCLUSION) {
-      if (S.models[s.modelOffset + model].opaque) {
-        occluded = true;
-        return true;
+      if (!h)
+        continue;
+      if (MODE == MODE_OCCLUSION) {
+        if (S.models[s.modelOffset + model].opaque) {
+          occluded = true;
+          return true;
+        }
+        s.sawTransparent = true;
+        if (RECORD)
+          recordHit(ovf, t, (uint32_t)s.inst, first + k, 0);
+        continue;
       }
-      s.sawTransparent = true;
-      if (RECORD)
-        recordHit(ovf, t, (uint32_t)s.inst, first + k, 0);
-      continue;
+      const bool nt = TIES != TIES_OFF && best.hit && nearTie(t, best.t);
+      if (better(t, (uint32_t)s.inst, model, primID, half, best)) {
+        if (TIES != TIES_OFF)
+          s.tie = nt; // a hit below the window of the previous closest one clears the flag
+        s.tb = TIES != TIES_OFF ? fminf(t + kTieEps * t, s.tfar) : t;
+        best.hit = true;
+        best.t = t;
+        best.u = u;
+        best.v = v;
+        best.Ng = Ng;
+        best.inst = (uint32_t)s.inst;
+        best.model = model;
+        best.prim = primID;
+        best.half = half;
+      } else if (nt) {
+        s.tie = true;
+      }
     }
-    const bool nt = TIES != TIES_OFF && best.hit && nearTie(t, best.t);
-    if (better(t, (uint32_t)s.inst, model, primID, half, best)) {
-      if (TIES != TIES_OFF)
-        s.tie = nt; // a hit below the window of the previous closest one clears the flag
-      best.hit = true;
-      best.t = t;
-      best.u = u;
-      best.v = v;
-      best.Ng = Ng;
-      best.inst = (uint32_t)s.inst;
-      best.model = model;
-      best.prim = primID;
-      best.half = half;
-    } else if (nt) {
-      s.tie = true;
-    }
+  }
+  if (s.cur == kMarker) {
+    s.o = s.worg;
+    s.d = s.wdir;
+    s.box = boxRay(s.worg, s.wdir, S.extent);
+    s.inst = -1;
+    s.cur = s.sp == 0 ? kTraceDone : tracePop(s, lds, ovf);
   }
   return s.cur == kTraceDone;
 }
@@ -730,11 +792,11 @@ __device__ bool traceRay(const DScene &S, vec3f worg, vec3f wdir, float t0, floa
   traceBegin(s, S, worg, wdir, t0, tfar, best);
   bool occluded = false;
   for (;;) {
-    traceDescend<TIES, STATS>(s, S, best, lds, ovf, st);
-    if (s.post == 0) { // nothing held: the lane has no node left
-      if (s.cur == kTraceDone)
+    traceDescend<STATS>(s, S, lds, ovf, st);
+    if (!traceHolds(s)) {
+      if (s.cur == kTraceDone) // no node left
         break;
-      continue; // (cannot happen: a lane without a held leaf can step)
+      continue; // other lanes hold leaves
     }
     if (traceLeaf<MODE, STATS, RECORD, TIES>(s, S, best, lds, ovf, st, occluded))
       break;

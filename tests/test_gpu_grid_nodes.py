@@ -1,0 +1,65 @@
+"""The traversal's nodes hold their children's boxes on an 8-bit grid, rounded
+outwards: whatever the boxes' sizes (flat, far apart in size, tiny, far from
+the origin) and however many slots a node uses, the closest hits are the
+oracle's bit for bit, since the boxes only cull."""
+import numpy as np
+import pytest
+
+from ospray_amd import api as A
+from ospray_amd import capi as K
+from ospray_amd import scenes
+from oracle import orc
+
+pytestmark = pytest.mark.gpu
+
+
+def _triangles(shape, n, scale, offset, rng):
+    c = rng.uniform(-1, 1, (n, 1, 3))
+    size = {"cloud": 0.3, "flat": 0.3, "sizes": 1.0}[shape]
+    if shape == "sizes":  # over four orders of magnitude within one tree
+        size = 10.0 ** rng.uniform(-4, 0, (n, 1, 1))
+    v = c + size * rng.uniform(-1, 1, (n, 3, 3))
+    if shape == "flat":  # every box without extent along y
+        v[:, :, 1] = 0.25
+    return (scale * v + np.array(offset)).reshape(-1, 3).astype(np.float32)
+
+
+def _rays(v, rng, n=4000):
+    lo, hi = v.min(0), v.max(0)
+    mid, ext = 0.5 * (lo + hi), float((hi - lo).max())
+    o = mid + ext * rng.uniform(-1.5, 1.5, (n, 3))
+    t = v[rng.integers(0, len(v), n)] + 0.05 * ext * rng.normal(size=(n, 3))
+    d = t - o
+    axis = rng.integers(0, 3, n // 4)  # a quarter parallel to an axis
+    d[: n // 4] = np.eye(3)[axis] * rng.choice([-1.0, 1.0], (n // 4, 1))
+    o[: n // 4] = t[: n // 4] - 2.0 * ext * d[: n // 4]
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    return np.concatenate([o, d, np.zeros((n, 1)), np.full((n, 1), np.inf)], 1).astype(np.float32)
+
+
+@pytest.mark.parametrize("host", [True, False])
+@pytest.mark.parametrize("shape,n,scale,offset", [
+    ("cloud", 1, 1.0, (0, 0, 0)), ("cloud", 2, 1.0, (0, 0, 0)), ("cloud", 3, 1.0, (0, 0, 0)),
+    ("cloud", 5, 1.0, (0, 0, 0)), ("cloud", 9, 1e-3, (0, 0, 0)), ("cloud", 700, 1.0, (40, -30, 90)),
+    ("flat", 300, 1.0, (0, 0, 0)), ("flat", 2, 100.0, (0, 7, 0)), ("sizes", 600, 1.0, (0, 0, 0)),
+    ("sizes", 600, 50.0, (0, 500, 0))])
+def test_hits_equal_the_oracle(hip_device, shape, n, scale, offset, host):
+    rng = np.random.default_rng(n)
+    v = _triangles(shape, n, scale, offset, rng)
+    geoms = [scenes.Geometry("triangles", vertex=v, index=np.arange(3 * n, dtype=np.uint32).reshape(-1, 3))]
+    insts = [scenes.Instance(0), scenes.Instance(0, xfm=(0.5, 0, 0, 0, -0.7, 0, 0.1, 0, 0.6, 0.3 * scale, 0, 0))]
+    sc = scenes.Scene("grid", 8, 8, geoms, [scenes.Model(0, 0)], [[0]], insts, [{"type": "obj"}],
+                      [{"type": "ambient"}], {"position": (0, 0, -1), "direction": (0, 0, 1)}, {"pixelSamples": 1})
+    dev = K.lib().ospGetCurrentDevice()
+    A.set_device_param(dev, "hostBvh", host)
+    K.lib().ospDeviceCommit(dev)
+    try:
+        s = scenes.to_ospray(sc)
+    finally:
+        A.set_device_param(dev, "hostBvh", True)
+        K.lib().ospDeviceCommit(dev)
+    rays = _rays(v, rng)
+    tuv, ids, _ = A.trace_rays(s.world, rays)
+    otuv, oids, _ = orc.OracleScene(sc).intersect(rays)
+    assert np.array_equal(ids, oids) and np.array_equal(tuv, otuv)
+    assert (ids[:, 0] != 0xFFFFFFFF).any()
