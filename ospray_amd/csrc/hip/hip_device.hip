@@ -1167,7 +1167,7 @@ class HipDevice : public Device
         HIP_CHECK(hipStreamCreateWithFlags(&L->stream, hipStreamNonBlocking));
         L->ownsStream = true;
       }
-      L->counters.ensure(64);
+      L->counters.ensure(4 * hpt::kCounterWords);
       if (residentTraceBlocks > 0)
         ensureScratch(*L);
       L->paths.counters = L->counters.as<int32_t>();

@@ -206,8 +206,14 @@ __global__ void k_reset(int32_t *counters, uint32_t mask, int32_t keep, const ui
     }
     cancelled = __shfl(cancelled, 0);
   }
-  if (i < kNumCounters && (((mask >> i) & 1u) || (cancelled && i == keep)))
-    counters[i] = 0;
+  if (i < kCntFetchExtend) {
+    if (((mask >> i) & 1u) || (cancelled && i == keep))
+      counters[i] = 0;
+  } else if (i < kCntFetchExtend + 2 * kXcds) { // the fetch counters of a traversal
+    const int k = i - kCntFetchExtend;
+    if ((mask >> (k < kXcds ? kCntFetchExtend : kCntFetchShadow)) & 1u)
+      counters[kFetchBase + k * kFetchStride] = 0;
+  }
   if (cancelled && i == 0)
     __hip_atomic_store(cancelLatch, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -338,13 +344,46 @@ __global__ __launch_bounds__(256) void k_generate(DFrame F, DPaths P)
 
 // Work distribution of the traversal kernels: each wave takes batches of
 // 64 consecutive queue entries (neighbouring pixels' rays, which share node
-// fetches) with one atomic per batch, until the queue is exhausted.
-__device__ __forceinline__ int nextBatch(int32_t *counter)
+// fetches) with one atomic per batch, until the queue is exhausted.  The
+// queue is cut into one contiguous part per XCD: blocks go to the XCDs in
+// turn, so a wave takes from its XCD's part first and from the next parts
+// once that is exhausted.  An XCD's L2 then holds the nodes under an eighth
+// of the rays in flight instead of under all of them, and a fetch counter
+// serves an eighth of the waves.  Streams serialised, before -> now: 1080p
+// terrain at 4 spp k_extend 7.57 -> 6.71 ms, k_shadow 9.03 -> 7.95 ms;
+// volume scene 1.69 -> 1.24 and 1.41 -> 1.14 ms.
+struct Fetch
 {
-  int base = 0;
-  if (laneId() == 0)
-    base = atomicAdd(counter, 64);
-  return __shfl(base, 0);
+  int32_t *counters; // of the XCDs' parts
+  int n, per;        // entries, entries of a part (a multiple of 64)
+  int part, left;    // the part taken from, parts not yet found exhausted
+};
+
+__device__ __forceinline__ Fetch fetchBegin(int32_t *counters, int n)
+{
+  return {counters, n, ((n + 64 * kXcds - 1) / (64 * kXcds)) * 64, (int)(blockIdx.x % kXcds), kXcds};
+}
+
+// the next batch's first entry, n when there is none; size: its entries
+__device__ __forceinline__ int nextBatch(Fetch &f, int &size)
+{
+  while (f.left > 0) {
+    const int lo = f.part * f.per, hi = min(f.n, lo + f.per);
+    int at = f.per;
+    if (lo < hi) {
+      if (laneId() == 0)
+        at = atomicAdd(f.counters + f.part * kFetchStride, 64);
+      at = __builtin_amdgcn_readfirstlane(at);
+    }
+    if (lo + at < hi) {
+      size = min(64, hi - lo - at);
+      return lo + at;
+    }
+    f.part = f.part + 1 == kXcds ? 0 : f.part + 1;
+    f.left--;
+  }
+  size = 0;
+  return f.n;
 }
 
 #ifndef HPT_SPREAD_SHORT_QUEUES
@@ -390,10 +429,17 @@ __device__ __forceinline__ void traceQueue(const DScene &S, const uint32_t *queu
   const unsigned long long ltMask = (1ull << wl) - 1ull;
   const int waves = (int)((gridDim.x * blockDim.x) >> 6);
   const bool spread = HPT_SPREAD_SHORT_QUEUES && n < 64 * waves;
-  const int bCap = spread ? (n + waves - 1) / waves : 64; // entries per batch, 1..64
   // wave-uniform batch cursor; a spread queue's batches are the waves' own
-  int bBase = spread ? (globalId() >> 6) * bCap : nextBatch(fetch), bNext = 0;
-  uint32_t bEntry = wl < bCap && bBase + wl < n ? queue[bBase + wl] : 0u;
+  Fetch f = fetchBegin(fetch, n);
+  int bBase, bSize, bNext = 0;
+  if (spread) {
+    const int per = (n + waves - 1) / waves;
+    bBase = __builtin_amdgcn_readfirstlane(globalId() >> 6) * per;
+    bSize = min(per, n - bBase);
+  } else {
+    bBase = nextBatch(f, bSize);
+  }
+  uint32_t bEntry = wl < bSize ? queue[bBase + wl] : 0u;
   TraceState s;
   s.cur = kTraceDone;
   s.post = 0;
@@ -408,7 +454,6 @@ __device__ __forceinline__ void traceQueue(const DScene &S, const uint32_t *queu
         finish(ended, entry, best, occluded, s);
       ended = false;
       while (idle != 0ull && bBase < n) {
-        const int bSize = n - bBase < bCap ? n - bBase : bCap;
         const int avail = bSize - bNext;
         const int rank = __popcll(idle & ltMask);
         const int src = bNext + rank;
@@ -427,9 +472,12 @@ __device__ __forceinline__ void traceQueue(const DScene &S, const uint32_t *queu
         idle = __ballot(!busy);
         if (bNext == bSize) {
           // a spread queue: the first batches of all waves cover it
-          bBase = spread ? n : nextBatch(fetch);
           bNext = 0;
-          bEntry = !spread && bBase + wl < n ? queue[bBase + wl] : 0u;
+          if (spread)
+            bBase = n;
+          else
+            bBase = nextBatch(f, bSize);
+          bEntry = bBase < n && wl < bSize ? queue[bBase + wl] : 0u;
         }
       }
       if (idle == ~0ull) // the queue is exhausted and every lane waits
@@ -460,7 +508,7 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(5))
   uint32_t *ovf = P.overflow + (size_t)globalId() * kThreadRow;
   TraceStats st = {0, 0};
   uint32_t rays = 0;
-  traceQueue<MODE_CLOSEST, STATS, false, TIES_REPORT, kExtendRefill>(S, P.queue[qin], n, &P.counters[kCntFetchExtend], lds, ovf, st,
+  traceQueue<MODE_CLOSEST, STATS, false, TIES_REPORT, kExtendRefill>(S, P.queue[qin], n, P.counters + kFetchBase, lds, ovf, st,
       [&](uint32_t p, vec3f &org, vec3f &dir, float &t0, float &tfar) {
         const float4 o = ld4(P.org + 4 * (size_t)p);
         const float4 d = ld4(P.dir + 4 * (size_t)p);
@@ -1094,7 +1142,7 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(6))
   uint32_t *ovf = P.overflow + (size_t)globalId() * kThreadRow;
   TraceStats st = {0, 0};
   uint32_t rays = 0;
-  traceQueue<MODE_OCCLUSION, STATS, true, TIES_OFF, kShadowRefill>(S, P.shadowQueue, n, &P.counters[kCntFetchShadow], lds, ovf, st,
+  traceQueue<MODE_OCCLUSION, STATS, true, TIES_OFF, kShadowRefill>(S, P.shadowQueue, n, P.counters + kFetchBase + kXcds * kFetchStride, lds, ovf, st,
       [&](uint32_t r, vec3f &org, vec3f &dir, float &t0, float &tfar) {
         const float4 o4 = ld4(P.recOrg + 4 * (size_t)r);
         const float4 d4 = ld4(P.recDir + 4 * (size_t)r);
@@ -1627,7 +1675,7 @@ inline uint32_t extensionSideMask(int q)
 }
 hipError_t launchReset(const DPaths &p, uint32_t mask, int keep, hipStream_t s)
 {
-  hipLaunchKernelGGL(k_reset, dim3(1), dim3(kNumCounters), 0, s, p.counters, mask, keep, p.cancelFlag, p.cancelGen,
+  hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, s, p.counters, mask, keep, p.cancelFlag, p.cancelGen,
       p.cancelLatch);
   return hipGetLastError();
 }
@@ -1652,7 +1700,7 @@ hipError_t hpt_reset_extension_counters(const HptPaths *P, int keepIndex, hipStr
 hipError_t hpt_reset_append_counters(const HptPaths *P, int keepIndex, hipStream_t s)
 {
   const DPaths &p = *reinterpret_cast<const DPaths *>(P);
-  hipLaunchKernelGGL(k_reset, dim3(1), dim3(kNumCounters), 0, s, p.counters, 3u << (2 * (keepIndex ^ 1)), -1,
+  hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, s, p.counters, 3u << (2 * (keepIndex ^ 1)), -1,
       (const uint32_t *)nullptr, 0u, (uint32_t *)nullptr);
   return hipGetLastError();
 }
@@ -1660,7 +1708,7 @@ hipError_t hpt_reset_append_counters(const HptPaths *P, int keepIndex, hipStream
 hipError_t hpt_reset_shadow_counters(const HptPaths *P, hipStream_t s)
 {
   const DPaths &p = *reinterpret_cast<const DPaths *>(P);
-  hipLaunchKernelGGL(k_reset, dim3(1), dim3(kNumCounters), 0, s, p.counters, kShadowSideMask, -1,
+  hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, s, p.counters, kShadowSideMask, -1,
       (const uint32_t *)nullptr, 0u, (uint32_t *)nullptr);
   return hipGetLastError();
 }

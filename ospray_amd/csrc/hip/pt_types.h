@@ -291,14 +291,19 @@ struct DPaths
 // queue counters: [2q] entries of extension queue q (q = 0, 1), [2q+1] NEE
 // light samples appended while queue q was filled, then:
 constexpr int kCntShadow = 4; // shadow-ray records
-constexpr int kCntFetchExtend = 5; // work fetch of the extension traversal
-constexpr int kCntFetchShadow = 6; // work fetch of the shadow traversal
-constexpr int kCntTrans = 7; // records for the transparency pass
-constexpr int kCntTies = 8; // extension rays whose closest hit has a near-tie
-constexpr int kNumBounceCounters = 9; // the counters above are reset every bounce
-constexpr int kCntNrcQuery = 9; // radiance-cache queries of the pass
-constexpr int kCntNrcTrain = 10; // radiance-cache training records of the pass
+constexpr int kCntTrans = 5; // records for the transparency pass
+constexpr int kCntTies = 6; // extension rays whose closest hit has a near-tie
+constexpr int kCntNrcQuery = 7; // radiance-cache queries of the pass
+constexpr int kCntNrcTrain = 8; // radiance-cache training records of the pass
+// bits of a reset mask for the work fetch of the extension and the shadow
+// traversal
+constexpr int kCntFetchExtend = 9, kCntFetchShadow = 10;
 constexpr int kNumCounters = 11;
+// Work fetch: one counter per XCD and traversal, each on a cache line of
+// its own, after the counters above
+constexpr int kXcds = 8, kFetchStride = 32;
+constexpr int kFetchBase = 32; // word of the extension traversal's first counter
+constexpr int kCounterWords = kFetchBase + 2 * kXcds * kFetchStride;
 
 // path flags in ld[3]
 constexpr uint32_t FLAG_DEPTH_MASK = 0xffu; // bits 0-7
