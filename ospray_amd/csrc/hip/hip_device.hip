@@ -2405,9 +2405,9 @@ void World::commit() // World.cpp:70-188 plus the Group BLAS builds (Group.cpp:9
   // the traversal stack holds the TLAS entries of one root-to-leaf path,
   // the next TLAS node (a held instance leaf is entered after the lane went
   // on in the TLAS), the instance marker and the BLAS entries
-  if (T.stackNeed + 2 + blasStackNeed > hpt_stack_capacity())
-    throw std::runtime_error("BVH too deep for the traversal stack");
   stackNeed = T.stackNeed + 2 + blasStackNeed;
+  if (stackNeed > hpt_stack_capacity())
+    throw std::runtime_error("BVH too deep for the traversal stack");
   maxDepth = std::max(maxDepth, T.maxDepth);
   built = true;
 }

@@ -443,14 +443,13 @@ __device__ __forceinline__ void traceQueue(const DScene &S, const uint32_t *queu
   TraceState s;
   s.cur = kTraceDone;
   s.post = 0;
-  s.sp = 0;
   Hit best;
   uint32_t entry = 0;
   bool busy = false, ended = false, occluded = false;
   for (;;) {
-    unsigned long long idle = __ballot(!busy);
-    if (idle == ~0ull || (bBase < n && __popcll(idle) >= REFILL)) {
-      if (__any(ended))
+    unsigned long long idle = waveMask(!busy);
+    if (idle == ~0ull || (bBase < n && __builtin_popcountll(idle) >= REFILL)) {
+      if (waveMask(ended) != 0ull)
         finish(ended, entry, best, occluded, s);
       ended = false;
       while (idle != 0ull && bBase < n) {
@@ -465,11 +464,11 @@ __device__ __forceinline__ void traceQueue(const DScene &S, const uint32_t *queu
           vec3f org, dir;
           float t0, tfar;
           load(entry, org, dir, t0, tfar);
-          traceBegin(s, S, org, dir, t0, tfar, best);
+          traceBegin(s, S, org, dir, t0, tfar, best, lds);
         }
-        const int waiting = __popcll(idle);
+        const int waiting = __builtin_popcountll(idle);
         bNext += waiting < avail ? waiting : avail;
-        idle = __ballot(!busy);
+        idle = waveMask(!busy);
         if (bNext == bSize) {
           // a spread queue: the first batches of all waves cover it
           bNext = 0;
@@ -491,7 +490,6 @@ __device__ __forceinline__ void traceQueue(const DScene &S, const uint32_t *queu
       ended = true;
       s.cur = kTraceDone;
       s.post = 0;
-      s.sp = 0;
     }
   }
 }
@@ -1613,7 +1611,7 @@ __global__ __launch_bounds__(kTraceBlock) void k_trace_rays(DScene S, const floa
 
 // The traversal scratch rows of hpt_trace_rays_noalloc: a file-scope device
 // array, kThreadRow words for each thread of at most kNoAllocTraceBlocks
-// resident blocks (62 MiB).  Every GPU that runs the module holds its own
+// resident blocks (64 MiB).  Every GPU that runs the module holds its own
 // copy until the process ends; host code reaches it only through the
 // address hipGetSymbolAddress returns on that GPU, looked up once per
 // device on the first call there.
@@ -1928,6 +1926,6 @@ int hpt_trace_noalloc_max_blocks() { return kNoAllocTraceBlocks; }
 int hpt_trace_block_size() { return kTraceBlock; }
 int hpt_overflow_depth() { return kThreadRow; }
 int hpt_trans_record_hits() { return kTransRecHits; }
-int hpt_stack_capacity() { return kLdsDepth + kOverflowDepth; }
+int hpt_stack_capacity() { return kStackCapacity; }
 
 } // extern "C"

@@ -39,7 +39,11 @@ namespace hpt {
 
 constexpr int kTraceBlock = 128;
 constexpr int kLdsDepth = 24;
-constexpr int kOverflowDepth = 104;
+constexpr int kOverflowDepth = 108;
+// entries a tree may need: the rows but the sentinel's, rounded down so that
+// the recorded hits stay 16-byte aligned
+constexpr int kStackCapacity = 128;
+static_assert(kStackCapacity < kLdsDepth + kOverflowDepth && kOverflowDepth % 4 == 0, "stack rows");
 // transparent hits an occlusion traversal records for the transparency pass
 constexpr int kTransRecHits = 4;
 // words of scratch per resident traversal thread: the stack overflow, then
@@ -531,7 +535,8 @@ struct TraceState
   TriPre pc;
   float t0, tfar;
   float tb; // hits beyond it are of no interest: the closest one (with TIES, a near-tie beyond it)
-  int inst, modelOffset, sp, cur, post;
+  int inst, modelOffset, cur, post;
+  int sp; // see stackAt
   bool tie;            // a near-tie of the current closest hit has been seen (TIES != TIES_OFF)
   bool sawTransparent; // MODE_OCCLUSION: a non-opaque primitive was hit
 };
@@ -540,7 +545,7 @@ struct TraceState
 constexpr int kTraceDone = 0x7ffffffe;
 
 __device__ __forceinline__ void traceBegin(
-    TraceState &s, const DScene &S, vec3f worg, vec3f wdir, float t0, float tfar, Hit &best)
+    TraceState &s, const DScene &S, vec3f worg, vec3f wdir, float t0, float tfar, Hit &best, uint32_t *lds)
 {
   best.hit = false;
   best.t = tfar;
@@ -559,33 +564,49 @@ __device__ __forceinline__ void traceBegin(
   s.tb = tfar;
   s.inst = -1;
   s.modelOffset = 0;
-  s.sp = 0;
+  lds[threadIdx.x] = (uint32_t)kTraceDone;
+  s.sp = 4 * ((int)threadIdx.x + kTraceBlock); // entry 1 (kStackRow)
   s.cur = S.tlasRoot;
   s.post = 0;
   s.tie = false;
   s.sawTransparent = false;
 }
 
-// callers check sp < kLdsDepth + kOverflowDepth before pushing
-__device__ __forceinline__ void tracePush(TraceState &s, uint32_t *lds, uint32_t *ovf, int v)
+// The stack of a lane: s.sp is the byte offset in the block's LDS rows of
+// the next free entry (row d of lane l at d * kStackRow + 4 l), entries from
+// row kLdsDepth on live in the overflow row.  Entry 0 is kTraceDone, so a
+// pop needs no test for an empty stack.
+constexpr int kStackRow = 4 * kTraceBlock;
+constexpr int kStackLds = kLdsDepth * kStackRow;
+
+__device__ __forceinline__ uint32_t *stackAt(uint32_t *lds, int sp)
 {
-  if (s.sp < kLdsDepth)
-    lds[s.sp * kTraceBlock + threadIdx.x] = (uint32_t)v;
-  else
-    ovf[s.sp - kLdsDepth] = (uint32_t)v;
-  s.sp++;
+  return reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(lds) + sp);
 }
 
-// the LDS read is unconditional (a clamped slot), the overflow row is read
+// the entry's word in the overflow row (sp >= kStackLds)
+__device__ __forceinline__ uint32_t *overflowAt(uint32_t *ovf, int sp) { return ovf + (sp / kStackRow - kLdsDepth); }
+
+// callers check that the stack holds another entry
+__device__ __forceinline__ void tracePush(TraceState &s, uint32_t *lds, uint32_t *ovf, int v)
+{
+  if (s.sp < kStackLds)
+    *stackAt(lds, s.sp) = (uint32_t)v;
+  else
+    *overflowAt(ovf, s.sp) = (uint32_t)v;
+  s.sp += kStackRow;
+}
+
+// the LDS read is unconditional (a clamped row), the overflow row is read
 // only by the rare lanes whose stack is deeper than kLdsDepth (a volatile
 // read, so the compiler keeps the two reads apart instead of merging them
 // into one generic-address load)
-__device__ __forceinline__ int tracePop(TraceState &s, const uint32_t *lds, const uint32_t *ovf)
+__device__ __forceinline__ int tracePop(TraceState &s, uint32_t *lds, uint32_t *ovf)
 {
-  s.sp--;
-  int v = (int)lds[(s.sp < kLdsDepth ? s.sp : kLdsDepth - 1) * kTraceBlock + threadIdx.x];
-  if (s.sp >= kLdsDepth)
-    v = (int)*reinterpret_cast<const volatile uint32_t *>(ovf + (s.sp - kLdsDepth));
+  s.sp -= kStackRow;
+  int v = (int)*stackAt(lds, s.sp < kStackLds ? s.sp : 4 * (int)threadIdx.x);
+  if (s.sp >= kStackLds)
+    v = (int)*reinterpret_cast<const volatile uint32_t *>(overflowAt(ovf, s.sp));
   return v;
 }
 
@@ -603,6 +624,10 @@ __device__ __forceinline__ int tracePop(TraceState &s, const uint32_t *lds, cons
 // held instance leaf is entered from the world level, with the next world
 // node pushed below the marker.  Lanes with cur == kTraceDone and no held
 // leaf (finished or idle) only take part in the wave vote.
+// the lanes of the wave for which x holds (__ballot takes an int, which
+// costs two more vector instructions)
+__device__ __forceinline__ unsigned long long waveMask(bool x) { return __builtin_amdgcn_ballot_w64(x); }
+
 // a lane that needs traceLeaf: it holds a leaf or stands at the exit of an
 // instance
 __device__ __forceinline__ bool traceHolds(const TraceState &s) { return s.post != 0 || s.cur == kMarker; }
@@ -612,7 +637,7 @@ __device__ __forceinline__ void traceDescend(
     TraceState &s, const DScene &S, uint32_t *lds, uint32_t *ovf, TraceStats &st)
 {
   for (;;) {
-    if (s.cur >= 0 && s.cur < kTraceDone) {
+    if ((uint32_t)s.cur < (uint32_t)kTraceDone) {
       const Node4 nd = loadNode(S.nodes, s.cur);
       if (STATS)
         st.nodes++;
@@ -626,28 +651,28 @@ __device__ __forceinline__ void traceDescend(
       cswap(t1c, c1, t3c, c3);
       cswap(t1c, c1, t2c, c2);
       if (t0c == kInf) {
-        s.cur = s.sp == 0 ? kTraceDone : tracePop(s, lds, ovf);
+        s.cur = tracePop(s, lds, ovf);
       } else {
-        const int npush = (t1c != kInf) + (t2c != kInf) + (t3c != kInf);
-        if (s.sp + 3 <= kLdsDepth) {
+        const bool h1 = t1c != kInf, h2 = t2c != kInf, h3 = t3c != kInf;
+        const int grow = h3 ? 3 * kStackRow : (h2 ? 2 * kStackRow : (h1 ? kStackRow : 0));
+        if (s.sp < kStackLds - 2 * kStackRow) {
           // the children after the nearest, farthest first: the sorted
-          // boxes that were hit are a prefix, so the npush entries pushed
-          // are c_npush .. c1; the slots above them get don't-care copies
-          uint32_t *top = lds + s.sp * kTraceBlock + threadIdx.x;
-          top[0] = (uint32_t)(npush == 3 ? c3 : (npush == 2 ? c2 : c1));
-          top[kTraceBlock] = (uint32_t)(npush == 3 ? c2 : c1);
+          // boxes that were hit are a prefix, so the entries pushed are the
+          // last child hit .. c1; the rows above them get don't-care copies
+          uint32_t *top = stackAt(lds, s.sp);
+          top[0] = (uint32_t)(h3 ? c3 : (h2 ? c2 : c1));
+          top[kTraceBlock] = (uint32_t)(h3 ? c2 : c1);
           top[2 * kTraceBlock] = (uint32_t)c1;
-          s.sp += npush;
+          s.sp += grow;
           s.cur = c0;
-        } else if (s.sp + npush > kLdsDepth + kOverflowDepth) { // cannot happen: the world commit checks the stack need
+        } else if (s.sp + grow >= (kLdsDepth + kOverflowDepth + 1) * kStackRow) { // cannot happen: the world commit checks the stack need
           s.cur = kTraceDone;
-          s.sp = 0;
         } else {
-          if (t3c != kInf)
+          if (h3)
             tracePush(s, lds, ovf, c3);
-          if (t2c != kInf)
+          if (h2)
             tracePush(s, lds, ovf, c2);
-          if (t1c != kInf)
+          if (h1)
             tracePush(s, lds, ovf, c1);
           s.cur = c0;
         }
@@ -655,10 +680,11 @@ __device__ __forceinline__ void traceDescend(
     }
     if (s.cur < 0 && s.post == 0) { // hold the leaf, go on
       s.post = s.cur;
-      s.cur = s.sp == 0 ? kTraceDone : tracePop(s, lds, ovf);
+      s.cur = tracePop(s, lds, ovf);
     }
-    const unsigned long long searching = __ballot(s.cur >= 0 && s.cur < kTraceDone && s.post == 0);
-    if (__popcll(searching) <= __popcll(__ballot(traceHolds(s))))
+    const unsigned long long holding = waveMask(s.post != 0) | waveMask(s.cur == kMarker);
+    const unsigned long long stepping = waveMask((uint32_t)s.cur < (uint32_t)kTraceDone);
+    if (__builtin_popcountll(stepping & ~holding) <= __builtin_popcountll(holding))
       break;
   }
 }
@@ -686,10 +712,9 @@ __device__ __forceinline__ bool traceLeaf(TraceState &s, const DScene &S, Hit &b
       s.box = boxRay(s.o, s.d, I.extent);
       s.pc = triPrecompute(s.d);
       s.modelOffset = I.modelOffset;
-      if (s.sp + 2 > kLdsDepth + kOverflowDepth)
+      if (s.sp + kStackRow >= (kLdsDepth + kOverflowDepth) * kStackRow) // cannot happen, as above
         return true;
-      if (s.cur != kTraceDone)
-        tracePush(s, lds, ovf, s.cur);
+      tracePush(s, lds, ovf, s.cur); // kTraceDone too: it goes back where it came from
       tracePush(s, lds, ovf, kMarker);
       s.cur = I.blasRoot;
       return false;
@@ -779,7 +804,7 @@ __device__ __forceinline__ bool traceLeaf(TraceState &s, const DScene &S, Hit &b
     s.d = s.wdir;
     s.box = boxRay(s.worg, s.wdir, S.extent);
     s.inst = -1;
-    s.cur = s.sp == 0 ? kTraceDone : tracePop(s, lds, ovf);
+    s.cur = tracePop(s, lds, ovf);
   }
   return s.cur == kTraceDone;
 }
@@ -789,7 +814,7 @@ __device__ bool traceRay(const DScene &S, vec3f worg, vec3f wdir, float t0, floa
     uint32_t *lds, uint32_t *ovf, bool &sawTransparent, TraceStats &st)
 {
   TraceState s;
-  traceBegin(s, S, worg, wdir, t0, tfar, best);
+  traceBegin(s, S, worg, wdir, t0, tfar, best, lds);
   bool occluded = false;
   for (;;) {
     traceDescend<STATS>(s, S, lds, ovf, st);
