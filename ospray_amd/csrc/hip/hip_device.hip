@@ -2206,6 +2206,9 @@ void World::commit() // World.cpp:70-188 plus the Group BLAS builds (Group.cpp:9
     std::memcpy(di.xfm, x, 48);
     di.blasRoot = blasNodeOff[blasSlot[&B]];
     di.modelOffset = groupModelOffset[gi];
+    di.allOpaque = 1;
+    for (size_t k = 0; k < groups[gi]->models.size(); k++)
+      di.allOpaque &= models[groupModelOffset[gi] + k].opaque;
     di.userID = I.userID;
     di.extent = boxExtent(B.bounds);
     di.epsScale = hpt::maxf(std::fabs(x[0]), hpt::maxf(std::fabs(x[4]), std::fabs(x[8])));
@@ -2270,7 +2273,7 @@ void World::commit() // World.cpp:70-188 plus the Group BLAS builds (Group.cpp:9
   D.gpu();
   HIP_CHECK(hipStreamSynchronize(D.stream)); // frames in flight read the old arrays
   dNodes.ensure(sizeof(hpt::DNode4) * totalNodeCount);
-  dPrims.ensure(sizeof(hpt::DPrim) * nPrims);
+  dPrims.ensure(sizeof(hpt::DPrim) * (nPrims + 1)); // the leaf test reads records in pairs
   hpt::DNode4 *gNodes = dNodes.as<hpt::DNode4>();
   hpt::DPrim *gPrims = dPrims.as<hpt::DPrim>();
   HIP_CHECK(hipMemsetAsync(gPrims, 0, sizeof(hpt::DPrim), D.stream));

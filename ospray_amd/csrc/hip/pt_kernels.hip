@@ -443,7 +443,7 @@ __device__ __forceinline__ void traceQueue(const DScene &S, const uint32_t *queu
   TraceState s;
   s.cur = kTraceDone;
   s.post = 0;
-  Hit best;
+  TraceHit best;
   uint32_t entry = 0;
   bool busy = false, ended = false, occluded = false;
   for (;;) {
@@ -482,7 +482,7 @@ __device__ __forceinline__ void traceQueue(const DScene &S, const uint32_t *queu
       if (idle == ~0ull) // the queue is exhausted and every lane waits
         break;
     }
-    traceDescend<STATS>(s, S, lds, ovf, st);
+    traceDescend<MODE, STATS>(s, S, lds, ovf, st);
     if (busy
         && (traceHolds(s) ? traceLeaf<MODE, STATS, RECORD, TIES>(s, S, best, lds, ovf, st, occluded)
                           : s.cur == kTraceDone)) {
@@ -515,9 +515,10 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(5))
         t0 = o.w;
         tfar = kInf;
       },
-      [&](bool ended, uint32_t p, const Hit &h, bool, const TraceState &ts) {
+      [&](bool ended, uint32_t p, const TraceHit &best, bool, const TraceState &ts) {
         if (!ended)
           return;
+        const Hit h = hitFromTrace(S, ts.worg, ts.wdir, ts.t0, best);
         st4(P.hitA + 4 * (size_t)p, h.hit ? h.t : kInf, h.u, h.v, __uint_as_float(h.hit ? h.inst : kInvalidID));
         st4(P.hitB + 4 * (size_t)p, h.Ng.x, h.Ng.y, h.Ng.z, __uint_as_float(h.model));
         P.hitPrim[p] = h.prim | (h.half << 31);
@@ -1149,7 +1150,7 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(6))
         t0 = 0.f;
         tfar = o4.w;
       },
-      [&](bool ended, uint32_t r, const Hit &, bool occluded, const TraceState &ts) {
+      [&](bool ended, uint32_t r, const TraceHit &, bool occluded, const TraceState &ts) {
         bool toTrans = false;
         const bool sawT = ended && ts.sawTransparent;
         if (ended) {

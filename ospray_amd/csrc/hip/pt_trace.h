@@ -83,27 +83,33 @@ __device__ __forceinline__ float boxInv(float d)
   return __builtin_amdgcn_rcpf(ad < 1e-18f ? copysignf(1e-18f, d) : d);
 }
 
+// The shear of the watertight test along the ray's largest axis kz, with
+// the other two axes in cyclic order.  (Exchanging them for a negative
+// direction, as the paper does, negates U, V, W and their sum exactly and
+// with them nothing of t, u, v: the sign tests are symmetric.)
 struct TriPre
 {
-  int kx, ky, kz;
+  int kz;
   float Sx, Sy, Sz;
 };
+
+// component kz of a and the two after it
+HPT_HD void rotateTo(int kz, vec3f a, float &x, float &y, float &z)
+{
+  x = kz == 0 ? a.y : (kz == 1 ? a.z : a.x);
+  y = kz == 0 ? a.z : (kz == 1 ? a.x : a.y);
+  z = kz == 0 ? a.x : (kz == 1 ? a.y : a.z);
+}
 
 HPT_HD TriPre triPrecompute(vec3f dir)
 {
   TriPre p;
   const vec3f ad = vabs(dir);
   p.kz = ad.x > ad.y ? (ad.x > ad.z ? 0 : 2) : (ad.y > ad.z ? 1 : 2);
-  p.kx = p.kz == 2 ? 0 : p.kz + 1;
-  p.ky = p.kx == 2 ? 0 : p.kx + 1;
-  if (comp(dir, p.kz) < 0.0f) {
-    const int t = p.kx;
-    p.kx = p.ky;
-    p.ky = t;
-  }
-  const float dz = comp(dir, p.kz);
-  p.Sx = comp(dir, p.kx) / dz;
-  p.Sy = comp(dir, p.ky) / dz;
+  float dx, dy, dz;
+  rotateTo(p.kz, dir, dx, dy, dz);
+  p.Sx = dx / dz;
+  p.Sy = dy / dz;
   p.Sz = 1.0f / dz;
   return p;
 }
@@ -111,16 +117,16 @@ HPT_HD TriPre triPrecompute(vec3f dir)
 HPT_HD bool intersectTriangle(vec3f org, float t0, const TriPre &pc, vec3f v0, vec3f v1, vec3f v2, float tmax,
     float &t, float &u, float &v)
 {
-  const vec3f A = v0 - org;
-  const vec3f B = v1 - org;
-  const vec3f C = v2 - org;
-  const float Az_ = comp(A, pc.kz), Bz_ = comp(B, pc.kz), Cz_ = comp(C, pc.kz);
-  const float Ax = comp(A, pc.kx) - pc.Sx * Az_;
-  const float Ay = comp(A, pc.ky) - pc.Sy * Az_;
-  const float Bx = comp(B, pc.kx) - pc.Sx * Bz_;
-  const float By = comp(B, pc.ky) - pc.Sy * Bz_;
-  const float Cx = comp(C, pc.kx) - pc.Sx * Cz_;
-  const float Cy = comp(C, pc.ky) - pc.Sy * Cz_;
+  float Ax_, Ay_, Az_, Bx_, By_, Bz_, Cx_, Cy_, Cz_;
+  rotateTo(pc.kz, v0 - org, Ax_, Ay_, Az_);
+  rotateTo(pc.kz, v1 - org, Bx_, By_, Bz_);
+  rotateTo(pc.kz, v2 - org, Cx_, Cy_, Cz_);
+  const float Ax = Ax_ - pc.Sx * Az_;
+  const float Ay = Ay_ - pc.Sy * Az_;
+  const float Bx = Bx_ - pc.Sx * Bz_;
+  const float By = By_ - pc.Sy * Bz_;
+  const float Cx = Cx_ - pc.Sx * Cz_;
+  const float Cy = Cy_ - pc.Sy * Cz_;
   const float U = Cx * By - Cy * Bx;
   const float V = Ax * Cy - Ay * Cx;
   const float W = Bx * Ay - By * Ax;
@@ -523,6 +529,16 @@ __device__ void resolveNearTie(const DScene &S, vec3f worg, vec3f wdir, float t0
 // and its registers out of the traversal kernel
 constexpr int TIES_OFF = 0, TIES_RESOLVE = 1, TIES_REPORT = 2;
 
+// The closest hit as a traversal keeps it: what depends on the primitive
+// alone (model, ids, normal) is read again from its record once the ray has
+// ended (hitFromTrace), so an update in the leaf loop is five moves.
+struct TraceHit
+{
+  float t, u, v;  // u, v of the record's own triangle
+  uint32_t inst;
+  uint32_t prim; // index into DScene::prims, kInvalidID: no hit
+};
+
 // Per-lane state of one traversal.  A traversal runs as rounds of
 // traceDescend (inner nodes, speculative while-while) and traceLeaf (the
 // leaf the lane holds); traceRay runs one ray to its end, traceQueue (in
@@ -530,12 +546,13 @@ constexpr int TIES_OFF = 0, TIES_RESOLVE = 1, TIES_REPORT = 2;
 struct TraceState
 {
   vec3f worg, wdir; // the world ray
-  vec3f o, d;       // the current (world or object) ray
-  BoxRay box;       // of the current ray
+  vec3f o;          // origin of the object ray (inside an instance)
+  BoxRay box;       // of the current (world or object) ray
   TriPre pc;
   float t0, tfar;
   float tb; // hits beyond it are of no interest: the closest one (with TIES, a near-tie beyond it)
-  int inst, modelOffset, cur, post;
+  int inst, cur, post;
+  int modelOffset;     // MODE_OCCLUSION: the instance's first model, -1 if all are opaque
   int sp; // see stackAt
   bool tie;            // a near-tie of the current closest hit has been seen (TIES != TIES_OFF)
   bool sawTransparent; // MODE_OCCLUSION: a non-opaque primitive was hit
@@ -545,25 +562,21 @@ struct TraceState
 constexpr int kTraceDone = 0x7ffffffe;
 
 __device__ __forceinline__ void traceBegin(
-    TraceState &s, const DScene &S, vec3f worg, vec3f wdir, float t0, float tfar, Hit &best, uint32_t *lds)
+    TraceState &s, const DScene &S, vec3f worg, vec3f wdir, float t0, float tfar, TraceHit &best, uint32_t *lds)
 {
-  best.hit = false;
   best.t = tfar;
   best.u = best.v = 0.f;
-  best.Ng = v3(0.f);
-  best.inst = best.model = best.prim = kInvalidID;
-  best.half = 0;
+  best.inst = best.prim = kInvalidID;
   s.worg = worg;
   s.wdir = wdir;
   s.o = worg;
-  s.d = wdir;
   s.box = boxRay(worg, wdir, S.extent);
-  s.pc = {0, 1, 2, 0.f, 0.f, 0.f};
+  s.pc = {0, 0.f, 0.f, 0.f};
   s.t0 = t0;
   s.tfar = tfar;
   s.tb = tfar;
   s.inst = -1;
-  s.modelOffset = 0;
+  s.modelOffset = -1;
   lds[threadIdx.x] = (uint32_t)kTraceDone;
   s.sp = 4 * ((int)threadIdx.x + kTraceBlock); // entry 1 (kStackRow)
   s.cur = S.tlasRoot;
@@ -632,7 +645,7 @@ __device__ __forceinline__ unsigned long long waveMask(bool x) { return __builti
 // instance
 __device__ __forceinline__ bool traceHolds(const TraceState &s) { return s.post != 0 || s.cur == kMarker; }
 
-template <bool STATS>
+template <int MODE, bool STATS>
 __device__ __forceinline__ void traceDescend(
     TraceState &s, const DScene &S, uint32_t *lds, uint32_t *ovf, TraceStats &st)
 {
@@ -642,7 +655,7 @@ __device__ __forceinline__ void traceDescend(
       if (STATS)
         st.nodes++;
       float tc[4];
-      nodeNear(nd, s.box, s.t0, s.tb, tc);
+      nodeNear(nd, s.box, MODE == MODE_OCCLUSION ? 0.f : s.t0, s.tb, tc); // shadow rays start at 0
       float t0c = tc[0], t1c = tc[1], t2c = tc[2], t3c = tc[3];
       int c0 = nd.child.x, c1 = nd.child.y, c2 = nd.child.z, c3 = nd.child.w;
       cswap(t0c, c0, t1c, c1);
@@ -689,119 +702,195 @@ __device__ __forceinline__ void traceDescend(
   }
 }
 
+__device__ __forceinline__ void objectRay(const DInstance &I, vec3f worg, vec3f wdir, vec3f &o, vec3f &d)
+{
+  const linear3f rl = {{I.rcp[0], I.rcp[1], I.rcp[2]}, {I.rcp[3], I.rcp[4], I.rcp[5]}, {I.rcp[6], I.rcp[7], I.rcp[8]}};
+  o = mul(rl, worg) + v3(I.rcp[9], I.rcp[10], I.rcp[11]);
+  d = mul(rl, wdir);
+}
+
+// model, primitive and half of a record
+__device__ __forceinline__ void primKey(const DScene &S, uint32_t index, uint32_t &model, uint32_t &prim, uint32_t &half)
+{
+  const DPrim &P = S.prims[index];
+  model = P.modelKind & 0x0fffffffu;
+  prim = P.primID;
+  half = (P.modelKind >> 28) == PRIM_QUAD1 ? 1u : 0u;
+}
+
+// the order of two hits at the same distance (rare: kept out of line)
+__device__ __forceinline__ bool primLess(const DScene &S, uint32_t inst, uint32_t prim, const TraceHit &best)
+{
+  Hit b;
+  uint32_t m, p, h;
+  primKey(S, prim, m, p, h);
+  primKey(S, best.prim, b.model, b.prim, b.half);
+  b.inst = best.inst;
+  return keyLess(inst, m, p, h, b);
+}
+
+// the hit record of a traversal's result: the same primitive test on the
+// same object ray gives a sphere's normal bit for bit
+__device__ __forceinline__ Hit hitFromTrace(const DScene &S, vec3f worg, vec3f wdir, float t0, const TraceHit &b)
+{
+  Hit h;
+  h.hit = b.prim != kInvalidID;
+  h.t = b.t;
+  h.u = b.u;
+  h.v = b.v;
+  h.Ng = v3(0.f);
+  h.inst = h.model = h.prim = kInvalidID;
+  h.half = 0;
+  if (h.hit) {
+    const float4 *P = reinterpret_cast<const float4 *>(S.prims + b.prim);
+    const float4 pa = P[0], pb = P[1], pc = P[2];
+    const uint32_t mk = __float_as_uint(pb.w), kind = mk >> 28;
+    const vec3f A = v3(pa.x, pa.y, pa.z);
+    h.inst = b.inst;
+    h.model = mk & 0x0fffffffu;
+    h.prim = __float_as_uint(pa.w);
+    if (kind == PRIM_SPHERE) {
+      vec3f o, d;
+      objectRay(S.instances[b.inst], worg, wdir, o, d);
+      intersectSphere(o, d, t0, A, pb.x, b.t, h.t, h.Ng);
+    } else {
+      h.Ng = cross(v3(pb.x, pb.y, pb.z) - A, v3(pc.x, pc.y, pc.z) - A);
+      if (kind == PRIM_QUAD1) {
+        h.half = 1;
+        h.u = 1.0f - h.u;
+        h.v = 1.0f - h.v;
+      }
+    }
+  }
+  return h;
+}
+
+// The words of a primitive record the test needs, each a register of its
+// own (held as the loaded quads they would be allocated, and spilled, four
+// at a time).
+struct PrimWords
+{
+  vec3f A, B, C;
+  uint32_t mk;
+};
+
+__device__ __forceinline__ PrimWords primWords(float4 a, float4 b, float4 c)
+{
+  return {v3(a.x, a.y, a.z), v3(b.x, b.y, b.z), v3(c.x, c.y, c.z), __float_as_uint(b.w)};
+}
+
+// One primitive record (index k) of the current instance.
+// Returns true for an opaque occluder (MODE_OCCLUSION).
+template <int MODE, bool RECORD, int TIES>
+__device__ __forceinline__ bool tracePrim(
+    TraceState &s, const DScene &S, TraceHit &best, const PrimWords &w, uint32_t k, uint32_t *ovf)
+{
+  const uint32_t mk = w.mk;
+  float t, u = 0.f, v = 0.f, tX = 0.f;
+  int roots = 1;
+  if (mk >> 28 != PRIM_SPHERE) {
+    if (!intersectTriangle(s.o, MODE == MODE_OCCLUSION ? 0.f : s.t0, s.pc, w.A, w.B, w.C, s.tb, t, u, v))
+      return false;
+  } else {
+    // the object direction again, rather than three registers held for it
+    vec3f o, d, NE, NX;
+    objectRay(S.instances[s.inst], s.worg, s.wdir, o, d);
+    roots = sphereRoots(o, d, MODE == MODE_OCCLUSION ? 0.f : s.t0, w.A, w.B.x, s.tb, t, NE, tX, NX);
+    if (roots == 0)
+      return false;
+    if (MODE == MODE_CLOSEST && !(roots & 1))
+      t = tX;
+  }
+  if (MODE == MODE_OCCLUSION) {
+    if (s.modelOffset < 0 || S.models[s.modelOffset + (int)(mk & 0x0fffffffu)].opaque)
+      return true;
+    s.sawTransparent = true;
+    if (RECORD) {
+      if (roots & 1)
+        recordHit(ovf, t, (uint32_t)s.inst, k, 0);
+      if (roots & 2)
+        recordHit(ovf, tX, (uint32_t)s.inst, k, 1);
+    }
+    return false;
+  }
+  const bool any = best.prim != kInvalidID;
+  const bool nt = TIES != TIES_OFF && any && nearTie(t, best.t);
+  // t <= tfar: without a hit yet every hit is the closest
+  if (!any || t < best.t || (t == best.t && primLess(S, (uint32_t)s.inst, k, best))) {
+    if (TIES != TIES_OFF)
+      s.tie = nt; // a hit below the window of the previous closest one clears the flag
+    // (the reporting traversal's rays have no far end)
+    s.tb = TIES == TIES_OFF ? t : (TIES == TIES_REPORT ? t + kTieEps * t : fminf(t + kTieEps * t, s.tfar));
+    best.t = t;
+    best.u = u;
+    best.v = v;
+    best.inst = (uint32_t)s.inst;
+    best.prim = k;
+  } else if (nt) {
+    s.tie = true;
+  }
+  return false;
+}
+
 // What a lane holds (traceHolds): an instance leaf enters the instance's
 // BLAS with the object ray; a BLAS leaf tests its primitives; the marker
 // leaves the instance.  Returns true when the lane's traversal has ended: no node left, an
 // opaque occluder (MODE_OCCLUSION, `occluded` set) or a full stack.
 template <int MODE, bool STATS, bool RECORD, int TIES>
-__device__ __forceinline__ bool traceLeaf(TraceState &s, const DScene &S, Hit &best, uint32_t *lds, uint32_t *ovf,
+__device__ __forceinline__ bool traceLeaf(TraceState &s, const DScene &S, TraceHit &best, uint32_t *lds, uint32_t *ovf,
     TraceStats &st, bool &occluded)
 {
   if (s.post != 0) {
     const uint32_t enc = ~(uint32_t)s.post;
     s.post = 0;
     const uint32_t first = enc >> 3;
-    const uint32_t count = (enc & 7u) + 1u;
-    if (s.inst < 0) {
+    // An instance's transform and a primitive record are both three 16-byte
+    // words, and a BLAS leaf holds at most two records as a rule: six loads
+    // fetch what either kind of leaf needs, so a round waits for memory once
+    // and not for the instances, the first and the second records in turn.
+    // (Once the node loop leaves early, leaf rounds are half of the work;
+    // 1080p terrain at 4 spp, streams serialised, with the lean hit update
+    // below: k_extend 6.43 -> 5.71 ms, k_shadow 7.65 -> 6.97 ms.)
+    const bool enter = s.inst < 0;
+    const float4 *P = enter ? reinterpret_cast<const float4 *>(S.instances + first)
+                            : reinterpret_cast<const float4 *>(S.prims + first);
+    const float4 r0 = P[0], r1 = P[1], r2 = P[2], r3 = P[3], r4 = P[4], r5 = P[5];
+    if (enter) {
       // world leaf: one instance; continue in its BLAS with the object ray
       s.inst = (int)first;
-      const DInstance &I = S.instances[s.inst];
-      const linear3f rl = {{I.rcp[0], I.rcp[1], I.rcp[2]}, {I.rcp[3], I.rcp[4], I.rcp[5]}, {I.rcp[6], I.rcp[7], I.rcp[8]}};
-      s.o = mul(rl, s.worg) + v3(I.rcp[9], I.rcp[10], I.rcp[11]);
-      s.d = mul(rl, s.wdir);
-      s.box = boxRay(s.o, s.d, I.extent);
-      s.pc = triPrecompute(s.d);
-      s.modelOffset = I.modelOffset;
+      const linear3f rl = {{r0.x, r0.y, r0.z}, {r0.w, r1.x, r1.y}, {r1.z, r1.w, r2.x}};
+      s.o = mul(rl, s.worg) + v3(r2.y, r2.z, r2.w);
+      const vec3f d = mul(rl, s.wdir);
+      s.box = boxRay(s.o, d, r3.w);
+      s.pc = triPrecompute(d);
+      if (MODE == MODE_OCCLUSION)
+        s.modelOffset = __float_as_int(r3.z) ? -1 : __float_as_int(r3.y);
       if (s.sp + kStackRow >= (kLdsDepth + kOverflowDepth) * kStackRow) // cannot happen, as above
         return true;
       tracePush(s, lds, ovf, s.cur); // kTraceDone too: it goes back where it came from
       tracePush(s, lds, ovf, kMarker);
-      s.cur = I.blasRoot;
+      s.cur = __float_as_int(r3.x);
       return false;
     }
-    const float t0 = s.t0;
-    for (uint32_t k = 0; k < count; k++) {
-      const DPrim &P = S.prims[first + k];
-      const float4 pa = reinterpret_cast<const float4 *>(&P)[0];
-      const float4 pb = reinterpret_cast<const float4 *>(&P)[1];
-      const float4 pcv = reinterpret_cast<const float4 *>(&P)[2];
-      const uint32_t primID = __float_as_uint(pa.w);
-      const uint32_t mk = __float_as_uint(pb.w);
-      const uint32_t model = mk & 0x0fffffffu;
-      const uint32_t kind = mk >> 28;
+    const uint32_t end = first + (enc & 7u) + 1u;
+    PrimWords w = primWords(r0, r1, r2), next = primWords(r3, r4, r5);
+    for (uint32_t k = first;;) {
       if (STATS)
         st.prims++;
-      if (MODE == MODE_OCCLUSION && kind == PRIM_SPHERE) {
-        float tE, tX;
-        vec3f NE, NX;
-        const int roots = sphereRoots(s.o, s.d, t0, v3(pa.x, pa.y, pa.z), pb.x, s.tb, tE, NE, tX, NX);
-        if (!roots)
-          continue;
-        if (S.models[s.modelOffset + model].opaque) {
-          occluded = true;
-          return true;
-        }
-        s.sawTransparent = true;
-        if (RECORD) {
-          if (roots & 1)
-            recordHit(ovf, tE, (uint32_t)s.inst, first + k, 0);
-          if (roots & 2)
-            recordHit(ovf, tX, (uint32_t)s.inst, first + k, 1);
-        }
-        continue;
+      if (tracePrim<MODE, RECORD, TIES>(s, S, best, w, k, ovf)) {
+        occluded = true;
+        return true;
       }
-      float t, u = 0.f, v = 0.f;
-      vec3f Ng;
-      bool h;
-      uint32_t half = 0;
-      if (kind == PRIM_SPHERE) {
-        h = intersectSphere(s.o, s.d, t0, v3(pa.x, pa.y, pa.z), pb.x, s.tb, t, Ng);
-      } else {
-        const vec3f A = v3(pa.x, pa.y, pa.z), B = v3(pb.x, pb.y, pb.z), C = v3(pcv.x, pcv.y, pcv.z);
-        h = intersectTriangle(s.o, t0, s.pc, A, B, C, s.tb, t, u, v);
-        if (h) {
-          Ng = cross(B - A, C - A);
-          if (kind == PRIM_QUAD1) {
-            half = 1;
-            u = 1.0f - u;
-            v = 1.0f - v;
-          }
-        }
+      if (++k == end)
+        break;
+      if (k != first + 1) {
+        const float4 *N = reinterpret_cast<const float4 *>(S.prims + k);
+        next = primWords(N[0], N[1], N[2]);
       }
-      if (!h)
-        continue;
-      if (MODE == MODE_OCCLUSION) {
-        if (S.models[s.modelOffset + model].opaque) {
-          occluded = true;
-          return true;
-        }
-        s.sawTransparent = true;
-        if (RECORD)
-          recordHit(ovf, t, (uint32_t)s.inst, first + k, 0);
-        continue;
-      }
-      const bool nt = TIES != TIES_OFF && best.hit && nearTie(t, best.t);
-      if (better(t, (uint32_t)s.inst, model, primID, half, best)) {
-        if (TIES != TIES_OFF)
-          s.tie = nt; // a hit below the window of the previous closest one clears the flag
-        s.tb = TIES != TIES_OFF ? fminf(t + kTieEps * t, s.tfar) : t;
-        best.hit = true;
-        best.t = t;
-        best.u = u;
-        best.v = v;
-        best.Ng = Ng;
-        best.inst = (uint32_t)s.inst;
-        best.model = model;
-        best.prim = primID;
-        best.half = half;
-      } else if (nt) {
-        s.tie = true;
-      }
+      w = next;
     }
   }
   if (s.cur == kMarker) {
-    s.o = s.worg;
-    s.d = s.wdir;
     s.box = boxRay(s.worg, s.wdir, S.extent);
     s.inst = -1;
     s.cur = tracePop(s, lds, ovf);
@@ -814,21 +903,23 @@ __device__ bool traceRay(const DScene &S, vec3f worg, vec3f wdir, float t0, floa
     uint32_t *lds, uint32_t *ovf, bool &sawTransparent, TraceStats &st)
 {
   TraceState s;
-  traceBegin(s, S, worg, wdir, t0, tfar, best, lds);
+  TraceHit hit;
+  traceBegin(s, S, worg, wdir, t0, tfar, hit, lds);
   bool occluded = false;
   for (;;) {
-    traceDescend<STATS>(s, S, lds, ovf, st);
+    traceDescend<MODE, STATS>(s, S, lds, ovf, st);
     if (!traceHolds(s)) {
       if (s.cur == kTraceDone) // no node left
         break;
       continue; // other lanes hold leaves
     }
-    if (traceLeaf<MODE, STATS, RECORD, TIES>(s, S, best, lds, ovf, st, occluded))
+    if (traceLeaf<MODE, STATS, RECORD, TIES>(s, S, hit, lds, ovf, st, occluded))
       break;
   }
   sawTransparent = s.sawTransparent;
-  if (MODE == MODE_OCCLUSION && occluded)
-    return true;
+  if (MODE == MODE_OCCLUSION)
+    return occluded;
+  best = hitFromTrace(S, worg, wdir, t0, hit);
   if (TIES == TIES_RESOLVE && s.tie)
     resolveNearTie<STATS>(S, worg, wdir, t0, tfar, best, lds, ovf, st);
   if (TIES == TIES_REPORT)
@@ -843,10 +934,8 @@ __device__ bool traceRay(const DScene &S, vec3f worg, vec3f wdir, float t0, floa
 __device__ __forceinline__ void hitFromRecord(const DScene &S, vec3f worg, vec3f wdir, float4 r, Hit &h)
 {
   const uint32_t inst = __float_as_uint(r.y);
-  const DInstance &I = S.instances[inst];
-  const linear3f rl = {{I.rcp[0], I.rcp[1], I.rcp[2]}, {I.rcp[3], I.rcp[4], I.rcp[5]}, {I.rcp[6], I.rcp[7], I.rcp[8]}};
-  const vec3f o = mul(rl, worg) + v3(I.rcp[9], I.rcp[10], I.rcp[11]);
-  const vec3f d = mul(rl, wdir);
+  vec3f o, d;
+  objectRay(S.instances[inst], worg, wdir, o, d);
   const DPrim &P = S.prims[__float_as_uint(r.z)];
   const float4 pa = reinterpret_cast<const float4 *>(&P)[0];
   const float4 pb = reinterpret_cast<const float4 *>(&P)[1];

@@ -73,14 +73,16 @@ static_assert(sizeof(DPrim) == 48, "prim size");
 
 struct DInstance
 {
+  // what a ray needs to enter the instance: 64 B
   float rcp[12]; // inverse transform: columns vx, vy, vz, p
-  float xfm[12]; // forward transform
   int32_t blasRoot; // node index of the group's BLAS root
   int32_t modelOffset; // first DModel of the group
+  int32_t allOpaque; // every model of the group is opaque
+  float extent; // largest |coordinate| of the BLAS's bounds (0: no geometry)
+  float xfm[12]; // forward transform
   uint32_t userID; // kInvalidID if unset
   float epsScale; // max(|xfm.vx.x|, |xfm.vy.y|, |xfm.vz.z|)
-  float extent; // largest |coordinate| of the BLAS's bounds (0: no geometry)
-  int32_t pad[3];
+  int32_t pad[2];
 };
 static_assert(sizeof(DInstance) == 128, "instance size");
 
