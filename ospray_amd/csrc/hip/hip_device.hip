@@ -1051,7 +1051,7 @@ class HipDevice : public Device
   bool capturing = false; // enqueuing a batch of views into a HIP graph
   // ospCancel: pinned host words, one per frame generation modulo
   // kCancelRing; cancelling frame g writes g into word g % kCancelRing,
-  // which the frame's per-bounce counter resets read
+  // which the start of each pass and the shading of each bounce read
   static constexpr uint32_t kCancelRing = 256;
   uint32_t *cancelRing = nullptr, *cancelRingDev = nullptr;
   uint32_t frameGen = 0;
@@ -1167,10 +1167,8 @@ class HipDevice : public Device
         HIP_CHECK(hipStreamCreateWithFlags(&L->stream, hipStreamNonBlocking));
         L->ownsStream = true;
       }
-      L->counters.ensure(4 * hpt::kCounterWords);
       if (residentTraceBlocks > 0)
         ensureScratch(*L);
-      L->paths.counters = L->counters.as<int32_t>();
       L->paths.overflow = L->overflow.as<uint32_t>();
       L->paths.stats = (unsigned long long *)stats.ptr;
       lanes.push_back(std::move(L));
@@ -1502,6 +1500,7 @@ class HipDevice : public Device
   OSPPickResult pick(ManagedObject *fbo, ManagedObject *ro, ManagedObject *co, ManagedObject *wo, float x, float y) override;
 
   void ensurePaths(size_t slots, int maxRec, bool aux);
+  void ensureCounters(int bounces);
 
   // ---- batched views (no reference counterpart) ----
   // Many views (framebuffer, renderer, camera) of one world in one
@@ -2489,9 +2488,21 @@ void HipDevice::ensurePaths(size_t slots, int maxRec, bool aux)
   paths.transHits = (float *)L.transBuf.ptr;
   paths.transCount = (uint32_t *)((char *)L.transBuf.ptr + transHitBytes);
   paths.transCap = (int32_t)transCap;
-  paths.counters = L.counters.as<int32_t>();
   paths.overflow = L.overflow.as<uint32_t>();
   paths.stats = (unsigned long long *)stats.ptr;
+}
+
+// the lane's counters for passes of `bounces` bounces
+void HipDevice::ensureCounters(int bounces)
+{
+  const size_t bytes = 4 * hpt::counterWords(bounces);
+  if (lane->counters.bytes >= bytes)
+    return;
+  if (capturing)
+    throw std::runtime_error("batched views: counters would grow while capturing");
+  releaseGraph(); // a captured batch refers to the old ones
+  HIP_CHECK(hipStreamSynchronize(lane->stream));
+  lane->counters.ensure(bytes);
 }
 
 void HipDevice::ensureNrc(size_t slots)
@@ -2526,7 +2537,7 @@ void HipDevice::nrcPass(Renderer *r, World *w)
   const hipStream_t stream = lane->stream;
   const HptPaths *P = reinterpret_cast<const HptPaths *>(&paths);
   int32_t cnt[2] = {0, 0};
-  HIP_CHECK(hipMemcpyAsync(cnt, paths.counters + hpt::kCntNrcQuery, sizeof(cnt), hipMemcpyDeviceToHost, stream));
+  HIP_CHECK(hipMemcpyAsync(cnt, paths.pass + hpt::kPassNrcQuery, sizeof(cnt), hipMemcpyDeviceToHost, stream));
   HIP_CHECK(hipStreamSynchronize(stream));
   const int nQ = cnt[0], nT = cnt[1];
   r->nrcQueries += nQ;
@@ -2698,6 +2709,8 @@ ManagedObject *HipDevice::renderFrame(ManagedObject *fbo, ManagedObject *ro, Man
   F.fbObjID = fb->objID.as<uint32_t>();
   F.fbInstID = fb->instID.as<uint32_t>();
   F.taskVariance = fb->taskVar.as<float>();
+  F.fbConverted = fb->color.ptr && fb->format != OSP_FB_NONE ? fb->converted.ptr : nullptr;
+  F.fbFormat = (int)fb->format;
   // LocalFrameBuffer::getRenderTaskIDs (fb/LocalFB.cpp:238-261) with
   // minimumAdaptiveFrames = max(2, 16 / spp) (fb/FrameBuffer.h:183-186)
   if (r->errorThreshold > 0.f && fb->variance.ptr && fb->frameID >= std::max(2, 16 / std::max(1, r->spp)))
@@ -2743,6 +2756,7 @@ ManagedObject *HipDevice::renderFrame(ManagedObject *fbo, ManagedObject *ro, Man
     for (int k = nl - 1; k >= 0; k--) {
       lane = k == 0 ? frameLane : &ensureLane(k);
       ensurePaths((size_t)sppPerPass * F.numPixPadded, F.maxRec, aux);
+      ensureCounters(F.maxDepth + 1);
       lane->paths.aux = aux ? lane->auxBase : nullptr;
       lane->paths.overflow = lane->overflow.as<uint32_t>();
     }
@@ -2766,10 +2780,10 @@ ManagedObject *HipDevice::renderFrame(ManagedObject *fbo, ManagedObject *ro, Man
     if (travStats)
       HIP_CHECK(hpt_fill_u32((uint32_t *)stats.ptr, 32, 0u, stream));
     uint32_t *const latch = capturing ? nullptr : fb->cancelLatch.as<uint32_t>();
-    if (latch)
-      HIP_CHECK(hpt_fill_u32(latch, 1, 0u, stream));
     F.cancelLatch = latch;
-    if (nl > 1) { // fork: the other lanes start after the frame's earlier work
+    if (nl > 1) {
+      if (latch) // before any lane's passes
+        HIP_CHECK(hpt_fill_u32(latch, 1, 0u, stream)); // fork: the other lanes start after the frame's earlier work
       HIP_CHECK(hipEventRecord(laneEvents[0], stream));
       for (int k = 1; k < nl; k++)
         HIP_CHECK(hipStreamWaitEvent(lanes[k]->stream, laneEvents[0], 0));
@@ -2780,7 +2794,15 @@ ManagedObject *HipDevice::renderFrame(ManagedObject *fbo, ManagedObject *ro, Man
       lane->paths.cancelFlag = latch ? cancelRingDev + fut->gen % kCancelRing : nullptr;
       lane->paths.cancelGen = fut->gen;
       lane->paths.cancelLatch = latch;
-      const HptPaths *P = reinterpret_cast<const HptPaths *>(&lane->paths);
+      hpt::DPaths &paths = lane->paths;
+      const HptPaths *P = reinterpret_cast<const HptPaths *>(&paths);
+      paths.pass = lane->counters.as<int32_t>();
+      // the counters of bounce b
+      auto atBounce = [&](hpt::DPaths &p, int b) {
+        p.counters = p.pass + hpt::kPassWords + (size_t)b * hpt::kBounceWords;
+        p.next = p.counters + hpt::kBounceWords;
+      };
+      atBounce(paths, 0);
       F.passS0 = s0;
       F.passCount = std::min(sppPerPass, F.spp - s0);
       if (F.nrcBounce >= 0) { // every stride-th slot of the pass trains the cache
@@ -2797,7 +2819,7 @@ ManagedObject *HipDevice::renderFrame(ManagedObject *fbo, ManagedObject *ro, Man
       Fno.nrcBounce = -1;
       const HptFrame *Fp = reinterpret_cast<const HptFrame *>(&F);
       const HptFrame *FpNo = reinterpret_cast<const HptFrame *>(&Fno);
-      launch("reset", [&]() { return hpt_reset_counters(P, -1, stream); });
+      launch("reset", [&]() { return hpt_begin_pass(P, F.maxDepth + 1, nl == 1 && pass == 0 ? 1 : 0, stream); });
       launch("generate", [&]() { return hpt_generate(Fp, P, stream); });
       // with self-training no path goes beyond the vertex after the cache's
       // (in worlds without volumes: training paths from volume vertices run
@@ -2806,9 +2828,8 @@ ManagedObject *HipDevice::renderFrame(ManagedObject *fbo, ManagedObject *ro, Man
       if (F.nrcBounce >= 0 && F.nrcSelfTrain && !F.hasVolumes)
         lastBounce = std::min(F.maxDepth, F.nrcBounce + 1);
       // Shadow stages of bounce b on the lane's side stream, beside the
-      // extension of bounce b + 1 (they read and write disjoint path state;
-      // the side stream has its own traversal scratch rows and resets its
-      // own counters).  The shading of bounce b + 1 (and the free-path
+      // extension of bounce b + 1 (they read and write disjoint path state
+      // and counters; the side stream has its own traversal scratch rows).  The shading of bounce b + 1 (and the free-path
       // sampling, which shares the paths' volume sampler with the
       // transmittance estimates) waits for bounce b's resolve, so every
       // contribution is added in the same order as on one stream.
@@ -2824,10 +2845,8 @@ ManagedObject *HipDevice::renderFrame(ManagedObject *fbo, ManagedObject *ro, Man
       for (int b = 0; b <= lastBounce; b++) {
         const std::string at = profile && profileBounces ? "@" + std::to_string(b) : std::string();
         auto nm = [&](const char *stage) { return at.empty() ? std::string(stage) : stage + at; };
-        if (overlap)
-          launch(nm("reset").c_str(), [&]() { return hpt_reset_extension_counters(P, q, stream); });
-        else
-          launch(nm("reset").c_str(), [&]() { return hpt_reset_counters(P, q, stream); });
+        atBounce(paths, b);
+        atBounce(sidePaths, b);
         launch(nm("extend").c_str(),
             [&]() { return hpt_extend(S, P, q, residentTraceBlocks, travStats ? 1 : 0, stream); });
         launch(nm("ties").c_str(), [&]() { return hpt_ties(S, P, tieBlocks(), travStats ? 1 : 0, stream); });
@@ -2835,8 +2854,6 @@ ManagedObject *HipDevice::renderFrame(ManagedObject *fbo, ManagedObject *ro, Man
           HIP_CHECK(hipStreamWaitEvent(stream, lane->evRes[pendingRes & 1], 0));
           pendingRes = -1;
         }
-        if (overlap)
-          launch(nm("reset").c_str(), [&]() { return hpt_reset_append_counters(P, q, stream); });
         if (F.hasVolumes)
           launch(nm("volume").c_str(), [&]() { return hpt_volume(S, P, q, volBlocks, travStats ? 1 : 0, stream); });
         launch(nm("shade").c_str(),
@@ -2851,7 +2868,6 @@ ManagedObject *HipDevice::renderFrame(ManagedObject *fbo, ManagedObject *ro, Man
           if (overlap) {
             HIP_CHECK(hipEventRecord(lane->evShade[b & 1], stream));
             HIP_CHECK(hipStreamWaitEvent(side, lane->evShade[b & 1], 0));
-            launch(nm("reset").c_str(), [&]() { return hpt_reset_shadow_counters(PS, side); }, side);
           }
           launch(nm("nee").c_str(), [&]() { return hpt_nee(S, Fp, PS, q, shadeBlocks, shadowStream); }, shadowStream);
           launch(nm("shadow").c_str(),
@@ -2898,7 +2914,6 @@ ManagedObject *HipDevice::renderFrame(ManagedObject *fbo, ManagedObject *ro, Man
     if (!capturing)
       HIP_CHECK(hipEventRecord(fut->rendered, stream));
     const HptFrame *Fp = reinterpret_cast<const HptFrame *>(&F);
-    launch("fb_accumulate", [&]() { return hpt_fb_accumulate(Fp, stream); });
     // LocalFrameBuffer::postProcess (LocalFB.cpp:459-478)
     // (a captured frame runs them on every launch; they check the device-
     // resident frame index and do their work after odd frames)
@@ -2912,11 +2927,6 @@ ManagedObject *HipDevice::renderFrame(ManagedObject *fbo, ManagedObject *ro, Man
       if (!capturing) // a captured batch leaves the error estimate on the device
         HIP_CHECK(hipMemcpyAsync(fb->hostVariance, fb->varianceOut.ptr, sizeof(float), hipMemcpyDeviceToHost, stream));
       fb->varianceValid = true;
-    }
-    if (fb->color.ptr && fb->format != OSP_FB_NONE) {
-      launch("color_convert", [&]() {
-        return hpt_color_convert(F.fbColor, F.width * F.height, (int)fb->format, fb->converted.ptr, stream);
-      });
     }
   } else {
     if (!capturing)

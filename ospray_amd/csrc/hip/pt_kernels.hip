@@ -1,8 +1,8 @@
 // Wavefront path-tracing kernels for gfx950 and their C-ABI launch layer.
 //
 // One frame = for each pass of samples: generate -> (extend -> shade ->
-// shadow -> resolve) x (maxPathLength+1) -> finish_pass; then fb_accumulate,
-// variance (odd frames) and colour conversion.  This splits the reference's
+// shadow -> resolve) x (maxPathLength+1) -> finish_pass (the last pass's also
+// accumulates and converts); then the variance estimate on odd frames.  This splits the reference's
 // per-pixel megakernel (PathTracer_renderTask, PathTracer.ispc:218-249;
 // samplePath, PathSampler.ispc:109-415) into coherent stages:
 //   extend  closest-hit traversal only (LDS stack, lean registers);
@@ -188,40 +188,49 @@ __device__ __forceinline__ vec2f pixelFilterSample(const DFrame &F, vec2f s, con
 
 // ---- kernels ----------------------------------------------------------------------
 
-// Zeroes the counters whose bit is set in `mask`.  A cancelled frame (the
-// host wrote its generation into *cancelFlag, or the latch is already set)
-// latches *cancelLatch and also zeroes counter `keep` (the entry count of
-// the extension queue being read), so the frame's remaining kernels find no
-// work.  One wave: lane 0's reads are broadcast.
-__global__ void k_reset(int32_t *counters, uint32_t mask, int32_t keep, const uint32_t *cancelFlag, uint32_t gen,
-    uint32_t *cancelLatch)
+// The host's cancellation of a frame (it wrote the frame's generation into
+// *cancelFlag): one thread latches it for the frame's kernels
+__device__ __forceinline__ void latchCancel(const DPaths &P)
 {
-  const int i = globalId();
-  uint32_t cancelled = 0u;
-  if (cancelLatch) {
-    if (i == 0) {
-      cancelled = __hip_atomic_load(cancelLatch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (!cancelled && cancelFlag)
-        cancelled = __hip_atomic_load(cancelFlag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) == gen ? 1u : 0u;
-    }
-    cancelled = __shfl(cancelled, 0);
-  }
-  if (i < kCntFetchExtend) {
-    if (((mask >> i) & 1u) || (cancelled && i == keep))
-      counters[i] = 0;
-  } else if (i < kCntFetchExtend + 2 * kXcds) { // the fetch counters of a traversal
-    const int k = i - kCntFetchExtend;
-    if ((mask >> (k < kXcds ? kCntFetchExtend : kCntFetchShadow)) & 1u)
-      counters[kFetchBase + k * kFetchStride] = 0;
-  }
-  if (cancelled && i == 0)
-    __hip_atomic_store(cancelLatch, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (P.cancelLatch && __hip_atomic_load(P.cancelFlag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) == P.cancelGen)
+    __hip_atomic_store(P.cancelLatch, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// the frame's cancellation latch (read by kernels that run once per pass)
+// The start of a pass: clears its counters, one block for each bounce, and
+// on a frame's first pass the frame's cancellation latch.  Kernels of a
+// bounce then find their counters clear without a launch in between (three
+// resets a bounce were 12 of its 95 us on a 64x64 frame: 613 -> 563 us).
+__global__ __launch_bounds__(256) void k_begin_pass(DPaths P, uint32_t words, int first)
+{
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < words; i += gridDim.x * blockDim.x)
+    P.pass[i] = 0;
+  if (blockIdx.x == 0 && threadIdx.x == 0 && P.cancelLatch) {
+    if (first)
+      __hip_atomic_store(P.cancelLatch, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    latchCancel(P);
+  }
+}
+
+// the frame's cancellation latch
 __device__ __forceinline__ bool frameCancelled(const uint32_t *latch)
 {
   return latch && __hip_atomic_load(latch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u;
+}
+
+// The entries a bounce kernel has to work on: none once the frame is
+// cancelled.  Waves of one kernel may disagree (the latch is set while they
+// start), so a kernel with barriers asks in one thread (blockEntries).
+__device__ __forceinline__ int queueEntries(const DPaths &P, const int32_t *counter)
+{
+  return frameCancelled(P.cancelLatch) ? 0 : *counter;
+}
+__device__ __forceinline__ int blockEntries(const DPaths &P, const int32_t *counter)
+{
+  __shared__ int n;
+  if (threadIdx.x == 0)
+    n = queueEntries(P, counter);
+  __syncthreads();
+  return n;
 }
 
 __global__ void k_fill_u32(uint32_t *p, size_t n, uint32_t v)
@@ -333,13 +342,13 @@ __global__ __launch_bounds__(256) void k_generate(DFrame F, DPaths P)
         P.queue[0][pos] = (uint32_t)i;
       }
     } else {
-      const int slot = enqueue(&P.counters[0], valid); // extension queue 0
+      const int slot = enqueue(&P.counters[kCntExtend], valid);
       if (valid)
         P.queue[0][slot] = (uint32_t)i;
     }
   }
   if (adaptive == 0.f && globalId() == 0)
-    P.counters[0] = F.passCount * F.width * F.height;
+    P.counters[kCntExtend] = F.passCount * F.width * F.height;
 }
 
 // Work distribution of the traversal kernels: each wave takes batches of
@@ -500,13 +509,13 @@ template <bool STATS>
 __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(5))) void k_extend(DScene S, DPaths P, int qin)
 {
   __shared__ uint32_t lds[kLdsDepth * kTraceBlock];
-  const int n = P.counters[2 * qin];
+  const int n = queueEntries(P, &P.counters[kCntExtend]);
   if (n == 0) // an empty queue: no work fetch
     return;
   uint32_t *ovf = P.overflow + (size_t)globalId() * kThreadRow;
   TraceStats st = {0, 0};
   uint32_t rays = 0;
-  traceQueue<MODE_CLOSEST, STATS, false, TIES_REPORT, kExtendRefill>(S, P.queue[qin], n, P.counters + kFetchBase, lds, ovf, st,
+  traceQueue<MODE_CLOSEST, STATS, false, TIES_REPORT, kExtendRefill>(S, P.queue[qin], n, P.counters + kCntFetchExtend, lds, ovf, st,
       [&](uint32_t p, vec3f &org, vec3f &dir, float &t0, float &tfar) {
         const float4 o = ld4(P.org + 4 * (size_t)p);
         const float4 d = ld4(P.dir + 4 * (size_t)p);
@@ -540,7 +549,7 @@ template <bool STATS>
 __global__ __launch_bounds__(kTraceBlock) void k_ties(DScene S, DPaths P)
 {
   __shared__ uint32_t lds[kLdsDepth * kTraceBlock];
-  const int n = P.counters[kCntTies];
+  const int n = queueEntries(P, &P.counters[kCntTies]);
   uint32_t *ovf = P.overflow + (size_t)globalId() * kThreadRow;
   TraceStats st = {0, 0};
   for (int i = globalId(); i < n; i += gridStride()) {
@@ -578,7 +587,7 @@ __global__ __launch_bounds__(kTraceBlock) void k_ties(DScene S, DPaths P)
 // pass is [t0, inf) (no clipping geometry).
 __global__ __launch_bounds__(256) void k_volume(DScene S, DPaths P, int qin, int stats)
 {
-  const int n = P.counters[2 * qin];
+  const int n = queueEntries(P, &P.counters[kCntExtend]);
   VolCount cnt;
   for (int w0 = globalId() - laneId(); w0 < n; w0 += gridStride()) {
     const int i = w0 + laneId();
@@ -619,8 +628,10 @@ __global__ __launch_bounds__(256) void k_volume(DScene S, DPaths P, int qin, int
 template <bool VOL, bool NRC>
 __global__ __launch_bounds__(256, 3) void k_shade(DScene S, DFrame F, DPaths P, int qin)
 {
-  const int n = P.counters[2 * qin];
+  const int n = blockEntries(P, &P.counters[kCntExtend]);
   const int qout = qin ^ 1;
+  if (blockIdx.x == 0 && threadIdx.x == 0)
+    latchCancel(P); // for the kernels after this one
   VolCount vcnt; // transmittance work of the virtual-light MIS weights
   // block-uniform iterations: the queue appends are aggregated per block
   for (int b0 = (int)(blockIdx.x * blockDim.x); b0 < n; b0 += (int)(gridDim.x * blockDim.x)) {
@@ -895,17 +906,17 @@ __global__ __launch_bounds__(256, 3) void k_shade(DScene S, DFrame F, DPaths P, 
       P.neeN[p] = nNee;
     }
     if (NRC) {
-      const int qs = enqueue(&P.counters[kCntNrcQuery], nrcQuery);
+      const int qs = enqueue(&P.pass[kPassNrcQuery], nrcQuery);
       if (nrcQuery)
         P.nrcQueryQueue[qs] = p;
-      const int ts = enqueue(&P.counters[kCntNrcTrain], nrcTrain);
+      const int ts = enqueue(&P.pass[kPassNrcTrain], nrcTrain);
       if (nrcTrain)
         P.nrcTrainQueue[ts] = p;
     }
     // the continuing path to extension queue qout; the light-sample slots of
     // this vertex (records p*maxRec + [0, nNee)) to the NEE sample queue
     int so, first;
-    blockEnqueuePair(&P.counters[2 * qout], cont, nNee, so, first);
+    blockEnqueuePair(&P.next[kCntExtend], cont, nNee, so, first);
     if (cont)
       P.queue[qout][so] = p;
     for (uint32_t k = 0; k < nNee; k++)
@@ -1038,8 +1049,7 @@ __global__ __launch_bounds__(256) void k_nee(DScene S, DFrame F, DPaths P, int q
   __shared__ uint32_t stageCount, stageBase;
   if (threadIdx.x == 0)
     stageCount = 0;
-  __syncthreads();
-  const int n = P.counters[2 * (qin ^ 1) + 1];
+  const int n = blockEntries(P, &P.next[kCntNee]);
   for (int b0 = blockIdx.x * blockDim.x; b0 < n; b0 += gridDim.x * blockDim.x) {
     const int i = b0 + (int)threadIdx.x;
     bool emit = false;
@@ -1135,13 +1145,13 @@ template <bool STATS>
 __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(6))) void k_shadow(DScene S, DFrame F, DPaths P)
 {
   __shared__ uint32_t lds[kLdsDepth * kTraceBlock];
-  const int n = P.counters[kCntShadow];
+  const int n = queueEntries(P, &P.counters[kCntShadow]);
   if (n == 0) // an empty queue: no work fetch
     return;
   uint32_t *ovf = P.overflow + (size_t)globalId() * kThreadRow;
   TraceStats st = {0, 0};
   uint32_t rays = 0;
-  traceQueue<MODE_OCCLUSION, STATS, true, TIES_OFF, kShadowRefill>(S, P.shadowQueue, n, P.counters + kFetchBase + kXcds * kFetchStride, lds, ovf, st,
+  traceQueue<MODE_OCCLUSION, STATS, true, TIES_OFF, kShadowRefill>(S, P.shadowQueue, n, P.counters + kCntFetchShadow, lds, ovf, st,
       [&](uint32_t r, vec3f &org, vec3f &dir, float &t0, float &tfar) {
         const float4 o4 = ld4(P.recOrg + 4 * (size_t)r);
         const float4 d4 = ld4(P.recDir + 4 * (size_t)r);
@@ -1203,7 +1213,7 @@ template <bool STATS>
 __global__ __launch_bounds__(kTraceBlock) void k_shadow_trans(DScene S, DFrame F, DPaths P)
 {
   __shared__ uint32_t lds[kLdsDepth * kTraceBlock];
-  const int n = P.counters[kCntTrans];
+  const int n = queueEntries(P, &P.counters[kCntTrans]);
   if (n == 0) // an empty queue: no work fetch
     return;
   uint32_t *ovf = P.overflow + (size_t)globalId() * kThreadRow;
@@ -1306,7 +1316,7 @@ __global__ __launch_bounds__(kTraceBlock) void k_shadow_trans(DScene S, DFrame F
 template <bool VOL>
 __global__ __launch_bounds__(256) void k_resolve(DScene S, DFrame F, DPaths P, int qin)
 {
-  const int n = P.counters[2 * qin];
+  const int n = queueEntries(P, &P.counters[kCntExtend]);
   VolCount vcnt;
   for (int i = globalId(); i < n; i += gridStride()) {
     const uint32_t p = P.queue[qin][i];
@@ -1351,14 +1361,98 @@ __global__ __launch_bounds__(256) void k_resolve(DScene S, DFrame F, DPaths P, i
   }
 }
 
+__device__ __forceinline__ float lerpAcc(float old, float nw, float f) { return (1.f - f) * old + f * nw; }
+
+__device__ __forceinline__ uint32_t cvtU8(float f) { return (uint32_t)(255.f * clampf(f) + 0.5f); }
+__device__ __forceinline__ float linearToSrgb(float x)
+{
+  x = clampf(x);
+  return x <= 0.0031308f ? 12.92f * x : 1.055f * fexp(flog(x) * (1.f / 2.4f)) - 0.055f;
+}
+
+// ColorConversion_kernel (fb/frame_ops/ColorConversion.ispc:11-36)
+__device__ __forceinline__ void convertColor(const DFrame &F, int pix, float4 v)
+{
+  if (!F.fbConverted)
+    return;
+  if (F.fbFormat == 3) {
+    st4((float *)F.fbConverted + 4 * (size_t)pix, maxf(v.x, 0.f), maxf(v.y, 0.f), maxf(v.z, 0.f),
+        minf(maxf(v.w, 0.f), 1.f));
+  } else if (F.fbFormat == 1) {
+    ((uint32_t *)F.fbConverted)[pix] = cvtU8(v.x) | (cvtU8(v.y) << 8) | (cvtU8(v.z) << 16) | (cvtU8(v.w) << 24);
+  } else {
+    ((uint32_t *)F.fbConverted)[pix] = cvtU8(linearToSrgb(v.x)) | (cvtU8(linearToSrgb(v.y)) << 8)
+        | (cvtU8(linearToSrgb(v.z)) << 16) | (cvtU8(v.w) << 24);
+  }
+}
+
+// ScreenSample_normalize + LocalFB_accumulateSample (ScreenSample.ih:79-92,
+// fb/LocalFB.ispc:14-78) and the colour's conversion, of a pixel whose
+// samples have all been summed
+__device__ __forceinline__ void accumulatePixel(
+    const DFrame &F, int pix, float4 a, const float aux[12], float z, const uint32_t ids[3], int accumID, bool accVar)
+{
+  const float rspp = 1.0f / (float)F.spp;
+  const float accScale = 1.0f / (float)(accumID + 1);
+  const float accVarScale = 1.0f / (float)(accumID / 2 + 1);
+  const float4 n = make_float4(a.x * rspp, a.y * rspp, a.z * rspp, a.w * rspp);
+  auto blend = [&](float *c, float scale) {
+    float4 r = n;
+    if (!(scale > 0.8f)) {
+      const float4 old = ld4(c);
+      r = make_float4(lerpAcc(old.x, n.x, scale), lerpAcc(old.y, n.y, scale), lerpAcc(old.z, n.z, scale),
+          lerpAcc(old.w, n.w, scale));
+    }
+    st4(c, r.x, r.y, r.z, r.w);
+    return r;
+  };
+  if (F.fbColor)
+    convertColor(F, pix, blend(F.fbColor + 4 * (size_t)pix, accScale));
+  if (F.fbVariance && accVar)
+    blend(F.fbVariance + 4 * (size_t)pix, accVarScale);
+  bool updateIDs = accumID == 0;
+  if (F.fbDepth) {
+    if (accumID > 0 && fabsf(z) < fabsf(F.fbDepth[pix]))
+      updateIDs = true;
+    if (updateIDs)
+      F.fbDepth[pix] = z;
+  }
+  if (updateIDs) {
+    if (F.fbPrimID)
+      F.fbPrimID[pix] = ids[0];
+    if (F.fbObjID)
+      F.fbObjID[pix] = ids[1];
+    if (F.fbInstID)
+      F.fbInstID[pix] = ids[2];
+  }
+  float *dsts[4] = {F.fbPosition, F.fbFirstNormal, F.fbNormal, F.fbAlbedo};
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    float *dst = dsts[k];
+    if (!dst)
+      continue;
+    for (int c = 0; c < 3; c++) {
+      const float v = aux[3 * k + c] * rspp;
+      float *d = dst + 3 * (size_t)pix + c;
+      *d = accScale > 0.8f ? v : lerpAcc(*d, v, accScale);
+    }
+  }
+}
+
 // end of samplePath + ScreenSample_accumulate over the pass's samples
-// (PathSampler.ispc:409-414, PathTracer.ispc:196-197, ScreenSample.ih:59-77)
+// (PathSampler.ispc:409-414, PathTracer.ispc:196-197, ScreenSample.ih:59-77).
+// A frame's last pass goes on to the framebuffer with the sums in registers:
+// HBM bound, and as three kernels the sums and the colour made another trip
+// (1920x1080 at 4 spp 0.118 -> 0.092 ms, on small frames two launches).
 __global__ __launch_bounds__(256) void k_finish_pass(DFrame F, DPaths P)
 {
   if (frameCancelled(F.cancelLatch))
     return;
   const int npix = F.width * F.height;
   const float adaptive = frameAdaptive(F);
+  const bool last = F.passS0 + F.passCount >= F.spp;
+  const int accumID = (int)frameAccumID(F);
+  const bool accVar = frameAccVar(F);
   for (int pix = globalId(); pix < npix; pix += gridStride()) {
     const int ix = pix % F.width, iy = pix / F.width;
     if (!taskActive(F, adaptive, ix, iy))
@@ -1405,6 +1499,10 @@ __global__ __launch_bounds__(256) void k_finish_pass(DFrame F, DPaths P)
         ids[2] = P.ids[4 * p + 2];
       }
     }
+    if (last) {
+      accumulatePixel(F, pix, acc, aux, z, ids, accumID, accVar);
+      continue;
+    }
     st4(F.accRGBA + 4 * (size_t)pix, acc.x, acc.y, acc.z, acc.w);
     if (F.accAux)
       for (int k = 0; k < 12; k++)
@@ -1412,76 +1510,6 @@ __global__ __launch_bounds__(256) void k_finish_pass(DFrame F, DPaths P)
     F.accZ[pix] = z;
     for (int k = 0; k < 3; k++)
       F.accIDs[3 * (size_t)pix + k] = ids[k];
-  }
-}
-
-__device__ __forceinline__ float lerpAcc(float old, float nw, float f) { return (1.f - f) * old + f * nw; }
-
-// ScreenSample_normalize + LocalFB_accumulateSample (ScreenSample.ih:79-92,
-// fb/LocalFB.ispc:14-78)
-__global__ __launch_bounds__(256) void k_fb_accumulate(DFrame F)
-{
-  if (frameCancelled(F.cancelLatch)) // a cancelled frame leaves the framebuffer as it was
-    return;
-  const int npix = F.width * F.height;
-  const float rspp = 1.0f / (float)F.spp;
-  const int accumID = (int)frameAccumID(F);
-  const float accScale = 1.0f / (float)(accumID + 1);
-  const float accVarScale = 1.0f / (float)(accumID / 2 + 1);
-  const bool accVar = frameAccVar(F);
-  const float adaptive = frameAdaptive(F);
-  for (int pix = globalId(); pix < npix; pix += gridStride()) {
-    if (!taskActive(F, adaptive, pix % F.width, pix / F.width))
-      continue;
-    const float4 a = ld4(F.accRGBA + 4 * (size_t)pix);
-    const float r = a.x * rspp, g = a.y * rspp, b = a.z * rspp, al = a.w * rspp;
-    if (F.fbColor) {
-      float *c = F.fbColor + 4 * (size_t)pix;
-      if (accScale > 0.8f)
-        st4(c, r, g, b, al);
-      else {
-        const float4 old = ld4(c);
-        st4(c, lerpAcc(old.x, r, accScale), lerpAcc(old.y, g, accScale), lerpAcc(old.z, b, accScale),
-            lerpAcc(old.w, al, accScale));
-      }
-    }
-    if (F.fbVariance && accVar) {
-      float *c = F.fbVariance + 4 * (size_t)pix;
-      if (accVarScale > 0.8f)
-        st4(c, r, g, b, al);
-      else {
-        const float4 old = ld4(c);
-        st4(c, lerpAcc(old.x, r, accVarScale), lerpAcc(old.y, g, accVarScale), lerpAcc(old.z, b, accVarScale),
-            lerpAcc(old.w, al, accVarScale));
-      }
-    }
-    const float z = F.accZ[pix];
-    bool updateIDs = accumID == 0;
-    if (F.fbDepth) {
-      if (accumID > 0 && fabsf(z) < fabsf(F.fbDepth[pix]))
-        updateIDs = true;
-      if (updateIDs)
-        F.fbDepth[pix] = z;
-    }
-    if (updateIDs) {
-      if (F.fbPrimID)
-        F.fbPrimID[pix] = F.accIDs[3 * (size_t)pix];
-      if (F.fbObjID)
-        F.fbObjID[pix] = F.accIDs[3 * (size_t)pix + 1];
-      if (F.fbInstID)
-        F.fbInstID[pix] = F.accIDs[3 * (size_t)pix + 2];
-    }
-    float *dsts[4] = {F.fbPosition, F.fbFirstNormal, F.fbNormal, F.fbAlbedo};
-    for (int k = 0; k < 4; k++) {
-      float *dst = dsts[k];
-      if (!dst)
-        continue;
-      for (int c = 0; c < 3; c++) {
-        const float v = F.accAux[12 * (size_t)pix + 3 * k + c] * rspp;
-        float *d = dst + 3 * (size_t)pix + c;
-        *d = accScale > 0.8f ? v : lerpAcc(*d, v, accScale);
-      }
-    }
   }
 }
 
@@ -1558,29 +1586,6 @@ __global__ __launch_bounds__(256) void k_variance_reduce(const float *taskVar, i
   }
   if (threadIdx.x == 0)
     out[0] = sCnt[0] ? (float)(sSum[0] / (double)sCnt[0]) : sMax[0];
-}
-
-__device__ __forceinline__ uint32_t cvtU8(float f) { return (uint32_t)(255.f * clampf(f) + 0.5f); }
-__device__ __forceinline__ float linearToSrgb(float x)
-{
-  x = clampf(x);
-  return x <= 0.0031308f ? 12.92f * x : 1.055f * fexp(flog(x) * (1.f / 2.4f)) - 0.055f;
-}
-
-// ColorConversion_kernel (fb/frame_ops/ColorConversion.ispc:11-36)
-__global__ __launch_bounds__(256) void k_color_convert(const float *color, int npix, int format, void *out)
-{
-  for (int i = globalId(); i < npix; i += gridStride()) {
-    const float4 v = ld4(color + 4 * (size_t)i);
-    if (format == 3) {
-      st4((float *)out + 4 * (size_t)i, maxf(v.x, 0.f), maxf(v.y, 0.f), maxf(v.z, 0.f), minf(maxf(v.w, 0.f), 1.f));
-    } else if (format == 1) {
-      ((uint32_t *)out)[i] = cvtU8(v.x) | (cvtU8(v.y) << 8) | (cvtU8(v.z) << 16) | (cvtU8(v.w) << 24);
-    } else {
-      ((uint32_t *)out)[i] = cvtU8(linearToSrgb(v.x)) | (cvtU8(linearToSrgb(v.y)) << 8)
-          | (cvtU8(linearToSrgb(v.z)) << 16) | (cvtU8(v.w) << 24);
-    }
-  }
 }
 
 // closest hits of an explicit ray list (first-hit parity checks and BVH
@@ -1663,52 +1668,11 @@ inline int gridFor(size_t n, int block, int maxBlocks)
 
 extern "C" {
 
-namespace {
-// counter masks: the shadow side of a bounce (records, their work fetch and
-// the transparency queue) and the extension side of the bounce reading queue q
-// (the next queue's pair, the extension work fetch, the near-tie queue)
-constexpr uint32_t kShadowSideMask = (1u << kCntShadow) | (1u << kCntFetchShadow) | (1u << kCntTrans);
-inline uint32_t extensionSideMask(int q)
+hipError_t hpt_begin_pass(const HptPaths *P, int bounces, int firstPass, hipStream_t s)
 {
-  return (3u << (2 * (q ^ 1))) | (1u << kCntFetchExtend) | (1u << kCntTies);
-}
-hipError_t launchReset(const DPaths &p, uint32_t mask, int keep, hipStream_t s)
-{
-  hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, s, p.counters, mask, keep, p.cancelFlag, p.cancelGen,
-      p.cancelLatch);
-  return hipGetLastError();
-}
-} // namespace
-
-hipError_t hpt_reset_counters(const HptPaths *P, int keepIndex, hipStream_t s)
-{
-  const DPaths &p = *reinterpret_cast<const DPaths *>(P);
-  // a full reset clears every counter; the per-bounce reset both sides of a
-  // bounce, keeping the pair of the extension queue being read
-  if (keepIndex < 0)
-    return launchReset(p, (1u << kNumCounters) - 1u, -1, s);
-  return launchReset(p, extensionSideMask(keepIndex) | kShadowSideMask, 2 * keepIndex, s);
-}
-
-hipError_t hpt_reset_extension_counters(const HptPaths *P, int keepIndex, hipStream_t s)
-{
-  const DPaths &p = *reinterpret_cast<const DPaths *>(P);
-  return launchReset(p, (1u << kCntFetchExtend) | (1u << kCntTies), 2 * keepIndex, s);
-}
-
-hipError_t hpt_reset_append_counters(const HptPaths *P, int keepIndex, hipStream_t s)
-{
-  const DPaths &p = *reinterpret_cast<const DPaths *>(P);
-  hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, s, p.counters, 3u << (2 * (keepIndex ^ 1)), -1,
-      (const uint32_t *)nullptr, 0u, (uint32_t *)nullptr);
-  return hipGetLastError();
-}
-
-hipError_t hpt_reset_shadow_counters(const HptPaths *P, hipStream_t s)
-{
-  const DPaths &p = *reinterpret_cast<const DPaths *>(P);
-  hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, s, p.counters, kShadowSideMask, -1,
-      (const uint32_t *)nullptr, 0u, (uint32_t *)nullptr);
+  const uint32_t words = (uint32_t)counterWords(bounces);
+  hipLaunchKernelGGL(k_begin_pass, dim3(gridFor(words, 256, 1024)), dim3(256), 0, s,
+      *reinterpret_cast<const DPaths *>(P), words, firstPass);
   return hipGetLastError();
 }
 
@@ -1868,13 +1832,6 @@ hipError_t hpt_finish_pass(const HptFrame *F, const HptPaths *P, hipStream_t s)
   return hipGetLastError();
 }
 
-hipError_t hpt_fb_accumulate(const HptFrame *F, hipStream_t s)
-{
-  const DFrame &f = *reinterpret_cast<const DFrame *>(F);
-  hipLaunchKernelGGL(k_fb_accumulate, dim3(gridFor((size_t)f.width * f.height, 256, 16384)), dim3(256), 0, s, f);
-  return hipGetLastError();
-}
-
 hipError_t hpt_variance(const HptFrame *F, hipStream_t s)
 {
   const DFrame &f = *reinterpret_cast<const DFrame *>(F);
@@ -1887,12 +1844,6 @@ hipError_t hpt_variance_reduce(const float *taskVariance, int n, float threshold
     const uint32_t *frameState, hipStream_t s)
 {
   hipLaunchKernelGGL(k_variance_reduce, dim3(1), dim3(256), 0, s, taskVariance, n, threshold, out, frameState);
-  return hipGetLastError();
-}
-
-hipError_t hpt_color_convert(const float *color, int npix, int format, void *out, hipStream_t s)
-{
-  hipLaunchKernelGGL(k_color_convert, dim3(gridFor((size_t)npix, 256, 16384)), dim3(256), 0, s, color, npix, format, out);
   return hipGetLastError();
 }
 

@@ -17,6 +17,7 @@
 //   materials, media, lights, light CDF: small tables.
 #pragma once
 
+#include <cstddef>
 #include <cstdint>
 
 namespace hpt {
@@ -255,10 +256,10 @@ struct DPaths
   uint32_t *transQueue; // shadow records that hit only non-opaque surfaces
   uint32_t *neeSampleQueue; // record slots (path * maxRec + sample) to evaluate
   uint32_t *tieQueue; // path slots whose extension hit is re-resolved in FP64
-  // queue counters, see kCnt*: the pair (2q, 2q+1) is one 64-bit word so
-  // that k_shade appends to extension queue q and to the NEE sample queue
-  // with a single atomic
-  int32_t *counters;
+  // counters of the bounce at hand and of the next one (kCnt*), and of the
+  // pass (kPass*): each bounce has a block of its own in one buffer, cleared
+  // once when the pass begins
+  int32_t *counters, *next, *pass;
   uint32_t *overflow; // traversal scratch row per resident thread: stack overflow, recorded hits
   // transparent hits recorded by the occlusion pass for the records of the
   // transparency queue, by queue slot < transCap: 4 float4 and a count
@@ -281,31 +282,35 @@ struct DPaths
   unsigned long long *stats;
   // cancellation (FrameBuffer::cancelFrame, FrameBuffer.cpp:180-187): the
   // host writes the frame's generation into *cancelFlag (pinned host
-  // memory); the per-bounce counter reset reads it and latches
-  // *cancelLatch (device memory, one word per framebuffer, cleared when the
-  // frame begins), after which the frame's kernels do no more work.  Null
-  // in captured frames.
+  // memory); the start of a pass and the shading of each bounce read it and
+  // latch *cancelLatch (device memory, one word per framebuffer, cleared
+  // when the frame begins), after which the frame's kernels do no more work.
+  // Null in captured frames.
   const uint32_t *cancelFlag;
   uint32_t cancelGen;
   uint32_t *cancelLatch;
 };
 
-// queue counters: [2q] entries of extension queue q (q = 0, 1), [2q+1] NEE
-// light samples appended while queue q was filled, then:
-constexpr int kCntShadow = 4; // shadow-ray records
-constexpr int kCntTrans = 5; // records for the transparency pass
-constexpr int kCntTies = 6; // extension rays whose closest hit has a near-tie
-constexpr int kCntNrcQuery = 7; // radiance-cache queries of the pass
-constexpr int kCntNrcTrain = 8; // radiance-cache training records of the pass
-// bits of a reset mask for the work fetch of the extension and the shadow
-// traversal
-constexpr int kCntFetchExtend = 9, kCntFetchShadow = 10;
-constexpr int kNumCounters = 11;
-// Work fetch: one counter per XCD and traversal, each on a cache line of
-// its own, after the counters above
+// A bounce's counters.  The first two words are one 64-bit word, so that
+// the shading of a bounce appends to the next bounce's extension queue and
+// its own light samples to the NEE sample queue with a single atomic.
+constexpr int kCntExtend = 0; // entries of the bounce's extension queue
+constexpr int kCntNee = 1; // NEE light samples appended while that queue was filled
+constexpr int kCntShadow = 2; // shadow-ray records
+constexpr int kCntTrans = 3; // records for the transparency pass
+constexpr int kCntTies = 4; // extension rays whose closest hit has a near-tie
+// work fetch: one counter per XCD and traversal, each on a cache line of
+// its own
 constexpr int kXcds = 8, kFetchStride = 32;
-constexpr int kFetchBase = 32; // word of the extension traversal's first counter
-constexpr int kCounterWords = kFetchBase + 2 * kXcds * kFetchStride;
+constexpr int kCntFetchExtend = 32, kCntFetchShadow = kCntFetchExtend + kXcds * kFetchStride;
+constexpr int kBounceWords = kCntFetchShadow + kXcds * kFetchStride;
+// A pass's counters: the words before its first bounce's
+constexpr int kPassNrcQuery = 0; // radiance-cache queries
+constexpr int kPassNrcTrain = 1; // radiance-cache training records
+constexpr int kPassWords = 32;
+// words of the counters of a pass of `bounces` bounces; the last one's
+// shading has a next block too
+constexpr size_t counterWords(int bounces) { return kPassWords + (size_t)(bounces + 1) * kBounceWords; }
 
 // path flags in ld[3]
 constexpr uint32_t FLAG_DEPTH_MASK = 0xffu; // bits 0-7
@@ -360,6 +365,9 @@ struct DFrame
   float *fbFirstNormal;
   float *fbPosition;
   uint32_t *fbPrimID, *fbObjID, *fbInstID;
+  // the colour as it is mapped (an OSPFrameBufferFormat; null: not mapped)
+  void *fbConverted;
+  int32_t fbFormat;
   float *taskVariance;
   // adaptive accumulation: > 0 renders only the tasks whose taskVariance
   // exceeds it
