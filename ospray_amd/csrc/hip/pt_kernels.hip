@@ -24,6 +24,7 @@
 #include "ospray_hip/hip_pt.h"
 #include "pt_shade.h"
 #include "pt_volume.h"
+#include "pt_wide.h"
 
 using namespace hpt;
 
@@ -410,6 +411,15 @@ __device__ __forceinline__ int nextBatch(Fetch &f, int &size)
 #endif
 constexpr int kExtendRefill = HPT_EXTEND_REFILL, kShadowRefill = HPT_SHADOW_REFILL;
 
+// A queue of at most this many entries per wave of the grid is traversed by
+// whole waves, one ray after another (traceWide): by lanes a launch over few
+// rays lasts as long as the longest one's chain of node fetches, 35 to 75
+// us; a wave needs about 10 us a ray.  Streams serialised, by lanes -> now:
+// 64x64 frame of 82 k triangles k_extend 0.195 -> 0.091 ms, k_shadow 0.157 ->
+// 0.098 ms; 641x359 at 2 spp, 21 bounces 1.59 -> 1.03 and 1.36 -> 0.91 ms
+// (at most 1, 2, 8, 16 entries: k_extend 1.11, 1.06, 1.06, 1.19 ms).
+constexpr int kWideRays = 4;
+
 // Traversal of every entry of a queue with the lanes of each wave kept
 // busy: a lane whose ray has ended waits; once at least REFILL lanes
 // wait (any number once the whole wave waits), the rays that ended are
@@ -419,8 +429,9 @@ constexpr int kExtendRefill = HPT_EXTEND_REFILL, kShadowRefill = HPT_SHADOW_REFI
 // traversal round.  load(entry, org, dir, t0, tfar) gives an entry's ray;
 // finish(ended, entry, best, occluded, state) runs on every lane of the
 // wave (`ended` on the lanes whose ray ended), so it may use wave-wide
-// appends.  A queue shorter than 64 entries per wave of the grid (the
-// last bounces' few paths) is spread over every wave instead: wave w owns
+// appends.  A queue of at most kWideRays entries per wave of the grid is
+// left to whole waves; one shorter than 64 entries per wave (the last
+// bounces' few paths) is spread over every wave: wave w owns
 // the ceil(n / waves) entries from w * ceil(n / waves) on, so the few rays
 // run in many waves side by side rather than 64 to a wave (where each
 // round waits for the slowest of 64 node fetches and the longest of 64
@@ -437,6 +448,21 @@ __device__ __forceinline__ void traceQueue(const DScene &S, const uint32_t *queu
   const int wl = laneId();
   const unsigned long long ltMask = (1ull << wl) - 1ull;
   const int waves = (int)((gridDim.x * blockDim.x) >> 6);
+  if (n <= kWideRays * waves) {
+    static_assert(sizeof(WideLds) <= kLdsDepth * 64 * 4, "wide LDS");
+    WideLds &W = *reinterpret_cast<WideLds *>(lds + (threadIdx.x >> 6) * (kLdsDepth * 64));
+    uint32_t *row0 = ovf - (size_t)wl * kThreadRow;
+    for (int r = __builtin_amdgcn_readfirstlane(globalId() >> 6); r < n; r += waves) {
+      const uint32_t entry = (uint32_t)__builtin_amdgcn_readfirstlane((int)queue[r]);
+      TraceState s;
+      TraceHit best;
+      load(entry, s.worg, s.wdir, s.t0, s.tfar);
+      const bool occluded = traceWide<MODE, STATS, RECORD, TIES>(
+          S, s.worg, s.wdir, s.t0, s.tfar, best, s.tie, s.sawTransparent, W, row0, st);
+      finish(wl == 0, entry, best, occluded, s);
+    }
+    return;
+  }
   const bool spread = HPT_SPREAD_SHORT_QUEUES && n < 64 * waves;
   // wave-uniform batch cursor; a spread queue's batches are the waves' own
   Fetch f = fetchBegin(fetch, n);
@@ -1142,7 +1168,7 @@ __global__ __launch_bounds__(256) void k_nee(DScene S, DFrame F, DPaths P, int q
 // Unoccluded records get their result; records that hit only non-opaque
 // primitives go to the transparency queue (k_shadow_trans).
 template <bool STATS>
-__global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(6))) void k_shadow(DScene S, DFrame F, DPaths P)
+__global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(5))) void k_shadow(DScene S, DFrame F, DPaths P)
 {
   __shared__ uint32_t lds[kLdsDepth * kTraceBlock];
   const int n = queueEntries(P, &P.counters[kCntShadow]);
