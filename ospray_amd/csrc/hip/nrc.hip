@@ -327,23 +327,33 @@ __global__ __launch_bounds__(256) void k_nrc_init(HptNrc N, uint32_t seed)
     reinterpret_cast<__bf16 *>(N.wT)[kOffT[3] + (i / 16) * 32 + 16 + (i & 15)] = (__bf16)0.f;
 }
 
-// 64 parameters per block, the tiles' gradient rows split over 4 groups of
-// 64 threads (group k sums tiles k, k + 4, ... in order) and combined in a
-// fixed order: deterministic
-__global__ __launch_bounds__(256) void k_nrc_adam(HptNrc N, int tiles, float lr, float bc1, float bc2)
+// 64 parameters per block, the tiles' gradient rows split over kAdamGroups
+// waves (wave k sums tiles k, k + kAdamGroups, ... in order) and combined in
+// a fixed order: deterministic.  The rows (94 KB a tile) come from HBM, and
+// a thread waits for its rows in turn: with 4 waves a block (64 rows each of
+// 256 tiles) 35.2 us, 0.69 TB/s; with 16 waves 6.4 us, 3.7 TB/s.
+constexpr int kAdamGroups = 16;
+__global__ __launch_bounds__(64 * kAdamGroups) void k_nrc_adam(HptNrc N, int tiles, float lr, float bc1, float bc2)
 {
-  __shared__ float part[4][64];
+  __shared__ float part[kAdamGroups][64];
   const int col = threadIdx.x & 63, grp = threadIdx.x >> 6;
   for (int p0 = blockIdx.x * 64; p0 < kP; p0 += gridDim.x * 64) {
     const int p = p0 + col;
     float gs = 0.f;
-    if (p < kP)
-      for (int t = grp; t < tiles; t += 4)
+    if (p < kP) {
+#pragma unroll 8
+      for (int t = grp; t < tiles; t += kAdamGroups)
         gs += N.partial[(size_t)t * kP + p];
+    }
     part[grp][col] = gs;
     __syncthreads();
+    for (int h = kAdamGroups / 2; h > 0; h >>= 1) {
+      if (grp < h)
+        part[grp][col] += part[grp + h][col];
+      __syncthreads();
+    }
     if (grp == 0 && p < kP) {
-      const float g = (part[0][col] + part[1][col]) + (part[2][col] + part[3][col]);
+      const float g = part[0][col];
       const float m = 0.9f * N.adamM[p] + 0.1f * g;
       const float v = 0.99f * N.adamV[p] + 0.01f * g * g;
       N.adamM[p] = m;
@@ -352,11 +362,14 @@ __global__ __launch_bounds__(256) void k_nrc_adam(HptNrc N, int tiles, float lr,
     }
     __syncthreads();
   }
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
+  if (blockIdx.x == 0 && grp == 0) {
     float L = 0.f;
-    for (int t = 0; t < tiles; t++)
+    for (int t = col; t < tiles; t += 64)
       L += N.tileLoss[t];
-    N.loss[0] = L;
+    for (int o = 32; o > 0; o >>= 1)
+      L += __shfl_xor(L, o);
+    if (col == 0)
+      N.loss[0] = L;
   }
 }
 
@@ -556,7 +569,7 @@ hipError_t hpt_nrc_adam(const HptNrc *N, int n, float lr, int step, hipStream_t 
   if (tiles <= 0 || tiles > N->maxTiles || step < 1)
     return hipErrorInvalidValue;
   const float bc1 = 1.f - powf(0.9f, (float)step), bc2 = 1.f - powf(0.99f, (float)step);
-  hipLaunchKernelGGL(k_nrc_adam, dim3(gridFor(kP, 64, 1024)), dim3(256), 0, s, *N, tiles, lr, bc1, bc2);
+  hipLaunchKernelGGL(k_nrc_adam, dim3(gridFor(kP, 64, 1024)), dim3(64 * kAdamGroups), 0, s, *N, tiles, lr, bc1, bc2);
   return hipGetLastError();
 }
 
