@@ -1062,7 +1062,7 @@ class HipDevice : public Device
   // profileBounces: the stage timers of the bounce loop are kept per bounce
   // ("extend@2", ...).  overlapShadow: the shadow-ray stages of a bounce run
   // on a second stream beside the next bounce's extension (eager frames of
-  // one lane).
+  // one lane, passes of 2^17 paths or more).
   bool profile = false, travStats = false, profileBounces = false, overlapShadow = true;
   // BLAS build: on the host (binned SAH, the default: about 10 % fewer node
   // visits per ray than the device build on the 4.2M-triangle terrain) or on
@@ -2862,7 +2862,12 @@ ManagedObject *HipDevice::renderFrame(ManagedObject *fbo, ManagedObject *ro, Man
       // sampling, which shares the paths' volume sampler with the
       // transmittance estimates) waits for bounce b's resolve, so every
       // contribution is added in the same order as on one stream.
-      const bool overlap = overlapShadow && nl == 1 && !capturing && !inBatch && F.numFirstLightSamples > 0;
+      // Below 2^17 paths a pass the events between the streams cost more than
+      // the overlap gives (us a frame, two streams / one: 4 k paths 445 / 402,
+      // 16 k 509 / 464, 64 k 600 / 580 and 1184 / 1188, 262 k 796 / 814 and
+      // 1727 / 1815, volume scenes 16 k 1945 / 1850, 256 k 2766 / 2830).
+      const bool overlap = overlapShadow && nl == 1 && !capturing && !inBatch && F.numFirstLightSamples > 0
+          && (size_t)F.passCount * F.numPixPadded >= ((size_t)1 << 17);
       const hipStream_t side = overlap ? ensureSide(*lane) : nullptr;
       hpt::DPaths sidePaths = lane->paths;
       if (overlap)
