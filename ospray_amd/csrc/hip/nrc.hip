@@ -1,7 +1,8 @@
 // Neural radiance cache MLP on the gfx950 matrix cores.
 //
-// Fully fused: one wave runs a tile of 64 queries through every layer, the
-// activations staying in LDS between layers.  Every product is a
+// Fully fused: one wave runs a tile of queries through every layer, the
+// activations staying in registers between layers (training, which needs
+// them again, keeps them in LDS).  Every product is a
 // v_mfma_f32_16x16x32_bf16 (16x16 tile, K = 32, bf16 operands, fp32
 // accumulation).  Operand layout of that instruction, lane l = 16 g + r:
 //   A (16 x 32): row r, k = 8 g .. 8 g + 7      (one 16-byte load)
@@ -51,93 +52,85 @@ __device__ __forceinline__ bf16x8 zero8()
 }
 __device__ __forceinline__ f32x4 zero4() { return f32x4{0.f, 0.f, 0.f, 0.f}; }
 
-// layer 0: acc[nt][qt] = W0 (64 x 160) x X^T for the tile's 64 queries
-// read from the feature rows in HBM (zeros past n)
-__device__ __forceinline__ void layer0(const __bf16 *W, const __bf16 *X, int q0, int n, f32x4 acc[4][4], int r, int g)
+// max(x, 0), 0 for a NaN, in one instruction: fmaxf quiets x in another one
+// first, and so does a median with a bound that the compiler sees as infinity
+__device__ __forceinline__ float relu(float x)
 {
-  for (int nt = 0; nt < 4; nt++)
-    for (int qt = 0; qt < 4; qt++)
-      acc[nt][qt] = zero4();
-  for (int kb = 0; kb < kIn / 32; kb++) {
-    bf16x8 b[4];
-    for (int qt = 0; qt < 4; qt++) {
-      const int q = q0 + qt * 16 + r;
-      b[qt] = q < n ? ld8(X + (size_t)q * kIn + kb * 32 + g * 8) : zero8();
-    }
+  float inf = __builtin_inff();
+  asm("" : "+s"(inf));
+  return __builtin_amdgcn_fmed3f(x, 0.f, inf);
+}
+
+// Layers 1..4 of the forward pass in registers.  The D operand that a layer
+// leaves in lane (r, g) holds query r's neurons 16 nt + 4 g .. + 3, so the
+// next product takes them as its K slots as they are: of K block kb, slots
+// 8 g .. 8 g + 3 are neurons 32 kb + 4 g .. + 3 and slots 8 g + 4 .. 8 g + 7
+// those 16 above, and the weights' columns are read in that order.  No
+// activation goes through LDS.
+// acc[nt][qt]: layer 0's sums in, o[qt]: W4 (16 x 64) x h4; rows 0..2 are
+// the outputs.  wf(layer, row, kb) loads an A operand.
+template <int QT, typename WF>
+__device__ __forceinline__ void forwardTail(const WF &wf, f32x4 (&acc)[4][QT], f32x4 (&o)[QT])
+{
+  bf16x8 h[2][QT];
+#pragma unroll
+  for (int l = 1; l <= 4; l++) {
+    for (int kb = 0; kb < 2; kb++)
+      for (int qt = 0; qt < QT; qt++)
+        for (int e = 0; e < 4; e++) {
+          h[kb][qt][e] = (__bf16)relu(acc[2 * kb][qt][e]);
+          h[kb][qt][4 + e] = (__bf16)relu(acc[2 * kb + 1][qt][e]);
+        }
+    if (l == 4)
+      break;
     for (int nt = 0; nt < 4; nt++) {
-      const bf16x8 a = ld8(W + (nt * 16 + r) * kIn + kb * 32 + g * 8);
-      for (int qt = 0; qt < 4; qt++)
-        acc[nt][qt] = mma(a, b[qt], acc[nt][qt]);
+      for (int qt = 0; qt < QT; qt++)
+        acc[nt][qt] = zero4();
+      for (int kb = 0; kb < 2; kb++) {
+        const bf16x8 a = wf(l, nt * 16, kb);
+        for (int qt = 0; qt < QT; qt++)
+          acc[nt][qt] = mma(a, h[kb][qt], acc[nt][qt]);
+      }
     }
   }
-}
-
-// hidden layer: acc[nt][qt] = W (64 x 64) x act^T, act query-major in LDS
-__device__ __forceinline__ void layer64(const __bf16 *W, const __bf16 *act, f32x4 acc[4][4], int r, int g)
-{
-  for (int nt = 0; nt < 4; nt++)
-    for (int qt = 0; qt < 4; qt++)
-      acc[nt][qt] = zero4();
-  for (int kb = 0; kb < 2; kb++) {
-    bf16x8 b[4];
-    for (int qt = 0; qt < 4; qt++)
-      b[qt] = ld8(act + (qt * 16 + r) * kS + kb * 32 + g * 8);
-    for (int nt = 0; nt < 4; nt++) {
-      const bf16x8 a = ld8(W + (nt * 16 + r) * kH + kb * 32 + g * 8);
-      for (int qt = 0; qt < 4; qt++)
-        acc[nt][qt] = mma(a, b[qt], acc[nt][qt]);
-    }
-  }
-}
-
-// relu(acc) in bf16 to act[q][n] and, when given, to hT[n][q]
-__device__ __forceinline__ void storeAct(const f32x4 acc[4][4], __bf16 *act, __bf16 *hT, int r, int g)
-{
-  for (int nt = 0; nt < 4; nt++)
-    for (int qt = 0; qt < 4; qt++) {
-      const int q = qt * 16 + r, n0 = nt * 16 + 4 * g;
-      bf16x4 v;
-      for (int e = 0; e < 4; e++)
-        v[e] = (__bf16)fmaxf(acc[nt][qt][e], 0.f);
-      *reinterpret_cast<bf16x4 *>(act + q * kS + n0) = v;
-      if (hT)
-        for (int e = 0; e < 4; e++)
-          hT[(n0 + e) * kS + q] = v[e];
-    }
-}
-
-// output layer: o[qt] = W4 (16 x 64) x act^T; rows 0..2 are the outputs
-__device__ __forceinline__ void layerOut(const __bf16 *W4, const __bf16 *act, f32x4 o[4], int r, int g)
-{
-  for (int qt = 0; qt < 4; qt++)
+  for (int qt = 0; qt < QT; qt++)
     o[qt] = zero4();
   for (int kb = 0; kb < 2; kb++) {
-    const bf16x8 a = ld8(W4 + r * kH + kb * 32 + g * 8);
-    for (int qt = 0; qt < 4; qt++)
-      o[qt] = mma(a, ld8(act + (qt * 16 + r) * kS + kb * 32 + g * 8), o[qt]);
+    const bf16x8 a = wf(4, 0, kb);
+    for (int qt = 0; qt < QT; qt++)
+      o[qt] = mma(a, h[kb][qt], o[qt]);
   }
 }
 
 __global__ __launch_bounds__(64) void k_nrc_infer(HptNrc N, const __bf16 *X, int n, float *out)
 {
-  __shared__ __attribute__((aligned(16))) __bf16 act[64 * kS];
   const int lane = threadIdx.x, r = lane & 15, g = lane >> 4;
   const __bf16 *W = reinterpret_cast<const __bf16 *>(N.w);
+  const auto wf = [&](int l, int row, int kb) {
+    const __bf16 *w = W + kOff[l] + (row + r) * kH + kb * 32 + 4 * g;
+    const bf16x4 a = *reinterpret_cast<const bf16x4 *>(w), b = *reinterpret_cast<const bf16x4 *>(w + 16);
+    return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
+  };
   for (int tile = blockIdx.x; tile * 64 < n; tile += gridDim.x) {
     const int q0 = tile * 64;
     f32x4 acc[4][4];
-    layer0(W + kOff[0], X, q0, n, acc, r, g);
-    __syncthreads();
-    storeAct(acc, act, nullptr, r, g);
-    __syncthreads();
-    for (int l = 1; l < 4; l++) {
-      layer64(W + kOff[l], act, acc, r, g);
-      __syncthreads();
-      storeAct(acc, act, nullptr, r, g);
-      __syncthreads();
+    for (int nt = 0; nt < 4; nt++)
+      for (int qt = 0; qt < 4; qt++)
+        acc[nt][qt] = zero4();
+    for (int kb = 0; kb < kIn / 32; kb++) {
+      bf16x8 b[4];
+      for (int qt = 0; qt < 4; qt++) {
+        const int q = q0 + qt * 16 + r;
+        b[qt] = q < n ? ld8(X + (size_t)q * kIn + kb * 32 + g * 8) : zero8();
+      }
+      for (int nt = 0; nt < 4; nt++) {
+        const bf16x8 a = ld8(W + (nt * 16 + r) * kIn + kb * 32 + g * 8);
+        for (int qt = 0; qt < 4; qt++)
+          acc[nt][qt] = mma(a, b[qt], acc[nt][qt]);
+      }
     }
     f32x4 o[4];
-    layerOut(W + kOff[4], act, o, r, g);
+    forwardTail<4>(wf, acc, o);
     if (g == 0)
       for (int qt = 0; qt < 4; qt++) {
         const int q = q0 + qt * 16 + r;
@@ -147,7 +140,6 @@ __global__ __launch_bounds__(64) void k_nrc_infer(HptNrc N, const __bf16 *X, int
           out[3 * (size_t)q + 2] = o[qt][2];
         }
       }
-    __syncthreads();
   }
 }
 
@@ -468,81 +460,77 @@ __global__ __launch_bounds__(256) void k_nrc_encode(const float *raw, int n, flo
 // The path tracer's cache queries in one kernel: gather the queued vertex
 // records (per path slot: P, thr.x | wo, thr.y | Ns, thr.z | albedo, -),
 // encode them in registers, run the network with the weights staged once
-// per block in LDS (8 waves, one 64-query tile each per iteration), and add
-// throughput * max(prediction, 0) to the path's contribution.
-constexpr int kQueryWaves = 8;
-__global__ __launch_bounds__(64 * kQueryWaves) void k_nrc_query(HptNrc N, const float *rec16, const uint32_t *queue,
+// per block in LDS, and add throughput * max(prediction, 0) to the path's
+// contribution.  A wave takes 16 queries at a time.
+//
+// The encoding's VALU work bounds it.  LDS holds the weights only, their
+// rows padded (16 rows of one K chunk on distinct banks), so three blocks of
+// eight waves fit a CU, and a wave's 16 queries keep a short call short.
+// 573,245 queries: with activations in LDS (one block a CU), 64 queries a
+// wave and unpadded rows 98.7 us; without the three 64 queries 63.7, 32
+// queries 46.4, 16 queries 42.9.  1,000 queries: 18.6, 12.6, 8.5, 5.7.
+constexpr int kQueryWaves = 8, kQueryBlocks = 3; // waves a block, blocks a CU
+constexpr int kW0S = 168, kWS = 72; // LDS row strides (bf16) of W0 and of W1..W4
+__global__ __launch_bounds__(64 * kQueryWaves, 6) void k_nrc_query(HptNrc N, const float *rec16, const uint32_t *queue,
     int n, float lx, float ly, float lz, float hx, float hy, float hz, float *contrib4)
 {
-  __shared__ __attribute__((aligned(16))) __bf16 wl[kP];
-  __shared__ __attribute__((aligned(16))) __bf16 actAll[kQueryWaves][64 * kS];
+  __shared__ __attribute__((aligned(16))) __bf16 wl[64 * kW0S + 208 * kWS];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-  __bf16 *act = actAll[wave];
   {
     const bf16x8 *src = reinterpret_cast<const bf16x8 *>(N.w);
-    bf16x8 *dst = reinterpret_cast<bf16x8 *>(wl);
-    for (int i = threadIdx.x; i < kP / 8; i += blockDim.x)
-      dst[i] = src[i];
+    for (int i = threadIdx.x; i < kP / 8; i += 64 * kQueryWaves) {
+      const bf16x8 v = src[i];
+      if (i < kH * kIn / 8) {
+        const int row = i / (kIn / 8);
+        *reinterpret_cast<bf16x8 *>(wl + row * kW0S + (i - row * (kIn / 8)) * 8) = v;
+      } else { // W1..W4: 208 rows of 64, columns in forwardTail's order
+        const int j = i - kH * kIn / 8, row = j >> 3, c = (j & 7) * 8;
+        __bf16 *d = wl + 64 * kW0S + row * kWS + (c & 32) + ((c & 15) >> 2) * 8 + ((c & 16) >> 2);
+        *reinterpret_cast<bf16x4 *>(d) = __builtin_shufflevector(v, v, 0, 1, 2, 3);
+        *reinterpret_cast<bf16x4 *>(d + 8) = __builtin_shufflevector(v, v, 4, 5, 6, 7);
+      }
+    }
   }
   __syncthreads();
+  const auto wf = [&](int l, int row, int kb) {
+    return ld8(wl + 64 * kW0S + ((l - 1) * kH + row + r) * kWS + kb * 32 + g * 8);
+  };
   const float lo[3] = {lx, ly, lz}, inv[3] = {1.f / (hx - lx), 1.f / (hy - ly), 1.f / (hz - lz)};
-  // uniform trip count over the block: every wave reaches every barrier
-  for (int base = blockIdx.x * kQueryWaves * 64; base < n; base += gridDim.x * kQueryWaves * 64) {
-    const int q0 = base + wave * 64;
-    // raw inputs of this lane's 4 queries (tile rows qt * 16 + r)
-    float raw[4][12];
-    for (int qt = 0; qt < 4; qt++) {
-      const int q = q0 + qt * 16 + r;
-      if (q < n) {
-        const float *rec = rec16 + 16 * (size_t)queue[q];
-        for (int k = 0; k < 4; k++) {
-          const float4 v = *reinterpret_cast<const float4 *>(rec + 4 * k);
-          raw[qt][3 * k] = v.x;
-          raw[qt][3 * k + 1] = v.y;
-          raw[qt][3 * k + 2] = v.z;
-        }
-      } else {
-        for (int k = 0; k < 12; k++)
-          raw[qt][k] = 0.f;
-      }
+  const int step = gridDim.x * kQueryWaves * 16;
+  int q0 = (blockIdx.x * kQueryWaves + wave) * 16;
+  uint32_t pNext = q0 < n ? queue[min(q0 + r, n - 1)] : 0u;
+  for (; q0 < n; q0 += step) {
+    asm volatile("" ::: "memory"); // weights stay in LDS: in registers they leave two waves a SIMD
+    const int q = q0 + r; // this lane's query (column r of the products)
+    const bool valid = q < n;
+    const uint32_t p = pNext;
+    if (q0 + step < n)
+      pNext = queue[min(q + step, n - 1)];
+    const float *rec = rec16 + 16 * (size_t)p;
+    float raw[12], thr[3];
+    for (int k = 0; k < 4; k++) {
+      const float4 v = *reinterpret_cast<const float4 *>(rec + 4 * k);
+      raw[3 * k] = v.x;
+      raw[3 * k + 1] = v.y;
+      raw[3 * k + 2] = v.z;
+      if (k < 3)
+        thr[k] = v.w;
     }
-    f32x4 acc[4][4];
+    f32x4 acc[4][1];
     for (int nt = 0; nt < 4; nt++)
-      for (int qt = 0; qt < 4; qt++)
-        acc[nt][qt] = zero4();
+      acc[nt][0] = zero4();
     for (int kb = 0; kb < kIn / 32; kb++) {
-      bf16x8 b[4];
-      for (int qt = 0; qt < 4; qt++)
-        b[qt] = q0 + qt * 16 + r < n ? encodeGroup(raw[qt], 4 * kb + g, lo, inv) : zero8();
-      for (int nt = 0; nt < 4; nt++) {
-        const bf16x8 a = ld8(wl + kOff[0] + (nt * 16 + r) * kIn + kb * 32 + g * 8);
-        for (int qt = 0; qt < 4; qt++)
-          acc[nt][qt] = mma(a, b[qt], acc[nt][qt]);
-      }
+      const bf16x8 b = encodeGroup(raw, 4 * kb + g, lo, inv);
+      for (int nt = 0; nt < 4; nt++)
+        acc[nt][0] = mma(ld8(wl + (nt * 16 + r) * kW0S + kb * 32 + g * 8), b, acc[nt][0]);
     }
-    __syncthreads();
-    storeAct(acc, act, nullptr, r, g);
-    __syncthreads();
-    for (int l = 1; l < 4; l++) {
-      layer64(wl + kOff[l], act, acc, r, g);
-      __syncthreads();
-      storeAct(acc, act, nullptr, r, g);
-      __syncthreads();
+    f32x4 o[1];
+    forwardTail<1>(wf, acc, o);
+    if (g == 0 && valid) {
+      float *c = contrib4 + 4 * (size_t)p;
+      for (int k = 0; k < 3; k++)
+        c[k] = c[k] + thr[k] * fmaxf(o[0][k], 0.f);
     }
-    f32x4 o[4];
-    layerOut(wl + kOff[4], act, o, r, g);
-    if (g == 0)
-      for (int qt = 0; qt < 4; qt++) {
-        const int q = q0 + qt * 16 + r;
-        if (q < n) {
-          const uint32_t p = queue[q];
-          const float *rec = rec16 + 16 * (size_t)p;
-          float *c = contrib4 + 4 * (size_t)p;
-          for (int k = 0; k < 3; k++)
-            c[k] = c[k] + rec[4 * k + 3] * fmaxf(o[qt][k], 0.f);
-        }
-      }
-    __syncthreads();
   }
 }
 
@@ -576,7 +564,7 @@ hipError_t hpt_nrc_query(const HptNrc *N, const float *rec16, const uint32_t *qu
 {
   if (n <= 0)
     return hipSuccess;
-  hipLaunchKernelGGL(k_nrc_query, dim3(gridFor(n, 64 * kQueryWaves, 4096)), dim3(64 * kQueryWaves), 0, s, *N, rec16,
+  hipLaunchKernelGGL(k_nrc_query, dim3(gridFor(n, 16 * kQueryWaves, 256 * kQueryBlocks)), dim3(64 * kQueryWaves), 0, s, *N, rec16,
       queue, n, lo3[0], lo3[1], lo3[2], hi3[0], hi3[1], hi3[2], contrib4);
   return hipGetLastError();
 }

@@ -75,12 +75,9 @@ HPT_HD void fsincos(float x, float &s, float &c)
   pc = fmaf(z, pc, 4.166664568298827e-2f);
   const float tc = fmaf(z, -0.5f, 1.0f);
   const float cr = fmaf(z * z, pc, tc);
-  switch (q & 3) {
-  case 0: s = sr; c = cr; break;
-  case 1: s = cr; c = -sr; break;
-  case 2: s = -sr; c = -cr; break;
-  default: s = -cr; c = sr; break;
-  }
+  const float a = q & 1 ? cr : sr, b = q & 1 ? sr : cr;
+  s = q & 2 ? -a : a;
+  c = (q + 1) & 2 ? -b : b;
 }
 
 HPT_HD float fasin_core(float x)
