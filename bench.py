@@ -52,10 +52,9 @@ METRIC = "path samples/s at 1080p; plain vs neural-cache time-to-equal-RMSE"
 HBM_PEAK_GBS = 8000.0
 # algorithmic bytes of one traversal: 64 B per node visit and 48 B per
 # primitive test (the declared record sizes of the metric's definition),
-# plus 56 B per ray (32 B ray in, 24 B hit out).  The device's 4-wide node
-# is one 128-byte line; NODE_RECORD_BYTES gives that figure beside it.
+# plus 56 B per ray (32 B ray in, 24 B hit out).  These are the device's
+# record sizes: a 4-wide node is 64 bytes.
 NODE_BYTES, PRIM_BYTES, RAY_BYTES = 64, 48, 56
-NODE_RECORD_BYTES = 128
 # volume tracking: 32 B per voxel sample (8 corner densities of the
 # trilinear stencil), 8 B per macrocell interval (its majorant), 80 B per
 # extension ray k_volume takes (ray in, hit in, path state out) and 32 B per
@@ -555,13 +554,11 @@ def main() -> int:
         if not launches:
             continue
         per_frame_bytes = NODE_BYTES * nodes + PRIM_BYTES * prims + RAY_BYTES * rays
-        record_bytes = NODE_RECORD_BYTES * nodes + PRIM_BYTES * prims + RAY_BYTES * rays
         ms_frame = ms / args.steps
         kern[k] = {"ms_per_frame": ms_frame, "launches_per_frame": launches / args.steps,
                    "bytes_per_frame": per_frame_bytes, "rays_per_frame": rays,
                    "nodes_per_ray": nodes / max(rays, 1), "prims_per_ray": prims / max(rays, 1),
-                   "gbs": per_frame_bytes / (ms_frame * 1e-3) / 1e9,
-                   "record_gbs": record_bytes / (ms_frame * 1e-3) / 1e9}
+                   "gbs": per_frame_bytes / (ms_frame * 1e-3) / 1e9}
     if kstats.get("volume", (0, 0.0))[0]:
         launches, ms = kstats["volume"]
         samples_v, cells_v, tracks_v = vst[:3]
@@ -604,8 +601,6 @@ def main() -> int:
                               f"per ray"),
                 "bytes_per_launch": int(d["bytes_per_frame"] / lpf),
                 "launch_ms": round(launch_ms, 4)}
-    if "record_gbs" in d:
-        roofline["frac_alg_128B_node_record"] = round(d["record_gbs"] / HBM_PEAK_GBS, 4)
     valu = valu_profile(f"k_{dom}") if args.workload == "c1" else None
     if valu:
         roofline["valu"] = valu
