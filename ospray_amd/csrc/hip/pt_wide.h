@@ -191,7 +191,7 @@ __device__ __forceinline__ bool traceWide(const DScene &S, vec3f worg, vec3f wdi
               }
             }
             if (TIES != TIES_OFF) {
-              // another hit, of this round or before it, within the window
+              // another hit, in this batch of leaves or before it, within the window
               // of the closest one (the wider of the two hits' windows)
               const int near = bits(waveMask(roots != 0 && t - best.t <= kTieEps * t));
               if (near > 1 || (near == 1 && before < kInf && fabsf(before - tm) <= kTieEps * fmaxf(before, tm)))
