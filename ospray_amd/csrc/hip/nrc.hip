@@ -61,14 +61,20 @@ __device__ __forceinline__ float relu(float x)
   return __builtin_amdgcn_fmed3f(x, 0.f, inf);
 }
 
-// Layers 1..4 of the forward pass in registers.  The D operand that a layer
-// leaves in lane (r, g) holds query r's neurons 16 nt + 4 g .. + 3, so the
-// next product takes them as its K slots as they are: of K block kb, slots
-// 8 g .. 8 g + 3 are neurons 32 kb + 4 g .. + 3 and slots 8 g + 4 .. 8 g + 7
-// those 16 above, and the weights' columns are read in that order.  No
-// activation goes through LDS.
+// The D operand that a product leaves in lane (r, g) holds rows 16 nt + 4 g ..
+// + 3 of its A operand, and the next product takes from that lane the neurons
+// 32 kb + 8 g .. + 7.  The weight rows of layers 0..3 are therefore handed to
+// the matrix cores in this order: row s is neuron rowNeuron(s), so that tiles
+// 2 kb and 2 kb + 1 leave a lane its eight neurons, and no activation goes
+// through LDS.  Each sum runs over its inputs in their own order, as in the
+// training kernel.
+__device__ __forceinline__ int rowNeuron(int s) { return (s & 32) + ((s & 12) << 1) + ((s & 16) >> 2) + (s & 3); }
+__device__ __forceinline__ int neuronRow(int n) { return (n & 32) + ((n & 4) << 2) + ((n & 24) >> 1) + (n & 3); }
+
+// Layers 1..4 of the forward pass in registers.
 // acc[nt][qt]: layer 0's sums in, o[qt]: W4 (16 x 64) x h4; rows 0..2 are
-// the outputs.  wf(layer, row, kb) loads an A operand.
+// the outputs.  wf(layer, nt, kb) loads an A operand (of W4: nt 0, its own
+// rows).
 template <int QT, typename WF>
 __device__ __forceinline__ void forwardTail(const WF &wf, f32x4 (&acc)[4][QT], f32x4 (&o)[QT])
 {
@@ -87,7 +93,7 @@ __device__ __forceinline__ void forwardTail(const WF &wf, f32x4 (&acc)[4][QT], f
       for (int qt = 0; qt < QT; qt++)
         acc[nt][qt] = zero4();
       for (int kb = 0; kb < 2; kb++) {
-        const bf16x8 a = wf(l, nt * 16, kb);
+        const bf16x8 a = wf(l, nt, kb);
         for (int qt = 0; qt < QT; qt++)
           acc[nt][qt] = mma(a, h[kb][qt], acc[nt][qt]);
       }
@@ -106,10 +112,8 @@ __global__ __launch_bounds__(64) void k_nrc_infer(HptNrc N, const __bf16 *X, int
 {
   const int lane = threadIdx.x, r = lane & 15, g = lane >> 4;
   const __bf16 *W = reinterpret_cast<const __bf16 *>(N.w);
-  const auto wf = [&](int l, int row, int kb) {
-    const __bf16 *w = W + kOff[l] + (row + r) * kH + kb * 32 + 4 * g;
-    const bf16x4 a = *reinterpret_cast<const bf16x4 *>(w), b = *reinterpret_cast<const bf16x4 *>(w + 16);
-    return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
+  const auto wf = [&](int l, int nt, int kb) {
+    return ld8(W + kOff[l] + (l < 4 ? rowNeuron(nt * 16 + r) : r) * kH + kb * 32 + g * 8);
   };
   for (int tile = blockIdx.x; tile * 64 < n; tile += gridDim.x) {
     const int q0 = tile * 64;
@@ -124,7 +128,7 @@ __global__ __launch_bounds__(64) void k_nrc_infer(HptNrc N, const __bf16 *X, int
         b[qt] = q < n ? ld8(X + (size_t)q * kIn + kb * 32 + g * 8) : zero8();
       }
       for (int nt = 0; nt < 4; nt++) {
-        const bf16x8 a = ld8(W + (nt * 16 + r) * kIn + kb * 32 + g * 8);
+        const bf16x8 a = ld8(W + rowNeuron(nt * 16 + r) * kIn + kb * 32 + g * 8);
         for (int qt = 0; qt < 4; qt++)
           acc[nt][qt] = mma(a, b[qt], acc[nt][qt]);
       }
@@ -151,8 +155,9 @@ __global__ __launch_bounds__(64) void k_nrc_infer(HptNrc N, const __bf16 *X, int
 // tile's chain of layers sets its time: four waves share a tile, wave w
 // owning rows 16 w .. 16 w + 15 of every layer (queries 16 w .. of the
 // output layer), with every weight fragment it will need, forward and
-// transposed, loaded before the first layer.  Each output element's sums run
-// over the same operands in the same order as with one wave.  256 tiles:
+// transposed, loaded before the first layer.  Each output element's sums, and
+// the tile's loss, run over the same operands in the same order as with one
+// wave.  256 tiles:
 // 39.8 -> 21.8 us.
 constexpr int kSX = 168; // LDS row stride (bf16) of the query-major features
 __global__ __launch_bounds__(256) void k_nrc_train(HptNrc N, const __bf16 *X, const float *T, int n)
@@ -164,7 +169,7 @@ __global__ __launch_bounds__(256) void k_nrc_train(HptNrc N, const __bf16 *X, co
   __shared__ __attribute__((aligned(16))) __bf16 dzT[kH * kS]; // [n][q]
   __shared__ __attribute__((aligned(16))) __bf16 dyT[kOP * kS]; // [c][q]
   __shared__ __attribute__((aligned(16))) __bf16 dy[64 * kDyS]; // [q][c], c < 32
-  __shared__ float waveLoss[4];
+  __shared__ float lossTerms[3 * 64]; // [q][c]
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
   const __bf16 *W = reinterpret_cast<const __bf16 *>(N.w);
   const __bf16 *WT = reinterpret_cast<const __bf16 *>(N.wT);
@@ -238,29 +243,34 @@ __global__ __launch_bounds__(256) void k_nrc_train(HptNrc N, const __bf16 *X, co
       f32x4 o = zero4();
       for (int kb = 0; kb < 2; kb++)
         o = mma(wo[kb], ld8(act + qo * kS + kb * 32 + g * 8), o);
-      float loss = 0.f;
       bf16x4 dv;
       for (int e = 0; e < 4; e++) {
-        float d = 0.f;
+        float d = 0.f, loss = 0.f;
         if (g == 0 && e < 3 && qog < n) {
           const float y = o[e], t = t3[e];
           const float den = y * y + kLossEps;
           d = 2.f * (y - t) / den * scale;
-          loss += (y - t) * (y - t) / den * scale;
+          loss = (y - t) * (y - t) / den * scale;
         }
+        if (g == 0 && e < 3)
+          lossTerms[3 * qo + e] = loss;
         dv[e] = (__bf16)d;
         dyT[(4 * g + e) * kS + qo] = dv[e];
         dy[qo * kDyS + 16 + 4 * g + e] = (__bf16)0.f;
       }
       *reinterpret_cast<bf16x4 *>(dy + qo * kDyS + 4 * g) = dv;
-      for (int o2 = 32; o2 > 0; o2 >>= 1)
-        loss += __shfl_xor(loss, o2);
-      if (lane == 0)
-        waveLoss[wave] = loss;
     }
     __syncthreads();
-    if (threadIdx.x == 0)
-      N.tileLoss[tile] = (waveLoss[0] + waveLoss[1]) + (waveLoss[2] + waveLoss[3]);
+    if (threadIdx.x < 16) { // the tile's loss: queries r, r + 16, .. in order, then over r
+      float loss = 0.f;
+      for (int qt = 0; qt < 4; qt++)
+        for (int e = 0; e < 3; e++)
+          loss += lossTerms[3 * (qt * 16 + r) + e];
+      for (int o2 = 8; o2 > 0; o2 >>= 1)
+        loss += __shfl_xor(loss, o2);
+      if (r == 0)
+        N.tileLoss[tile] = loss;
+    }
     { // dW4 (16 x 64) = dy^T h4: this wave's 16 columns
       f32x4 a4 = zero4();
       for (int kb = 0; kb < 2; kb++)
@@ -357,49 +367,80 @@ __global__ __launch_bounds__(256) void k_nrc_init(HptNrc N, uint32_t seed)
     reinterpret_cast<__bf16 *>(N.wT)[kOffT[3] + (i / 16) * 32 + 16 + (i & 15)] = (__bf16)0.f;
 }
 
-// 64 parameters per block, the tiles' gradient rows split over kAdamGroups
-// waves (wave k sums tiles k, k + kAdamGroups, ... in order) and combined in
-// a fixed order: deterministic.  The rows (94 KB a tile) come from HBM, and
-// a thread waits for its rows in turn: with 4 waves a block (64 rows each of
-// 256 tiles) 35.2 us, 0.69 TB/s; with 16 waves 6.4 us, 3.7 TB/s.
-constexpr int kAdamGroups = 16;
-__global__ __launch_bounds__(64 * kAdamGroups) void k_nrc_adam(HptNrc N, int tiles, float lr, float bc1, float bc2)
+// 64 parameters per block.  Their sums over the tiles' gradient rows run in a
+// fixed order: of four groups, group k adds tiles k, k + 4, ... in turn, then
+// (0 + 1) + (2 + 3).  The rows (94 KB a tile) come from HBM, and with one wave
+// a group (64 rows each of 256 tiles, a few in flight) a step took 35.2 us,
+// 0.69 TB/s.  Four waves share a group: each has kAdamRows of its rows in
+// flight at once, and they add theirs to the group's sum one after another,
+// which keeps the order and costs four barriers: 7.1 us, 3.3 TB/s (sixteen
+// groups, an order of their own, 6.4).
+constexpr int kAdamGroups = 4, kAdamSegs = 4, kAdamRows = 16;
+__global__ __launch_bounds__(64 * kAdamGroups * kAdamSegs) void k_nrc_adam(HptNrc N, int tiles, float lr, float bc1, float bc2)
 {
   __shared__ float part[kAdamGroups][64];
-  const int col = threadIdx.x & 63, grp = threadIdx.x >> 6;
-  for (int p0 = blockIdx.x * 64; p0 < kP; p0 += gridDim.x * 64) {
-    const int p = p0 + col;
-    float gs = 0.f;
-    if (p < kP) {
-#pragma unroll 8
-      for (int t = grp; t < tiles; t += kAdamGroups)
-        gs += N.partial[(size_t)t * kP + p];
-    }
-    part[grp][col] = gs;
-    __syncthreads();
-    for (int h = kAdamGroups / 2; h > 0; h >>= 1) {
-      if (grp < h)
-        part[grp][col] += part[grp + h][col];
+  const int col = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int grp = wave % kAdamGroups, seg = wave / kAdamGroups;
+  if (blockIdx.x == kP / 64) { // the last block: the tiles' losses in order
+    constexpr int kLosses = 64 * kAdamGroups * kAdamSegs;
+    __shared__ float losses[kLosses];
+    float L = 0.f;
+    for (int t0 = 0; t0 < tiles; t0 += kLosses) {
+      const int t = t0 + (int)threadIdx.x;
+      losses[threadIdx.x] = t < tiles ? N.tileLoss[t] : 0.f;
+      __syncthreads();
+      if (wave == 0)
+        for (int k = 0; k < min(kLosses, tiles - t0); k += 64) {
+          const int x = __float_as_int(losses[k + col]);
+#pragma unroll
+          for (int i = 0; i < 64; i++) // (a lane past the last tile adds 0)
+            L += __int_as_float(__builtin_amdgcn_readlane(x, i));
+        }
       __syncthreads();
     }
-    if (grp == 0 && p < kP) {
-      const float g = part[0][col];
-      const float m = 0.9f * N.adamM[p] + 0.1f * g;
-      const float v = 0.99f * N.adamV[p] + 0.01f * g * g;
-      N.adamM[p] = m;
-      N.adamV[p] = v;
-      writeWeight(N, p, N.master[p] - lr * (m / bc1) / (sqrtf(v / bc2) + 1e-8f));
-    }
-    __syncthreads();
-  }
-  if (blockIdx.x == 0 && grp == 0) {
-    float L = 0.f;
-    for (int t = col; t < tiles; t += 64)
-      L += N.tileLoss[t];
-    for (int o = 32; o > 0; o >>= 1)
-      L += __shfl_xor(L, o);
-    if (col == 0)
+    if (threadIdx.x == 0)
       N.loss[0] = L;
+    return;
+  }
+  const int p = blockIdx.x * 64 + col;
+  if (seg == 0)
+    part[grp][col] = 0.f;
+  float m0 = 0.f, v0 = 0.f, w0 = 0.f; // on their way beside the rows
+  if (wave == 0) {
+    m0 = N.adamM[p];
+    v0 = N.adamV[p];
+    w0 = N.master[p];
+  }
+  for (int t0 = 0; t0 < tiles; t0 += kAdamGroups * kAdamSegs * kAdamRows) {
+    const int first = t0 + seg * kAdamGroups * kAdamRows + grp;
+    float x[kAdamRows] = {};
+    if (first < tiles) {
+#pragma unroll
+      for (int i = 0; i < kAdamRows; i++) { // loads without a branch between them
+        const int t = first + kAdamGroups * i;
+        const float v = N.partial[(size_t)min(t, tiles - 1) * kP + p];
+        x[i] = t < tiles ? v : 0.f;
+      }
+    }
+    for (int s = 0; s < kAdamSegs; s++) {
+      __syncthreads();
+      if (seg == s) {
+        float gs = part[grp][col];
+#pragma unroll
+        for (int i = 0; i < kAdamRows; i++)
+          gs += x[i];
+        part[grp][col] = gs;
+      }
+    }
+  }
+  __syncthreads();
+  if (wave == 0) {
+    const float g = (part[0][col] + part[1][col]) + (part[2][col] + part[3][col]);
+    const float m = 0.9f * m0 + 0.1f * g;
+    const float v = 0.99f * v0 + 0.01f * g * g;
+    N.adamM[p] = m;
+    N.adamV[p] = v;
+    writeWeight(N, p, w0 - lr * (m / bc1) / (sqrtf(v / bc2) + 1e-8f));
   }
 }
 
@@ -482,18 +523,17 @@ __global__ __launch_bounds__(64 * kQueryWaves, 6) void k_nrc_query(HptNrc N, con
       const bf16x8 v = src[i];
       if (i < kH * kIn / 8) {
         const int row = i / (kIn / 8);
-        *reinterpret_cast<bf16x8 *>(wl + row * kW0S + (i - row * (kIn / 8)) * 8) = v;
-      } else { // W1..W4: 208 rows of 64, columns in forwardTail's order
-        const int j = i - kH * kIn / 8, row = j >> 3, c = (j & 7) * 8;
-        __bf16 *d = wl + 64 * kW0S + row * kWS + (c & 32) + ((c & 15) >> 2) * 8 + ((c & 16) >> 2);
-        *reinterpret_cast<bf16x4 *>(d) = __builtin_shufflevector(v, v, 0, 1, 2, 3);
-        *reinterpret_cast<bf16x4 *>(d + 8) = __builtin_shufflevector(v, v, 4, 5, 6, 7);
+        *reinterpret_cast<bf16x8 *>(wl + neuronRow(row) * kW0S + (i - row * (kIn / 8)) * 8) = v;
+      } else { // W1..W4: 208 rows of 64, W4's as they are
+        const int j = i - kH * kIn / 8, row = j >> 3;
+        const int at = row < 3 * kH ? (row & ~(kH - 1)) + neuronRow(row & (kH - 1)) : row;
+        *reinterpret_cast<bf16x8 *>(wl + 64 * kW0S + at * kWS + (j & 7) * 8) = v;
       }
     }
   }
   __syncthreads();
-  const auto wf = [&](int l, int row, int kb) {
-    return ld8(wl + 64 * kW0S + ((l - 1) * kH + row + r) * kWS + kb * 32 + g * 8);
+  const auto wf = [&](int l, int nt, int kb) {
+    return ld8(wl + 64 * kW0S + ((l - 1) * kH + nt * 16 + r) * kWS + kb * 32 + g * 8);
   };
   const float lo[3] = {lx, ly, lz}, inv[3] = {1.f / (hx - lx), 1.f / (hy - ly), 1.f / (hz - lz)};
   const int step = gridDim.x * kQueryWaves * 16;
@@ -595,7 +635,7 @@ hipError_t hpt_nrc_adam(const HptNrc *N, int n, float lr, int step, hipStream_t 
   if (tiles <= 0 || tiles > N->maxTiles || step < 1)
     return hipErrorInvalidValue;
   const float bc1 = 1.f - powf(0.9f, (float)step), bc2 = 1.f - powf(0.99f, (float)step);
-  hipLaunchKernelGGL(k_nrc_adam, dim3(gridFor(kP, 64, 1024)), dim3(64 * kAdamGroups), 0, s, *N, tiles, lr, bc1, bc2);
+  hipLaunchKernelGGL(k_nrc_adam, dim3(kP / 64 + 1), dim3(64 * kAdamGroups * kAdamSegs), 0, s, *N, tiles, lr, bc1, bc2);
   return hipGetLastError();
 }
 
