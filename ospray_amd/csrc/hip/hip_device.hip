@@ -1198,7 +1198,6 @@ class HipDevice : public Device
       }
       if (residentTraceBlocks > 0)
         ensureScratch(*L);
-      L->paths.overflow = L->overflow.as<uint32_t>();
       L->paths.stats = (unsigned long long *)stats.ptr;
       lanes.push_back(std::move(L));
     }
@@ -1216,28 +1215,33 @@ class HipDevice : public Device
     for (auto &L : lanes) {
       HIP_CHECK(hipStreamSynchronize(L->stream));
       ensureScratch(*L);
-      L->paths.overflow = L->overflow.as<uint32_t>();
     }
   }
 
-  // the traversal scratch rows of a lane, cleared when (re)allocated: the
-  // occlusion pass keeps each row's recorded-hit count at 0 between rays
-  void ensureScratch(PathLane &L)
+  // Traversal scratch rows for the resident grid in force, used on stream s
+  // alone and cleared there when (re)allocated: the occlusion pass keeps each
+  // row's recorded-hit count at 0 between rays.  A kernel's threads index
+  // their rows without a check, so each buffer is looked at for itself before
+  // its kernels are enqueued: a lane's two grow at different times.
+  void ensureRows(DevBuf &rows, hipStream_t s)
   {
-    const size_t bytes = (size_t)residentTraceBlocks * hpt_trace_block_size() * hpt_overflow_depth() * 4;
-    if (L.overflow.ptr && L.overflow.bytes >= bytes)
+    const size_t words = (size_t)residentTraceBlocks * hpt_trace_block_size() * hpt_overflow_depth();
+    if (rows.ptr && rows.bytes >= 4 * words)
       return;
     if (capturing)
       throw std::runtime_error("batched views: traversal scratch would grow while capturing");
-    L.overflow.ensure(bytes);
-    HIP_CHECK(hipMemset(L.overflow.ptr, 0, bytes));
-    if (L.side) { // the side stream's rows follow the grid size too
-      L.sideOverflow.ensure(bytes);
-      HIP_CHECK(hipMemset(L.sideOverflow.ptr, 0, bytes));
-    }
+    HIP_CHECK(hipStreamSynchronize(s));
+    rows.ensure(4 * words);
+    HIP_CHECK(hpt_fill_u32(rows.as<uint32_t>(), words, 0u, s));
+  }
+  void ensureScratch(PathLane &L)
+  {
+    ensureRows(L.overflow, L.stream);
+    L.paths.overflow = L.overflow.as<uint32_t>();
   }
 
-  // the side stream of a lane, its scratch rows and events (first use)
+  // the side stream of a lane and its events (made on first use), with
+  // scratch rows for the grid in force
   hipStream_t ensureSide(PathLane &L)
   {
     if (!L.side) {
@@ -1246,10 +1250,8 @@ class HipDevice : public Device
         HIP_CHECK(hipEventCreateWithFlags(&L.evShade[k], hipEventDisableTiming));
         HIP_CHECK(hipEventCreateWithFlags(&L.evRes[k], hipEventDisableTiming));
       }
-      const size_t bytes = (size_t)residentTraceBlocks * hpt_trace_block_size() * hpt_overflow_depth() * 4;
-      L.sideOverflow.ensure(bytes);
-      HIP_CHECK(hipMemset(L.sideOverflow.ptr, 0, bytes));
     }
+    ensureRows(L.sideOverflow, L.side);
     return L.side;
   }
 
@@ -2787,7 +2789,7 @@ ManagedObject *HipDevice::renderFrame(ManagedObject *fbo, ManagedObject *ro, Man
       ensurePaths((size_t)sppPerPass * F.numPixPadded, F.maxRec, aux);
       ensureCounters(F.maxDepth + 1);
       lane->paths.aux = aux ? lane->auxBase : nullptr;
-      lane->paths.overflow = lane->overflow.as<uint32_t>();
+      ensureScratch(*lane);
     }
     if (F.nrcBounce >= 0) {
       ensureNrc(lane->pathSlots);
@@ -2976,6 +2978,7 @@ int HipDevice::traceRays(World *w, const float *rays8, int n, float *outTUV, uin
   if (!w->built)
     throw std::runtime_error("world not committed");
   gpu();
+  ensureScratch(*lanes[0]);
   DevBuf dr, dt, di;
   dr.ensure((size_t)std::max(n, 1) * 32);
   dt.ensure((size_t)std::max(n, 1) * 12);
