@@ -112,7 +112,7 @@ HPT_API hipError_t hpt_trace_rays(const HptScene *S, const float *rays8, int n, 
  * allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc).  No counterpart in the
  * reference.  The traversal scratch rows come from a fixed device array of
- * the module (64 MiB per GPU, held until the process ends), so
+ * the module (66 MiB per GPU, held until the process ends), so
  * residentBlocks must be in [1, hpt_trace_noalloc_max_blocks()]; anything
  * else returns hipErrorInvalidValue before launching.  Allocates nothing
  * (no hipMalloc, hipFree or allocating library call).  All calls on one GPU

@@ -585,6 +585,9 @@ __device__ __forceinline__ uint32_t gridAbove(double p, double s, double hi)
 }
 
 // One axis of a node: the grid over the children's bounds and their planes.
+// An unused slot has its planes the wrong way round, so that a ray enters it
+// only where the whole node is within the box test's padding; its leaf is one
+// that no ray hits, and the stack rows have room for it (kStackCapacity).
 __device__ __forceinline__ void gridAxis(const float lo[4], const float hi[4], const bool used[4], float &p, float &s,
     uint32_t &qlo, uint32_t &qhi)
 {
@@ -595,7 +598,7 @@ __device__ __forceinline__ void gridAxis(const float lo[4], const float hi[4], c
       b = fmaxf(b, hi[c]);
     }
   p = a <= b ? a : 0.f;
-  s = a <= b ? (float)(((double)b - a) / 255.0) : 0.f;
+  s = a <= b ? (float)(((double)b - a) / 255.0) : 1.f;
   if (a <= b && (double)p + 255.0 * (double)s < (double)b) // rounded down
     s = fmaxf(s * 1.0000002f, 1.17549435e-38f);
   qlo = qhi = 0;
@@ -603,6 +606,8 @@ __device__ __forceinline__ void gridAxis(const float lo[4], const float hi[4], c
     if (used[c]) {
       qlo |= gridBelow(p, s, lo[c]) << (8 * c);
       qhi |= gridAbove(p, s, hi[c]) << (8 * c);
+    } else {
+      qlo |= 255u << (8 * c);
     }
 }
 

@@ -1643,7 +1643,7 @@ __global__ __launch_bounds__(kTraceBlock) void k_trace_rays(DScene S, const floa
 
 // The traversal scratch rows of hpt_trace_rays_noalloc: a file-scope device
 // array, kThreadRow words for each thread of at most kNoAllocTraceBlocks
-// resident blocks (64 MiB).  Every GPU that runs the module holds its own
+// resident blocks (66 MiB).  Every GPU that runs the module holds its own
 // copy until the process ends; host code reaches it only through the
 // address hipGetSymbolAddress returns on that GPU, looked up once per
 // device on the first call there.

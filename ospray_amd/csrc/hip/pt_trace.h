@@ -39,11 +39,17 @@ namespace hpt {
 
 constexpr int kTraceBlock = 128;
 constexpr int kLdsDepth = 24;
-constexpr int kOverflowDepth = 108;
-// entries a tree may need: the rows but the sentinel's, rounded down so that
-// the recorded hits stay 16-byte aligned
+constexpr int kOverflowDepth = 112;
+// Entries a world may need by the builders' count: one less than its children
+// for each node on the way down, and the two of an instance's entry.  The rows
+// hold more: a ray that enters an unused slot of a node (k_relocate) pushes
+// that too, up to three entries beyond the count in the BLAS and in the TLAS
+// each, since only a node without inner children has unused slots; and one row
+// holds the sentinel.  (A multiple of four, so that the recorded hits stay
+// 16-byte aligned.)
 constexpr int kStackCapacity = 128;
-static_assert(kStackCapacity < kLdsDepth + kOverflowDepth && kOverflowDepth % 4 == 0, "stack rows");
+constexpr int kUnusedSlots = 6;
+static_assert(kStackCapacity + kUnusedSlots + 1 <= kLdsDepth + kOverflowDepth && kOverflowDepth % 4 == 0, "stack rows");
 // transparent hits an occlusion traversal records for the transparency pass
 constexpr int kTransRecHits = 4;
 // words of scratch per resident traversal thread: the stack overflow, then
@@ -430,7 +436,7 @@ __device__ void resolveNearTie(const DScene &S, vec3f worg, vec3f wdir, float t0
     const int ch[4] = {nd.child.x, nd.child.y, nd.child.z, nd.child.w};
     for (int c = 0; c < 4; c++)
       if (tc[c] != kInf) {
-        if (sp >= kLdsDepth + kOverflowDepth) // cannot happen: the world commit checks the stack need
+        if (sp >= kLdsDepth + kOverflowDepth) // cannot happen: the world commit checks the stack need (kStackCapacity)
           return false;
         push(ch[c]);
       }
@@ -678,7 +684,7 @@ __device__ __forceinline__ void traceDescend(
           top[2 * kTraceBlock] = (uint32_t)c1;
           s.sp += grow;
           s.cur = c0;
-        } else if (s.sp + grow >= (kLdsDepth + kOverflowDepth + 1) * kStackRow) { // cannot happen: the world commit checks the stack need
+        } else if (s.sp + grow >= (kLdsDepth + kOverflowDepth + 1) * kStackRow) { // cannot happen, as above
           s.cur = kTraceDone;
         } else {
           if (h3)

@@ -63,3 +63,30 @@ def test_hits_equal_the_oracle(hip_device, shape, n, scale, offset, host):
     otuv, oids, _ = orc.OracleScene(sc).intersect(rays)
     assert np.array_equal(ids, oids) and np.array_equal(tuv, otuv)
     assert (ids[:, 0] != 0xFFFFFFFF).any()
+
+
+@pytest.mark.parametrize("n", [1, 2, 3])
+def test_unused_slots_are_not_entered(hip_device, n):
+    """A node of one to three children leaves the others' slots unused: rays
+    into the node's own corners, the lowest ones among them, test no more
+    primitives than it has."""
+    rng = np.random.default_rng(7 + n)
+    v = rng.uniform(0.1, 0.9, (n, 3, 3)).astype(np.float32)
+    v[0, 0], v[0, 1], v[0, 2] = (0, 0, 0), (1, 1, 1), (0, 1, 0.5)  # the node's box: the unit cube
+    sc = scenes.Scene("corner", 8, 8, [scenes.Geometry("triangles", vertex=v.reshape(-1, 3),
+                                                       index=np.arange(3 * n, dtype=np.uint32).reshape(-1, 3))],
+                      [scenes.Model(0, 0)], [[0]], [scenes.Instance(0)], [{"type": "obj"}], [{"type": "ambient"}],
+                      {"position": (0, 0, -1), "direction": (0, 0, 1)}, {"pixelSamples": 1})
+    s = scenes.to_ospray(sc)
+    corners = np.array([[x, y, z] for x in (0, 1) for y in (0, 1) for z in (0, 1)], np.float64)
+    rays = []
+    for c in corners:
+        for _ in range(16):
+            d = rng.normal(size=3)
+            d /= np.linalg.norm(d)
+            rays.append(np.concatenate([c - 3 * d, d, [0, np.inf]]))
+    rays = np.array(rays, np.float32)
+    tuv, ids, (nodes, prims) = A.trace_rays(s.world, rays)
+    otuv, oids, _ = orc.OracleScene(sc).intersect(rays)
+    assert np.array_equal(ids, oids) and np.array_equal(tuv, otuv)
+    assert prims <= n * len(rays), prims
