@@ -584,7 +584,10 @@ __device__ __forceinline__ uint32_t gridAbove(double p, double s, double hi)
   return (uint32_t)q;
 }
 
-// One axis of a node: the grid over the children's bounds and their planes.
+// One axis of a node: the grid over the children's bounds and their planes,
+// moved outwards by 10 u of the node's size for the box test's roundings
+// (nodeNear) and by u / 2 of its largest coordinate, so that a ray along a face
+// of a box starts inside of it (u = 2^-24).
 // An unused slot has its planes the wrong way round, so that a ray enters it
 // only where the whole node is within the box test's padding; its leaf is one
 // that no ray hits, and the stack rows have room for it (kStackCapacity).
@@ -597,15 +600,18 @@ __device__ __forceinline__ void gridAxis(const float lo[4], const float hi[4], c
       a = fminf(a, lo[c]);
       b = fmaxf(b, hi[c]);
     }
-  p = a <= b ? a : 0.f;
-  s = a <= b ? (float)(((double)b - a) / 255.0) : 1.f;
-  if (a <= b && (double)p + 255.0 * (double)s < (double)b) // rounded down
-    s = fmaxf(s * 1.0000002f, 1.17549435e-38f);
+  const bool any = a <= b;
+  constexpr double u = 1.0 / 16777216.0;
+  const double pad = any ? 10.0 * u * ((double)b - a) + 0.5 * u * fmax(fabs((double)a), fabs((double)b)) : 0.0;
+  p = any ? __double2float_rd(a - pad) : 0.f;
+  s = any ? __double2float_ru(((double)b + pad - p) / 255.0) : 1.f;
+  if (s > 0.f)
+    s = fmaxf(s, 1.17549435e-38f);
   qlo = qhi = 0;
   for (int c = 0; c < 4; c++)
     if (used[c]) {
-      qlo |= gridBelow(p, s, lo[c]) << (8 * c);
-      qhi |= gridAbove(p, s, hi[c]) << (8 * c);
+      qlo |= gridBelow(p, s, lo[c] - pad) << (8 * c);
+      qhi |= gridAbove(p, s, hi[c] + pad) << (8 * c);
     } else {
       qlo |= 255u << (8 * c);
     }

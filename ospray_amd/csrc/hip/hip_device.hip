@@ -2085,16 +2085,6 @@ static std::shared_ptr<Blas> buildBlasHost(const std::vector<Geometry *> &geoms)
   return B;
 }
 
-// largest |coordinate| of a box, 0 of an empty one
-static float boxExtent(const hpt::BuildBox &b)
-{
-  float e = 0.f;
-  if (b.lo[0] <= b.hi[0])
-    for (int k = 0; k < 3; k++)
-      e = std::max(e, std::max(std::fabs(b.lo[k]), std::fabs(b.hi[k])));
-  return e;
-}
-
 void World::commit() // World.cpp:70-188 plus the Group BLAS builds (Group.cpp:93-143)
 {
   HipDevice &D = *dev;
@@ -2240,7 +2230,6 @@ void World::commit() // World.cpp:70-188 plus the Group BLAS builds (Group.cpp:9
     for (size_t k = 0; k < groups[gi]->models.size(); k++)
       di.allOpaque &= models[groupModelOffset[gi] + k].opaque;
     di.userID = I.userID;
-    di.extent = boxExtent(B.bounds);
     di.epsScale = hpt::maxf(std::fabs(x[0]), hpt::maxf(std::fabs(x[4]), std::fabs(x[8])));
     hpt::BuildBox wb;
     for (int k = 0; k < 3; k++) {
@@ -2414,7 +2403,6 @@ void World::commit() // World.cpp:70-188 plus the Group BLAS builds (Group.cpp:9
   scene.lightsCDF = dLightsCDF.as<const float>();
   scene.geoCDF = dGeoCDF.as<const float>();
   scene.tlasRoot = tlasOff;
-  scene.extent = boxExtent(T.bounds);
   scene.numInstances = (int)instances.size();
   scene.numLights = (int)dl.size();
   scene.numMaterials = (int)dmats.size();

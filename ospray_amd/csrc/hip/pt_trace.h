@@ -261,27 +261,16 @@ struct Node4
   int4 child;
 };
 
-// What the box test needs of a ray, per axis: 1 / d and -o / d shifted by
-// the padding of the near and far planes (see nodeNear).
+// What the box test needs of a ray: its origin and 1 / d per axis
 struct BoxRay
 {
-  vec3f inv, kn, kf;
+  vec3f o, inv;
 };
 
-// 10 ulp (of 2^-24) of the largest coordinate difference a box test forms
-constexpr float kBoxPad = 5.96046448e-7f;
+__device__ __forceinline__ BoxRay boxRay(vec3f o, vec3f d) { return {o, v3(boxInv(d.x), boxInv(d.y), boxInv(d.z))}; }
 
-__device__ __forceinline__ BoxRay boxRay(vec3f o, vec3f d, float extent)
-{
-  BoxRay r;
-  r.inv = v3(boxInv(d.x), boxInv(d.y), boxInv(d.z));
-  const vec3f k = v3(-o.x * r.inv.x, -o.y * r.inv.y, -o.z * r.inv.z);
-  const vec3f pad = v3(kBoxPad * (fabsf(o.x) + extent) * fabsf(r.inv.x), kBoxPad * (fabsf(o.y) + extent) * fabsf(r.inv.y),
-      kBoxPad * (fabsf(o.z) + extent) * fabsf(r.inv.z));
-  r.kn = k - pad;
-  r.kf = k + pad;
-  return r;
-}
+// 12 u, u = 2^-24, of the distance to a node's first plane (see nodeNear)
+constexpr float kBoxPad = 7.15255737e-7f;
 
 __device__ __forceinline__ Node4 loadNode(const DNode4 *nodes, int idx)
 {
@@ -314,12 +303,13 @@ struct NodeAxis
   uint32_t first, last;
 };
 
-__device__ __forceinline__ NodeAxis nodeAxis(float p, float s, uint32_t lo, uint32_t hi, float inv, float kn, float kf)
+__device__ __forceinline__ NodeAxis nodeAxis(float p, float s, uint32_t lo, uint32_t hi, float o, float inv)
 {
   NodeAxis x;
+  const float m = (p - o) * inv;
   x.a = s * inv;
-  x.near = fmaf(p, inv, kn);
-  x.far = fmaf(p, inv, kf);
+  x.near = fmaf(-kBoxPad, fabsf(m), m);
+  x.far = fmaf(kBoxPad, fabsf(m), m);
   const bool back = inv < 0.f;
   x.first = back ? hi : lo;
   x.last = back ? lo : hi;
@@ -329,20 +319,25 @@ __device__ __forceinline__ NodeAxis nodeAxis(float p, float s, uint32_t lo, uint
 // Entry distances t[c] of the four children's boxes over [t0, tb], +inf for
 // a box the ray misses.
 //
-// Conservative: with u = 2^-24, a plane's distance (p + q s - o) / d comes
-// out off by at most 5 u (|o| + extent) / |d| from the roundings of 1 / d (1
-// ulp), -o / d, p / d - o / d, s / d, the product and the sum, extent
-// bounding the tree's coordinates; the near planes are moved down and the
-// far ones up by twice that, which leaves 5 ulp of slack for a primitive's
-// own hit distance, so the closest hit does not depend on the tree.  A NaN
-// (overflow) leaves the axis out of the test.  The near plane of an axis is
-// picked once for the four children, a word at a time: a minimum or maximum
-// costs 4.3 cycles of a SIMD, a select or FMA 2.6 (measured).
+// Conservative: with u = 2^-24, M = (p - o) / d and Q = q s / d, the distance
+// M + Q of plane q comes out off by at most 6 u |M| + 4 u |Q|: p - o, 1 / d (1
+// ulp, 2 u), their product, the padding's and the last sum on M, 1 / d, s / d
+// and the last sum on Q.  The near planes are moved down and the far ones up
+// by 12 u |M| here and by 10 u of the node's size over |d| in the grid itself
+// (k_relocate), which leaves 6 u of both for a primitive's own hit distance,
+// so the closest hit does not depend on the tree.  Neither padding looks
+// further than the node and the ray's origin: culling next to an object does
+// not depend on what else is in the tree, nor on where the origin of the
+// coordinates lies.  (Padded by the tree's largest coordinate, one instance at
+// 1e6 widened every box of the world by 0.6.)  A NaN (overflow) leaves the
+// axis out of the test.  The near plane of an axis is picked once for the four
+// children, a word at a time: a minimum or maximum costs 4.3 cycles of a SIMD,
+// a select or FMA 2.6 (measured).
 __device__ __forceinline__ void nodeNear(const Node4 &n, const BoxRay &r, float t0, float tb, float t[4])
 {
-  const NodeAxis x = nodeAxis(n.a.x, n.a.w, __float_as_uint(n.b.z), __float_as_uint(n.b.w), r.inv.x, r.kn.x, r.kf.x);
-  const NodeAxis y = nodeAxis(n.a.y, n.b.x, n.c.x, n.c.y, r.inv.y, r.kn.y, r.kf.y);
-  const NodeAxis z = nodeAxis(n.a.z, n.b.y, n.c.z, n.c.w, r.inv.z, r.kn.z, r.kf.z);
+  const NodeAxis x = nodeAxis(n.a.x, n.a.w, __float_as_uint(n.b.z), __float_as_uint(n.b.w), r.o.x, r.inv.x);
+  const NodeAxis y = nodeAxis(n.a.y, n.b.x, n.c.x, n.c.y, r.o.y, r.inv.y);
+  const NodeAxis z = nodeAxis(n.a.z, n.b.y, n.c.z, n.c.w, r.o.z, r.inv.z);
 #pragma unroll
   for (int c = 0; c < 4; c++) {
     auto q = [c](uint32_t w) { return (float)((w >> (8 * c)) & 0xffu); };
@@ -408,7 +403,7 @@ __device__ void resolveNearTie(const DScene &S, vec3f worg, vec3f wdir, float t0
   const float tF = best.t;
   const float tHi = fminf(tF + kTieEps * tF, tfar);
   const float tLo = fmaxf(t0, kTieBoxLow * tF);
-  const BoxRay wbox = boxRay(worg, wdir, S.extent);
+  const BoxRay wbox = boxRay(worg, wdir);
   Hit w = best;
   double wD = 0.0;
   bool have = false;
@@ -455,7 +450,7 @@ __device__ void resolveNearTie(const DScene &S, vec3f worg, vec3f wdir, float t0
     const linear3f rl = {{I.rcp[0], I.rcp[1], I.rcp[2]}, {I.rcp[3], I.rcp[4], I.rcp[5]}, {I.rcp[6], I.rcp[7], I.rcp[8]}};
     const vec3f o = mul(rl, worg) + v3(I.rcp[9], I.rcp[10], I.rcp[11]);
     const vec3f d = mul(rl, wdir);
-    const BoxRay box = boxRay(o, d, I.extent);
+    const BoxRay box = boxRay(o, d);
     const TriPre pc = triPrecompute(d);
     double od[3], dd[3];
     fp64ObjectRay(I.rcp, worg, wdir, od, dd);
@@ -552,7 +547,6 @@ struct TraceHit
 struct TraceState
 {
   vec3f worg, wdir; // the world ray
-  vec3f o;          // origin of the object ray (inside an instance)
   BoxRay box;       // of the current (world or object) ray
   TriPre pc;
   float t0, tfar;
@@ -575,8 +569,7 @@ __device__ __forceinline__ void traceBegin(
   best.inst = best.prim = kInvalidID;
   s.worg = worg;
   s.wdir = wdir;
-  s.o = worg;
-  s.box = boxRay(worg, wdir, S.extent);
+  s.box = boxRay(worg, wdir);
   s.pc = {0, 0.f, 0.f, 0.f};
   s.t0 = t0;
   s.tfar = tfar;
@@ -795,7 +788,7 @@ __device__ __forceinline__ bool tracePrim(
   float t, u = 0.f, v = 0.f, tX = 0.f;
   int roots = 1;
   if (mk >> 28 != PRIM_SPHERE) {
-    if (!intersectTriangle(s.o, MODE == MODE_OCCLUSION ? 0.f : s.t0, s.pc, w.A, w.B, w.C, s.tb, t, u, v))
+    if (!intersectTriangle(s.box.o, MODE == MODE_OCCLUSION ? 0.f : s.t0, s.pc, w.A, w.B, w.C, s.tb, t, u, v))
       return false;
   } else {
     // the object direction again, rather than three registers held for it
@@ -865,9 +858,8 @@ __device__ __forceinline__ bool traceLeaf(TraceState &s, const DScene &S, TraceH
       // world leaf: one instance; continue in its BLAS with the object ray
       s.inst = (int)first;
       const linear3f rl = {{r0.x, r0.y, r0.z}, {r0.w, r1.x, r1.y}, {r1.z, r1.w, r2.x}};
-      s.o = mul(rl, s.worg) + v3(r2.y, r2.z, r2.w);
       const vec3f d = mul(rl, s.wdir);
-      s.box = boxRay(s.o, d, r3.w);
+      s.box = boxRay(mul(rl, s.worg) + v3(r2.y, r2.z, r2.w), d);
       s.pc = triPrecompute(d);
       if (MODE == MODE_OCCLUSION)
         s.modelOffset = __float_as_int(r3.z) ? -1 : __float_as_int(r3.y);
@@ -897,7 +889,7 @@ __device__ __forceinline__ bool traceLeaf(TraceState &s, const DScene &S, TraceH
     }
   }
   if (s.cur == kMarker) {
-    s.box = boxRay(s.worg, s.wdir, S.extent);
+    s.box = boxRay(s.worg, s.wdir);
     s.inst = -1;
     s.cur = tracePop(s, lds, ovf);
   }

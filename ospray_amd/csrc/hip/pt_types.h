@@ -79,7 +79,7 @@ struct DInstance
   int32_t blasRoot; // node index of the group's BLAS root
   int32_t modelOffset; // first DModel of the group
   int32_t allOpaque; // every model of the group is opaque
-  float extent; // largest |coordinate| of the BLAS's bounds (0: no geometry)
+  int32_t pad0; // (the 64 B end here)
   float xfm[12]; // forward transform
   uint32_t userID; // kInvalidID if unset
   float epsScale; // max(|xfm.vx.x|, |xfm.vy.y|, |xfm.vz.z|)
@@ -210,7 +210,6 @@ struct DScene
   const DVolume *volumes;
   const DVolInst *volInsts;
   int32_t tlasRoot;
-  float extent; // largest |coordinate| of the TLAS's bounds (0: no geometry)
   int32_t numInstances;
   int32_t numLights;
   int32_t numGeoLights;

@@ -25,7 +25,7 @@
 
 namespace hpt {
 
-constexpr int kWideSlots = 24, kWideSlotWords = 18;
+constexpr int kWideSlots = 24, kWideSlotWords = 13; // (odd: slots on distinct banks)
 constexpr int kWideStack = 320; // entries
 constexpr int kWideList = 96; // entries of the leaf and of the instance list
 constexpr int kWideBatch = 32; // listed leaves that are worth a test, instances that end the world phase
@@ -50,16 +50,15 @@ __device__ __forceinline__ float wideT(uint32_t ts) { return __uint_as_float(ts 
 
 struct WideLds
 {
-  float slots[kWideSlots * kWideSlotWords]; // inv, kn, kf, o, Sx, Sy, Sz, kz, instance, first model
+  float slots[kWideSlots * kWideSlotWords]; // o, 1 / d, Sx, Sy, Sz, kz, instance, first model
   WideEntry stack[kWideStack];
   WideEntry leaves[kWideList], insts[kWideList];
 };
 
 __device__ __forceinline__ void wideStoreBox(float *w, const BoxRay &b)
 {
-  w[0] = b.inv.x, w[1] = b.inv.y, w[2] = b.inv.z;
-  w[3] = b.kn.x, w[4] = b.kn.y, w[5] = b.kn.z;
-  w[6] = b.kf.x, w[7] = b.kf.y, w[8] = b.kf.z;
+  w[0] = b.o.x, w[1] = b.o.y, w[2] = b.o.z;
+  w[3] = b.inv.x, w[4] = b.inv.y, w[5] = b.inv.z;
 }
 
 // x of the lane `mask` away within the group of four (1, 2 or 3)
@@ -94,7 +93,7 @@ __device__ __forceinline__ bool traceWide(const DScene &S, vec3f worg, vec3f wdi
   float tb = tfar;
   uint32_t recorded = 0; // hits of non-opaque primitives
   if (lane == 0) {
-    wideStoreBox(W.slots, boxRay(worg, wdir, S.extent));
+    wideStoreBox(W.slots, boxRay(worg, wdir));
     W.stack[0] = {(uint32_t)S.tlasRoot, 0u};
   }
   // wave-uniform: entries of the stack, of the world's part of it, of the lists
@@ -122,7 +121,7 @@ __device__ __forceinline__ bool traceWide(const DScene &S, vec3f worg, vec3f wdi
         float t = kInf, u = 0.f, v = 0.f, tX = 0.f;
         int roots = 0;
         uint32_t mk = 0;
-        const uint32_t inst = __float_as_uint(w[16]);
+        const uint32_t inst = __float_as_uint(w[10]);
         if (k < end) {
           const float4 *P = reinterpret_cast<const float4 *>(S.prims + k);
           const PrimWords q = primWords(P[0], P[1], P[2]);
@@ -130,9 +129,9 @@ __device__ __forceinline__ bool traceWide(const DScene &S, vec3f worg, vec3f wdi
           if (STATS)
             st.prims++;
           if (mk >> 28 != PRIM_SPHERE) {
-            const TriPre pc = {__float_as_int(w[15]), w[12], w[13], w[14]};
+            const TriPre pc = {__float_as_int(w[9]), w[6], w[7], w[8]};
             float tt;
-            if (intersectTriangle(v3(w[9], w[10], w[11]), t0, pc, q.A, q.B, q.C, tb, tt, u, v)) {
+            if (intersectTriangle(v3(w[0], w[1], w[2]), t0, pc, q.A, q.B, q.C, tb, tt, u, v)) {
               roots = 1;
               t = tt;
             }
@@ -148,7 +147,7 @@ __device__ __forceinline__ bool traceWide(const DScene &S, vec3f worg, vec3f wdi
         const unsigned long long hits = waveMask(roots != 0);
         if (hits != 0ull) {
           if (MODE == MODE_OCCLUSION) {
-            const int offset = __float_as_int(w[17]);
+            const int offset = __float_as_int(w[11]);
             const bool opaque = roots != 0 && (offset < 0 || S.models[offset + (int)(mk & 0x0fffffffu)].opaque);
             if (waveMask(opaque) != 0ull)
               return true; // sawTransparent of no matter, and no count written
@@ -225,9 +224,9 @@ __device__ __forceinline__ bool traceWide(const DScene &S, vec3f worg, vec3f wdi
           const float *w = W.slots + slot * kWideSlotWords;
           if (STATS && c == 0)
             st.nodes++;
-          const NodeAxis x = nodeAxis(a.x, a.w, __float_as_uint(b.z), __float_as_uint(b.w), w[0], w[3], w[6]);
-          const NodeAxis y = nodeAxis(a.y, b.x, q.x, q.y, w[1], w[4], w[7]);
-          const NodeAxis z = nodeAxis(a.z, b.y, q.z, q.w, w[2], w[5], w[8]);
+          const NodeAxis x = nodeAxis(a.x, a.w, __float_as_uint(b.z), __float_as_uint(b.w), w[0], w[3]);
+          const NodeAxis y = nodeAxis(a.y, b.x, q.x, q.y, w[1], w[4]);
+          const NodeAxis z = nodeAxis(a.z, b.y, q.z, q.w, w[2], w[5]);
           const int sh = 8 * c;
           auto plane = [sh](uint32_t words) { return (float)((words >> sh) & 0xffu); };
           const float n = fmaxf(fmaxf(fmaf(plane(x.first), x.a, x.near), fmaf(plane(y.first), y.a, y.near)),
@@ -292,12 +291,11 @@ __device__ __forceinline__ bool traceWide(const DScene &S, vec3f worg, vec3f wdi
         const vec3f d = mul(rl, wdir);
         const TriPre pc = triPrecompute(d);
         float *w = W.slots + slot * kWideSlotWords;
-        wideStoreBox(w, boxRay(o, d, r3.w));
-        w[9] = o.x, w[10] = o.y, w[11] = o.z;
-        w[12] = pc.Sx, w[13] = pc.Sy, w[14] = pc.Sz;
-        w[15] = __int_as_float(pc.kz);
-        w[16] = __uint_as_float(inst);
-        w[17] = __int_as_float(__float_as_int(r3.z) ? -1 : __float_as_int(r3.y));
+        wideStoreBox(w, boxRay(o, d));
+        w[6] = pc.Sx, w[7] = pc.Sy, w[8] = pc.Sz;
+        w[9] = __int_as_float(pc.kz);
+        w[10] = __uint_as_float(inst);
+        w[11] = __int_as_float(__float_as_int(r3.z) ? -1 : __float_as_int(r3.y));
         const WideEntry e = {(uint32_t)root, (ts & ~31u) | slot};
         if (enter) // the first listed on top
           W.stack[sp + bits(em) - 1 - bits(em & below)] = e;

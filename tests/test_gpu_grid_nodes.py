@@ -90,3 +90,50 @@ def test_unused_slots_are_not_entered(hip_device, n):
     otuv, oids, _ = orc.OracleScene(sc).intersect(rays)
     assert np.array_equal(ids, oids) and np.array_equal(tuv, otuv)
     assert prims <= n * len(rays), prims
+
+
+def _visits(v, rays, xfms):
+    n = len(v) // 3
+    sc = scenes.Scene("scales", 8, 8, [scenes.Geometry("triangles", vertex=v,
+                                                       index=np.arange(3 * n, dtype=np.uint32).reshape(-1, 3))],
+                      [scenes.Model(0, 0)], [[0]], [scenes.Instance(0, xfm=x) for x in xfms], [{"type": "obj"}],
+                      [{"type": "ambient"}], {"position": (0, 0, -1), "direction": (0, 0, 1)}, {"pixelSamples": 1})
+    s = scenes.to_ospray(sc)
+    tuv, ids, visits = A.trace_rays(s.world, rays)
+    otuv, oids, _ = orc.OracleScene(sc).intersect(rays)
+    assert np.array_equal(ids, oids) and np.array_equal(tuv, otuv)
+    assert (ids[:, 0] != 0xFFFFFFFF).any()
+    return np.array(visits, np.float64)
+
+
+ID = (1, 0, 0, 0, 1, 0, 0, 0, 1)
+
+
+def test_culling_is_local(hip_device):
+    """What a ray visits next to small detail depends neither on objects far
+    away, in the world or in the same geometry, nor on the distance to the
+    origin of the coordinates: the padding of a box is made of the box's own
+    size and its distance to the ray's origin."""
+    rng = np.random.default_rng(5)
+    # 2,000 triangles of 0.1 in a cube of 8, on a grid of 1/64, so that they
+    # can be moved by 2^17 without a rounding
+    c = rng.uniform(-4, 4, (2000, 1, 3))
+    v = (np.round(64 * (c + 0.1 * rng.uniform(-1, 1, (2000, 3, 3)))) / 64).reshape(-1, 3).astype(np.float32)
+    # (rays along an axis through the grid's points would run in the faces of
+    # the oracle's boxes, which miss what lies in the face)
+    rays = _rays(v, rng)[1000:]
+    rays[:, :3] = np.round(64 * rays[:, :3]) / 64
+    base = _visits(v, rays, [ID + (0, 0, 0)])
+    # an instance far away: the same rays miss it at the root
+    far = _visits(v, rays, [ID + (0, 0, 0), ID + (1e6, 0, 0)])
+    assert np.all(far <= 1.02 * base + len(rays) * np.array([0.1, 0.1])), (far, base)
+    # one triangle far away: a node or two more above the others, and those
+    # the root's coarse grid lets a ray into
+    w = np.concatenate([v, v[:3] + np.float32([1e6, 0, 0])])
+    one = _visits(w, rays, [ID + (0, 0, 0)])
+    assert np.all(one <= 1.1 * base + len(rays) * np.array([3, 0.2])), (one, base)
+    # everything moved away from the origin
+    moved = rays.copy()
+    moved[:, :3] += np.float32(2 ** 17)
+    away = _visits(v + np.float32(2 ** 17), moved, [ID + (0, 0, 0)])
+    assert np.all(away <= 1.1 * base + len(rays) * 0.1), (away, base)
