@@ -71,11 +71,15 @@ HPT_API size_t hpt_bvh_workspace_bytes(uint64_t numItems);
  * outNodes, leaf `first` indices local to outPrims. */
 HPT_API hipError_t hpt_bvh_build(const HptBvhGeometry *geoms, int numGeoms, int radius, void *workspace,
     size_t workspaceBytes, void *outNodes, void *outPrims, uint64_t *hostWords, HptBvhResult *result, hipStream_t s);
+/* dst[i] = src[i] for n nodes as hpt_bvh_build writes them, inner child
+ * references + nodeOffset, leaf first indices + primOffset. */
+HPT_API hipError_t hpt_bvh_relocate(void *dst, const void *src, size_t n, int32_t nodeOffset, uint32_t primOffset,
+    hipStream_t s);
 /* Places a BVH in the world's arrays: dst[i] (hpt::DNode4) = src[i]
  * (hpt::BNode4) for n nodes, the boxes rounded outwards to the node's 8-bit
  * grid, inner child references + nodeOffset, leaf first indices +
  * primOffset, unused slots = unusedRef. */
-HPT_API hipError_t hpt_bvh_relocate(void *dst, const void *src, size_t n, int32_t nodeOffset, uint32_t primOffset,
+HPT_API hipError_t hpt_bvh_place(void *dst, const void *src, size_t n, int32_t nodeOffset, uint32_t primOffset,
     int32_t unusedRef, hipStream_t s);
 
 #ifdef __cplusplus

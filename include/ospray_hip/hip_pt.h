@@ -28,13 +28,39 @@ typedef struct HptPaths HptPaths; /* wavefront path state, queues and counters *
 #define HPT_API __attribute__((visibility("default")))
 #endif
 
-/* The start of a pass of `bounces` bounces: clears the pass's and its
- * bounces' counters (counterWords(bounces) words from P->pass on; bounce b's
- * kernels get P->counters = P->pass + kPassWords + b * kBounceWords and
- * P->next = the block after it) and polls the frame's cancellation, whose
- * latch firstPass != 0 clears before.  Stages of bounce b may run on a
- * second stream beside the extension of bounce b+1: they share no counter. */
+/* Counters of the queues, in one of two ways.
+ *
+ * A block for each bounce, cleared at once: P->pass points to
+ * hpt_counter_bytes(bounces) bytes of device memory.  hpt_begin_pass clears
+ * them for a pass of `bounces` bounces and polls the frame's cancellation,
+ * whose latch firstPass != 0 clears before.  hpt_at_bounce (host only) points
+ * P at the counters of bounce b (from 0) for the calls that follow.  Stages of
+ * bounce b may run on a second stream beside the extension of bounce b+1:
+ * they share no counter. */
+HPT_API size_t hpt_counter_bytes(int bounces);
 HPT_API hipError_t hpt_begin_pass(const HptPaths *P, int bounces, int firstPass, hipStream_t s);
+HPT_API void hpt_at_bounce(HptPaths *P, int bounce);
+/* The same counters for every bounce: P->pass is null and P->counters points
+ * to kNumCounters words; the calls below clear them between the bounces, and
+ * fail with hipErrorInvalidValue where P->pass is set.
+ * keepIndex -1: sets every counter to 0.  keepIndex 0 or 1: sets the
+ * per-bounce queue counters to 0 except the two words of extension queue
+ * `keepIndex` (its entry count and the NEE samples appended with it; the
+ * radiance-cache counters of the pass are kept).  A cancelled frame (the
+ * host wrote the frame's generation into the paths' cancellation word)
+ * also empties the kept queue and latches the cancellation. */
+HPT_API hipError_t hpt_reset_counters(const HptPaths *P, int keepIndex, hipStream_t s);
+/* The parts of the per-bounce reset, for a frame whose shadow-ray stages
+ * (hpt_nee .. hpt_resolve) of bounce b run on a second stream beside the
+ * extension of bounce b+1: before the extension, its work fetch and the
+ * near-tie queue (with the cancellation check); after bounce b's resolve
+ * (which still reads the queue it shaded), the two words of the queue the
+ * shading of bounce b+1 appends to (extension queue keepIndex ^ 1); on the
+ * second stream before bounce b+1's NEE, the shadow records, the
+ * transparency queue and their work fetch. */
+HPT_API hipError_t hpt_reset_extension_counters(const HptPaths *P, int keepIndex, hipStream_t s);
+HPT_API hipError_t hpt_reset_append_counters(const HptPaths *P, int keepIndex, hipStream_t s);
+HPT_API hipError_t hpt_reset_shadow_counters(const HptPaths *P, hipStream_t s);
 HPT_API hipError_t hpt_fill_u32(uint32_t *ptr, size_t n, uint32_t value, hipStream_t s);
 /* dst <- src, bytes a multiple of 16: a plain streaming copy that calibrates
  * bandwidth figures and HBM counters (no reference counterpart). */
@@ -91,10 +117,13 @@ HPT_API hipError_t hpt_nrc_targets(const HptPaths *P, int n, float *target3, hip
  * visible sample's transmittance estimates (NextEventEstimation.ispc:126-149). */
 HPT_API hipError_t hpt_resolve(
     const HptScene *S, const HptFrame *F, const HptPaths *P, int queue, int blocks, hipStream_t s);
-/* ScreenSample_accumulate over the pass (PathTracer.ispc:170-197); on the
- * frame's last pass also LocalFB_accumulateSample (fb/LocalFB.ispc:14-78)
- * and ColorConversion_kernel (fb/frame_ops/ColorConversion.ispc:11-36). */
+/* ScreenSample_accumulate over the pass (PathTracer.ispc:170-197). */
 HPT_API hipError_t hpt_finish_pass(const HptFrame *F, const HptPaths *P, hipStream_t s);
+/* LocalFB_accumulateSample (fb/LocalFB.ispc:14-78). */
+HPT_API hipError_t hpt_fb_accumulate(const HptFrame *F, hipStream_t s);
+/* A frame's last pass in one kernel: hpt_finish_pass, hpt_fb_accumulate and,
+ * where F->fbConverted is set, hpt_color_convert to F->fbFormat. */
+HPT_API hipError_t hpt_finish_frame(const HptFrame *F, const HptPaths *P, hipStream_t s);
 /* Variance_kernel (fb/frame_ops/Variance.ispc:11-59). */
 HPT_API hipError_t hpt_variance(const HptFrame *F, hipStream_t s);
 /* getAvgError (fb/frame_ops/Variance.cpp:32-46), FP64 sum, one float out.
@@ -102,6 +131,9 @@ HPT_API hipError_t hpt_variance(const HptFrame *F, hipStream_t s);
  * batch frame; the reduction then runs only when it is odd. */
 HPT_API hipError_t hpt_variance_reduce(const float *taskVariance, int n, float threshold, float *out,
     const uint32_t *frameState, hipStream_t s);
+/* ColorConversion_kernel (fb/frame_ops/ColorConversion.ispc:11-36);
+ * format is an OSPFrameBufferFormat. */
+HPT_API hipError_t hpt_color_convert(const float *color, int npix, int format, void *out, hipStream_t s);
 /* Closest hits of an explicit ray list: rays8 = org.xyz, dir.xyz, t0, t1;
  * outTUV = t,u,v; outIDs = instance, model, primitive (0xffffffff on miss);
  * stats (optional) += node visits, primitive tests. */

@@ -617,7 +617,29 @@ __device__ __forceinline__ void gridAxis(const float lo[4], const float hi[4], c
     }
 }
 
-__global__ __launch_bounds__(kBlock) void k_relocate(DNode4 *dst, const BNode4 *src, size_t n, int32_t nodeOff,
+// a used slot's child reference, moved
+__device__ __forceinline__ int32_t movedChild(int32_t ch, int32_t nodeOff, uint32_t primOff)
+{
+  if (ch >= 0)
+    return ch + nodeOff;
+  const uint32_t enc = ~(uint32_t)ch;
+  return (int32_t) ~((((enc >> 3) + primOff) << 3) | (enc & 7u));
+}
+
+__global__ __launch_bounds__(kBlock) void k_relocate(BNode4 *dst, const BNode4 *src, size_t n, int32_t nodeOff,
+    uint32_t primOff)
+{
+  const size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x;
+  if (i >= n)
+    return;
+  BNode4 N = src[i];
+  for (int c = 0; c < 4; c++)
+    if (N.lox[c] != kInfF)
+      N.child[c] = movedChild(N.child[c], nodeOff, primOff);
+  dst[i] = N;
+}
+
+__global__ __launch_bounds__(kBlock) void k_place(DNode4 *dst, const BNode4 *src, size_t n, int32_t nodeOff,
     uint32_t primOff, int32_t unusedRef)
 {
   const size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x;
@@ -628,15 +650,7 @@ __global__ __launch_bounds__(kBlock) void k_relocate(DNode4 *dst, const BNode4 *
   bool used[4];
   for (int c = 0; c < 4; c++) {
     used[c] = B.lox[c] != kInfF;
-    const int32_t ch = B.child[c];
-    if (!used[c]) {
-      N.child[c] = unusedRef;
-    } else if (ch >= 0) {
-      N.child[c] = ch + nodeOff;
-    } else {
-      const uint32_t enc = ~(uint32_t)ch;
-      N.child[c] = (int32_t) ~((((enc >> 3) + primOff) << 3) | (enc & 7u));
-    }
+    N.child[c] = used[c] ? movedChild(B.child[c], nodeOff, primOff) : unusedRef;
   }
   gridAxis(B.lox, B.hix, used, N.p[0], N.s[0], N.lox, N.hix);
   gridAxis(B.loy, B.hiy, used, N.p[1], N.s[1], N.loy, N.hiy);
@@ -838,11 +852,21 @@ HPT_API hipError_t hpt_bvh_build(const HptBvhGeometry *geoms, int numGeoms, int 
 }
 
 HPT_API hipError_t hpt_bvh_relocate(void *dst, const void *src, size_t n, int32_t nodeOffset, uint32_t primOffset,
+    hipStream_t s)
+{
+  if (n == 0)
+    return hipSuccess;
+  k_relocate<<<(unsigned)((n + kBlock - 1) / kBlock), kBlock, 0, s>>>((BNode4 *)dst, (const BNode4 *)src, n,
+      nodeOffset, primOffset);
+  return hipGetLastError();
+}
+
+HPT_API hipError_t hpt_bvh_place(void *dst, const void *src, size_t n, int32_t nodeOffset, uint32_t primOffset,
     int32_t unusedRef, hipStream_t s)
 {
   if (n == 0)
     return hipSuccess;
-  k_relocate<<<(unsigned)((n + kBlock - 1) / kBlock), kBlock, 0, s>>>((DNode4 *)dst, (const BNode4 *)src, n,
+  k_place<<<(unsigned)((n + kBlock - 1) / kBlock), kBlock, 0, s>>>((DNode4 *)dst, (const BNode4 *)src, n,
       nodeOffset, primOffset, unusedRef);
   return hipGetLastError();
 }

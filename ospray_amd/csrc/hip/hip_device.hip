@@ -2304,7 +2304,7 @@ void World::commit() // World.cpp:70-188 plus the Group BLAS builds (Group.cpp:9
       std::vector<hpt::BNode4>().swap(B.nodes);
       std::vector<hpt::DPrim>().swap(B.prims);
     }
-    HIP_CHECK(hpt_bvh_relocate(gNodes + blasNodeOff[k], B.dNodes.ptr, B.numNodes, blasNodeOff[k],
+    HIP_CHECK(hpt_bvh_place(gNodes + blasNodeOff[k], B.dNodes.ptr, B.numNodes, blasNodeOff[k],
         (uint32_t)blasPrimOff[k], kNoPrim, D.stream));
     if (B.numPrims > 0)
       HIP_CHECK(hipMemcpyAsync(gPrims + blasPrimOff[k], B.dPrims.ptr, sizeof(hpt::DPrim) * B.numPrims,
@@ -2312,7 +2312,7 @@ void World::commit() // World.cpp:70-188 plus the Group BLAS builds (Group.cpp:9
   }
   DevBuf tlas;
   tlas.upload(T.nodes);
-  HIP_CHECK(hpt_bvh_relocate(gNodes + tlasOff, tlas.ptr, T.nodes.size(), tlasOff, 0, noInstance, D.stream));
+  HIP_CHECK(hpt_bvh_place(gNodes + tlasOff, tlas.ptr, T.nodes.size(), tlasOff, 0, noInstance, D.stream));
   HIP_CHECK(hipStreamSynchronize(D.stream));
 
   // lights (PathTracerData.cpp:32-82): [geometry lights, world lights],
@@ -2514,7 +2514,7 @@ void HipDevice::ensurePaths(size_t slots, int maxRec, bool aux)
 // the lane's counters for passes of `bounces` bounces
 void HipDevice::ensureCounters(int bounces)
 {
-  const size_t bytes = 4 * hpt::counterWords(bounces);
+  const size_t bytes = hpt_counter_bytes(bounces);
   if (lane->counters.bytes >= bytes)
     return;
   if (capturing)
@@ -2771,11 +2771,12 @@ ManagedObject *HipDevice::renderFrame(ManagedObject *fbo, ManagedObject *ro, Man
       sppPerPass = std::min(sppPerPass, (F.spp + nl - 1) / nl);
       nl = std::min(nl, (F.spp + sppPerPass - 1) / sppPerPass);
     }
+    const int bounces = F.maxDepth + 1;
     PathLane *const frameLane = lane;
     for (int k = nl - 1; k >= 0; k--) {
       lane = k == 0 ? frameLane : &ensureLane(k);
       ensurePaths((size_t)sppPerPass * F.numPixPadded, F.maxRec, aux);
-      ensureCounters(F.maxDepth + 1);
+      ensureCounters(bounces);
       lane->paths.aux = aux ? lane->auxBase : nullptr;
       ensureScratch(*lane);
     }
@@ -2816,12 +2817,7 @@ ManagedObject *HipDevice::renderFrame(ManagedObject *fbo, ManagedObject *ro, Man
       hpt::DPaths &paths = lane->paths;
       const HptPaths *P = reinterpret_cast<const HptPaths *>(&paths);
       paths.pass = lane->counters.as<int32_t>();
-      // the counters of bounce b
-      auto atBounce = [&](hpt::DPaths &p, int b) {
-        p.counters = p.pass + hpt::kPassWords + (size_t)b * hpt::kBounceWords;
-        p.next = p.counters + hpt::kBounceWords;
-      };
-      atBounce(paths, 0);
+      hpt::atBounce(paths, 0);
       F.passS0 = s0;
       F.passCount = std::min(sppPerPass, F.spp - s0);
       if (F.nrcBounce >= 0) { // every stride-th slot of the pass trains the cache
@@ -2838,7 +2834,7 @@ ManagedObject *HipDevice::renderFrame(ManagedObject *fbo, ManagedObject *ro, Man
       Fno.nrcBounce = -1;
       const HptFrame *Fp = reinterpret_cast<const HptFrame *>(&F);
       const HptFrame *FpNo = reinterpret_cast<const HptFrame *>(&Fno);
-      launch("reset", [&]() { return hpt_begin_pass(P, F.maxDepth + 1, nl == 1 && pass == 0 ? 1 : 0, stream); });
+      launch("reset", [&]() { return hpt_begin_pass(P, bounces, nl == 1 && pass == 0 ? 1 : 0, stream); });
       launch("generate", [&]() { return hpt_generate(Fp, P, stream); });
       // with self-training no path goes beyond the vertex after the cache's
       // (in worlds without volumes: training paths from volume vertices run
@@ -2869,8 +2865,8 @@ ManagedObject *HipDevice::renderFrame(ManagedObject *fbo, ManagedObject *ro, Man
       for (int b = 0; b <= lastBounce; b++) {
         const std::string at = profile && profileBounces ? "@" + std::to_string(b) : std::string();
         auto nm = [&](const char *stage) { return at.empty() ? std::string(stage) : stage + at; };
-        atBounce(paths, b);
-        atBounce(sidePaths, b);
+        hpt::atBounce(paths, (size_t)b);
+        hpt::atBounce(sidePaths, (size_t)b);
         launch(nm("extend").c_str(),
             [&]() { return hpt_extend(S, P, q, residentTraceBlocks, travStats ? 1 : 0, stream); });
         launch(nm("ties").c_str(), [&]() { return hpt_ties(S, P, tieBlocks(), travStats ? 1 : 0, stream); });
@@ -2920,7 +2916,9 @@ ManagedObject *HipDevice::renderFrame(ManagedObject *fbo, ManagedObject *ro, Man
       }
       if (nl > 1 && pass > 0) // accumulate after the previous pass
         HIP_CHECK(hipStreamWaitEvent(stream, passEvents[(pass - 1) & 1], 0));
-      launch("finish_pass", [&]() { return hpt_finish_pass(Fp, P, stream); });
+      launch("finish_pass", [&]() {
+        return F.passS0 + F.passCount >= F.spp ? hpt_finish_frame(Fp, P, stream) : hpt_finish_pass(Fp, P, stream);
+      });
       if (nl > 1)
         HIP_CHECK(hipEventRecord(passEvents[pass & 1], stream));
       if (!capturing) {

@@ -218,6 +218,22 @@ __device__ __forceinline__ bool frameCancelled(const uint32_t *latch)
   return latch && __hip_atomic_load(latch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u;
 }
 
+// Counters that bounces use again (twoQueues): clears na words from a and nb
+// from b.  With keep, polls the frame's cancellation first, and a cancelled
+// frame empties the queue of that counter too.  One block.
+__global__ __launch_bounds__(256) void k_reset(DPaths P, int32_t *a, int na, int32_t *b, int nb, int32_t *keep, int poll)
+{
+  for (int i = threadIdx.x; i < na; i += blockDim.x)
+    a[i] = 0;
+  for (int i = threadIdx.x; i < nb; i += blockDim.x)
+    b[i] = 0;
+  if (threadIdx.x == 0 && poll) {
+    latchCancel(P);
+    if (keep && frameCancelled(P.cancelLatch))
+      *keep = 0;
+  }
+}
+
 // The entries a bounce kernel has to work on: none once the frame is
 // cancelled.  Waves of one kernel may disagree (the latch is set while they
 // start), so a kernel with barriers asks in one thread (blockEntries).
@@ -541,7 +557,7 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(5))
   uint32_t *ovf = P.overflow + (size_t)globalId() * kThreadRow;
   TraceStats st = {0, 0};
   uint32_t rays = 0;
-  traceQueue<MODE_CLOSEST, STATS, false, TIES_REPORT, kExtendRefill>(S, P.queue[qin], n, P.counters + kCntFetchExtend, lds, ovf, st,
+  traceQueue<MODE_CLOSEST, STATS, false, TIES_REPORT, kExtendRefill>(S, P.queue[qin], n, P.stage + kCntFetchExtend, lds, ovf, st,
       [&](uint32_t p, vec3f &org, vec3f &dir, float &t0, float &tfar) {
         const float4 o = ld4(P.org + 4 * (size_t)p);
         const float4 d = ld4(P.dir + 4 * (size_t)p);
@@ -559,7 +575,7 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(5))
         P.hitPrim[p] = h.prim | (h.half << 31);
         rays++;
         if (ts.tie) // rare: k_ties re-resolves the hit in FP64
-          P.tieQueue[atomicAdd(&P.counters[kCntTies], 1)] = p;
+          P.tieQueue[atomicAdd(&P.stage[kCntTies], 1)] = p;
       });
   if (STATS) {
     waveAdd(&P.stats[0], st.nodes);
@@ -575,7 +591,7 @@ template <bool STATS>
 __global__ __launch_bounds__(kTraceBlock) void k_ties(DScene S, DPaths P)
 {
   __shared__ uint32_t lds[kLdsDepth * kTraceBlock];
-  const int n = queueEntries(P, &P.counters[kCntTies]);
+  const int n = queueEntries(P, &P.stage[kCntTies]);
   uint32_t *ovf = P.overflow + (size_t)globalId() * kThreadRow;
   TraceStats st = {0, 0};
   for (int i = globalId(); i < n; i += gridStride()) {
@@ -1055,7 +1071,7 @@ __device__ __attribute__((noinline)) void flushShadowStage(DPaths &P, const uint
     before += x;
   }
   if (t == 0)
-    stageBase = (uint32_t)atomicAdd(&P.counters[kCntShadow], (int)cnt);
+    stageBase = (uint32_t)atomicAdd(&P.stage[kCntShadow], (int)cnt);
   __syncthreads();
   // column t now holds thread t's first position in each bucket
   for (int k = 0; k < kStagePerThread; k++)
@@ -1171,13 +1187,13 @@ template <bool STATS>
 __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(5))) void k_shadow(DScene S, DFrame F, DPaths P)
 {
   __shared__ uint32_t lds[kLdsDepth * kTraceBlock];
-  const int n = queueEntries(P, &P.counters[kCntShadow]);
+  const int n = queueEntries(P, &P.stage[kCntShadow]);
   if (n == 0) // an empty queue: no work fetch
     return;
   uint32_t *ovf = P.overflow + (size_t)globalId() * kThreadRow;
   TraceStats st = {0, 0};
   uint32_t rays = 0;
-  traceQueue<MODE_OCCLUSION, STATS, true, TIES_OFF, kShadowRefill>(S, P.shadowQueue, n, P.counters + kCntFetchShadow, lds, ovf, st,
+  traceQueue<MODE_OCCLUSION, STATS, true, TIES_OFF, kShadowRefill>(S, P.shadowQueue, n, P.stage + kCntFetchShadow, lds, ovf, st,
       [&](uint32_t r, vec3f &org, vec3f &dir, float &t0, float &tfar) {
         const float4 o4 = ld4(P.recOrg + 4 * (size_t)r);
         const float4 d4 = ld4(P.recDir + 4 * (size_t)r);
@@ -1205,7 +1221,7 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(5))
             }
           }
         }
-        const int slot = enqueue(&P.counters[kCntTrans], toTrans);
+        const int slot = enqueue(&P.stage[kCntTrans], toTrans);
         if (toTrans) {
           P.transQueue[slot] = r;
           if (slot < P.transCap) {
@@ -1239,7 +1255,7 @@ template <bool STATS>
 __global__ __launch_bounds__(kTraceBlock) void k_shadow_trans(DScene S, DFrame F, DPaths P)
 {
   __shared__ uint32_t lds[kLdsDepth * kTraceBlock];
-  const int n = queueEntries(P, &P.counters[kCntTrans]);
+  const int n = queueEntries(P, &P.stage[kCntTrans]);
   if (n == 0) // an empty queue: no work fetch
     return;
   uint32_t *ovf = P.overflow + (size_t)globalId() * kThreadRow;
@@ -1397,17 +1413,14 @@ __device__ __forceinline__ float linearToSrgb(float x)
 }
 
 // ColorConversion_kernel (fb/frame_ops/ColorConversion.ispc:11-36)
-__device__ __forceinline__ void convertColor(const DFrame &F, int pix, float4 v)
+__device__ __forceinline__ void convertColor(int format, void *out, int pix, float4 v)
 {
-  if (!F.fbConverted)
-    return;
-  if (F.fbFormat == 3) {
-    st4((float *)F.fbConverted + 4 * (size_t)pix, maxf(v.x, 0.f), maxf(v.y, 0.f), maxf(v.z, 0.f),
-        minf(maxf(v.w, 0.f), 1.f));
-  } else if (F.fbFormat == 1) {
-    ((uint32_t *)F.fbConverted)[pix] = cvtU8(v.x) | (cvtU8(v.y) << 8) | (cvtU8(v.z) << 16) | (cvtU8(v.w) << 24);
+  if (format == 3) {
+    st4((float *)out + 4 * (size_t)pix, maxf(v.x, 0.f), maxf(v.y, 0.f), maxf(v.z, 0.f), minf(maxf(v.w, 0.f), 1.f));
+  } else if (format == 1) {
+    ((uint32_t *)out)[pix] = cvtU8(v.x) | (cvtU8(v.y) << 8) | (cvtU8(v.z) << 16) | (cvtU8(v.w) << 24);
   } else {
-    ((uint32_t *)F.fbConverted)[pix] = cvtU8(linearToSrgb(v.x)) | (cvtU8(linearToSrgb(v.y)) << 8)
+    ((uint32_t *)out)[pix] = cvtU8(linearToSrgb(v.x)) | (cvtU8(linearToSrgb(v.y)) << 8)
         | (cvtU8(linearToSrgb(v.z)) << 16) | (cvtU8(v.w) << 24);
   }
 }
@@ -1432,8 +1445,11 @@ __device__ __forceinline__ void accumulatePixel(
     st4(c, r.x, r.y, r.z, r.w);
     return r;
   };
-  if (F.fbColor)
-    convertColor(F, pix, blend(F.fbColor + 4 * (size_t)pix, accScale));
+  if (F.fbColor) {
+    const float4 c = blend(F.fbColor + 4 * (size_t)pix, accScale);
+    if (F.fbConverted)
+      convertColor(F.fbFormat, F.fbConverted, pix, c);
+  }
   if (F.fbVariance && accVar)
     blend(F.fbVariance + 4 * (size_t)pix, accVarScale);
   bool updateIDs = accumID == 0;
@@ -1467,16 +1483,17 @@ __device__ __forceinline__ void accumulatePixel(
 
 // end of samplePath + ScreenSample_accumulate over the pass's samples
 // (PathSampler.ispc:409-414, PathTracer.ispc:196-197, ScreenSample.ih:59-77).
-// A frame's last pass goes on to the framebuffer with the sums in registers:
-// HBM bound, and as three kernels the sums and the colour made another trip
-// (1920x1080 at 4 spp 0.118 -> 0.092 ms, on small frames two launches).
+// LAST: a frame's last pass goes on to the framebuffer with the sums in
+// registers: HBM bound, and as three kernels (hpt_finish_pass,
+// hpt_fb_accumulate, hpt_color_convert) the sums and the colour made another
+// trip (1920x1080 at 4 spp 0.118 -> 0.092 ms, on small frames two launches).
+template <bool LAST>
 __global__ __launch_bounds__(256) void k_finish_pass(DFrame F, DPaths P)
 {
   if (frameCancelled(F.cancelLatch))
     return;
   const int npix = F.width * F.height;
   const float adaptive = frameAdaptive(F);
-  const bool last = F.passS0 + F.passCount >= F.spp;
   const int accumID = (int)frameAccumID(F);
   const bool accVar = frameAccVar(F);
   for (int pix = globalId(); pix < npix; pix += gridStride()) {
@@ -1525,7 +1542,7 @@ __global__ __launch_bounds__(256) void k_finish_pass(DFrame F, DPaths P)
         ids[2] = P.ids[4 * p + 2];
       }
     }
-    if (last) {
+    if (LAST) {
       accumulatePixel(F, pix, acc, aux, z, ids, accumID, accVar);
       continue;
     }
@@ -1537,6 +1554,35 @@ __global__ __launch_bounds__(256) void k_finish_pass(DFrame F, DPaths P)
     for (int k = 0; k < 3; k++)
       F.accIDs[3 * (size_t)pix + k] = ids[k];
   }
+}
+
+// the framebuffer's half of a last pass, from the stored sums
+__global__ __launch_bounds__(256) void k_fb_accumulate(DFrame F)
+{
+  if (frameCancelled(F.cancelLatch)) // a cancelled frame leaves the framebuffer as it was
+    return;
+  const int npix = F.width * F.height;
+  const float adaptive = frameAdaptive(F);
+  const int accumID = (int)frameAccumID(F);
+  const bool accVar = frameAccVar(F);
+  F.fbConverted = nullptr; // hpt_color_convert's
+  for (int pix = globalId(); pix < npix; pix += gridStride()) {
+    if (!taskActive(F, adaptive, pix % F.width, pix / F.width))
+      continue;
+    float aux[12];
+    for (int k = 0; k < 12; k++)
+      aux[k] = F.accAux ? F.accAux[12 * (size_t)pix + k] : 0.f;
+    uint32_t ids[3];
+    for (int k = 0; k < 3; k++)
+      ids[k] = F.accIDs[3 * (size_t)pix + k];
+    accumulatePixel(F, pix, ld4(F.accRGBA + 4 * (size_t)pix), aux, F.accZ[pix], ids, accumID, accVar);
+  }
+}
+
+__global__ __launch_bounds__(256) void k_color_convert(const float *color, int npix, int format, void *out)
+{
+  for (int i = globalId(); i < npix; i += gridStride())
+    convertColor(format, out, i, ld4(color + 4 * (size_t)i));
 }
 
 // Variance_kernel (fb/frame_ops/Variance.ispc:11-59), one thread per task;
@@ -1696,10 +1742,66 @@ extern "C" {
 
 hipError_t hpt_begin_pass(const HptPaths *P, int bounces, int firstPass, hipStream_t s)
 {
-  const uint32_t words = (uint32_t)counterWords(bounces);
-  hipLaunchKernelGGL(k_begin_pass, dim3(gridFor(words, 256, 1024)), dim3(256), 0, s,
-      *reinterpret_cast<const DPaths *>(P), words, firstPass);
+  const DPaths &p = *reinterpret_cast<const DPaths *>(P);
+  if (!p.pass || bounces < 0)
+    return hipErrorInvalidValue;
+  const uint32_t words = (uint32_t)counterWords((size_t)bounces);
+  hipLaunchKernelGGL(k_begin_pass, dim3(gridFor(words, 256, 1024)), dim3(256), 0, s, p, words, firstPass);
   return hipGetLastError();
+}
+
+size_t hpt_counter_bytes(int bounces) { return 4 * counterWords((size_t)(bounces < 0 ? 0 : bounces)); }
+
+void hpt_at_bounce(HptPaths *P, int bounce) { atBounce(*reinterpret_cast<DPaths *>(P), (size_t)bounce); }
+
+namespace {
+// the paths as the kernels of a bounce that reads extension queue `queue` see them
+DPaths pathsAt(const HptPaths *P, int queue)
+{
+  const DPaths &p = *reinterpret_cast<const DPaths *>(P);
+  return p.pass ? p : twoQueues(p, queue);
+}
+hipError_t launchReset(const HptPaths *P, int queue, int32_t *a, int na, int32_t *b, int nb, int32_t *keep, bool poll,
+    hipStream_t s)
+{
+  hipLaunchKernelGGL(k_reset, dim3(1), dim3(256), 0, s, pathsAt(P, queue), a, na, b, nb, keep, poll ? 1 : 0);
+  return hipGetLastError();
+}
+} // namespace
+
+hipError_t hpt_reset_counters(const HptPaths *P, int keepIndex, hipStream_t s)
+{
+  const DPaths p = pathsAt(P, keepIndex < 0 ? 0 : keepIndex);
+  if (reinterpret_cast<const DPaths *>(P)->pass)
+    return hipErrorInvalidValue;
+  if (keepIndex < 0)
+    return launchReset(P, 0, p.pass, kNumCounters, nullptr, 0, nullptr, true, s);
+  return launchReset(P, keepIndex, p.stage, kBounceWords, p.next, 2, p.counters + kCntExtend, true, s);
+}
+
+hipError_t hpt_reset_extension_counters(const HptPaths *P, int keepIndex, hipStream_t s)
+{
+  const DPaths p = pathsAt(P, keepIndex);
+  if (reinterpret_cast<const DPaths *>(P)->pass)
+    return hipErrorInvalidValue;
+  return launchReset(P, keepIndex, p.stage + kCntTies, 1, p.stage + kCntFetchExtend, kXcds * kFetchStride,
+      p.counters + kCntExtend, true, s);
+}
+
+hipError_t hpt_reset_append_counters(const HptPaths *P, int keepIndex, hipStream_t s)
+{
+  const DPaths p = pathsAt(P, keepIndex);
+  if (reinterpret_cast<const DPaths *>(P)->pass)
+    return hipErrorInvalidValue;
+  return launchReset(P, keepIndex, p.next, 2, nullptr, 0, nullptr, false, s);
+}
+
+hipError_t hpt_reset_shadow_counters(const HptPaths *P, hipStream_t s)
+{
+  const DPaths p = pathsAt(P, 0);
+  if (reinterpret_cast<const DPaths *>(P)->pass)
+    return hipErrorInvalidValue;
+  return launchReset(P, 0, p.stage + kCntShadow, 2, p.stage + kCntFetchShadow, kXcds * kFetchStride, nullptr, false, s);
 }
 
 hipError_t hpt_fill_u32(uint32_t *ptr, size_t n, uint32_t value, hipStream_t s)
@@ -1721,14 +1823,14 @@ hipError_t hpt_generate(const HptFrame *F, const HptPaths *P, hipStream_t s)
 {
   const DFrame &f = *reinterpret_cast<const DFrame *>(F);
   const size_t n = (size_t)f.passCount * f.numPixPadded;
-  hipLaunchKernelGGL(k_generate, dim3(gridFor(n, 256, 16384)), dim3(256), 0, s, f, *reinterpret_cast<const DPaths *>(P));
+  hipLaunchKernelGGL(k_generate, dim3(gridFor(n, 256, 16384)), dim3(256), 0, s, f, pathsAt(P, 0));
   return hipGetLastError();
 }
 
 hipError_t hpt_extend(const HptScene *S, const HptPaths *P, int queue, int residentBlocks, int stats, hipStream_t s)
 {
   const DScene &sc = *reinterpret_cast<const DScene *>(S);
-  const DPaths &p = *reinterpret_cast<const DPaths *>(P);
+  const DPaths p = pathsAt(P, queue);
   if (stats)
     hipLaunchKernelGGL(k_extend<true>, dim3(residentBlocks), dim3(kTraceBlock), 0, s, sc, p, queue);
   else
@@ -1739,7 +1841,7 @@ hipError_t hpt_extend(const HptScene *S, const HptPaths *P, int queue, int resid
 hipError_t hpt_ties(const HptScene *S, const HptPaths *P, int residentBlocks, int stats, hipStream_t s)
 {
   const DScene &sc = *reinterpret_cast<const DScene *>(S);
-  const DPaths &p = *reinterpret_cast<const DPaths *>(P);
+  const DPaths p = pathsAt(P, 0);
   if (stats)
     hipLaunchKernelGGL(k_ties<true>, dim3(residentBlocks), dim3(kTraceBlock), 0, s, sc, p);
   else
@@ -1751,7 +1853,7 @@ hipError_t hpt_shade(const HptScene *S, const HptFrame *F, const HptPaths *P, in
 {
   const DScene &sc = *reinterpret_cast<const DScene *>(S);
   const DFrame &f = *reinterpret_cast<const DFrame *>(F);
-  const DPaths &p = *reinterpret_cast<const DPaths *>(P);
+  const DPaths p = pathsAt(P, queue);
   // the volume variant carries the sampler and transmittance code (more
   // registers), the cache variant the cache records (the caller passes a
   // frame with nrcBounce -1 for the other bounces); surface-only worlds run
@@ -1800,7 +1902,7 @@ hipError_t hpt_nrc_targets(const HptPaths *P, int n, float *target3, hipStream_t
 hipError_t hpt_nee(const HptScene *S, const HptFrame *F, const HptPaths *P, int queue, int blocks, hipStream_t s)
 {
   hipLaunchKernelGGL(k_nee, dim3(blocks), dim3(kNeeBlock), 0, s, *reinterpret_cast<const DScene *>(S),
-      *reinterpret_cast<const DFrame *>(F), *reinterpret_cast<const DPaths *>(P), queue);
+      *reinterpret_cast<const DFrame *>(F), pathsAt(P, queue), queue);
   return hipGetLastError();
 }
 
@@ -1809,7 +1911,7 @@ hipError_t hpt_shadow(
 {
   const DScene &sc = *reinterpret_cast<const DScene *>(S);
   const DFrame &f = *reinterpret_cast<const DFrame *>(F);
-  const DPaths &p = *reinterpret_cast<const DPaths *>(P);
+  const DPaths p = pathsAt(P, 0);
   if (stats) {
     hipLaunchKernelGGL(k_shadow<true>, dim3(residentBlocks), dim3(kTraceBlock), 0, s, sc, f, p);
   } else {
@@ -1823,7 +1925,7 @@ hipError_t hpt_shadow_trans(
 {
   const DScene &sc = *reinterpret_cast<const DScene *>(S);
   const DFrame &f = *reinterpret_cast<const DFrame *>(F);
-  const DPaths &p = *reinterpret_cast<const DPaths *>(P);
+  const DPaths p = pathsAt(P, 0);
   if (stats)
     hipLaunchKernelGGL(k_shadow_trans<true>, dim3(residentBlocks), dim3(kTraceBlock), 0, s, sc, f, p);
   else
@@ -1834,7 +1936,7 @@ hipError_t hpt_shadow_trans(
 hipError_t hpt_volume(const HptScene *S, const HptPaths *P, int queue, int blocks, int stats, hipStream_t s)
 {
   hipLaunchKernelGGL(k_volume, dim3(blocks), dim3(256), 0, s, *reinterpret_cast<const DScene *>(S),
-      *reinterpret_cast<const DPaths *>(P), queue, stats);
+      pathsAt(P, queue), queue, stats);
   return hipGetLastError();
 }
 
@@ -1842,7 +1944,7 @@ hipError_t hpt_resolve(const HptScene *S, const HptFrame *F, const HptPaths *P, 
 {
   const DScene &sc = *reinterpret_cast<const DScene *>(S);
   const DFrame &f = *reinterpret_cast<const DFrame *>(F);
-  const DPaths &p = *reinterpret_cast<const DPaths *>(P);
+  const DPaths p = pathsAt(P, queue);
   if (sc.numVolInsts > 0)
     hipLaunchKernelGGL(k_resolve<true>, dim3(blocks), dim3(256), 0, s, sc, f, p, queue);
   else
@@ -1853,8 +1955,23 @@ hipError_t hpt_resolve(const HptScene *S, const HptFrame *F, const HptPaths *P, 
 hipError_t hpt_finish_pass(const HptFrame *F, const HptPaths *P, hipStream_t s)
 {
   const DFrame &f = *reinterpret_cast<const DFrame *>(F);
-  hipLaunchKernelGGL(k_finish_pass, dim3(gridFor((size_t)f.width * f.height, 256, 16384)), dim3(256), 0, s, f,
+  hipLaunchKernelGGL(k_finish_pass<false>, dim3(gridFor((size_t)f.width * f.height, 256, 16384)), dim3(256), 0, s, f,
       *reinterpret_cast<const DPaths *>(P));
+  return hipGetLastError();
+}
+
+hipError_t hpt_finish_frame(const HptFrame *F, const HptPaths *P, hipStream_t s)
+{
+  const DFrame &f = *reinterpret_cast<const DFrame *>(F);
+  hipLaunchKernelGGL(k_finish_pass<true>, dim3(gridFor((size_t)f.width * f.height, 256, 16384)), dim3(256), 0, s, f,
+      *reinterpret_cast<const DPaths *>(P));
+  return hipGetLastError();
+}
+
+hipError_t hpt_fb_accumulate(const HptFrame *F, hipStream_t s)
+{
+  const DFrame &f = *reinterpret_cast<const DFrame *>(F);
+  hipLaunchKernelGGL(k_fb_accumulate, dim3(gridFor((size_t)f.width * f.height, 256, 16384)), dim3(256), 0, s, f);
   return hipGetLastError();
 }
 
@@ -1870,6 +1987,12 @@ hipError_t hpt_variance_reduce(const float *taskVariance, int n, float threshold
     const uint32_t *frameState, hipStream_t s)
 {
   hipLaunchKernelGGL(k_variance_reduce, dim3(1), dim3(256), 0, s, taskVariance, n, threshold, out, frameState);
+  return hipGetLastError();
+}
+
+hipError_t hpt_color_convert(const float *color, int npix, int format, void *out, hipStream_t s)
+{
+  hipLaunchKernelGGL(k_color_convert, dim3(gridFor((size_t)npix, 256, 16384)), dim3(256), 0, s, color, npix, format, out);
   return hipGetLastError();
 }
 

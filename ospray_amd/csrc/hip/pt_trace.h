@@ -42,7 +42,7 @@ constexpr int kLdsDepth = 24;
 constexpr int kOverflowDepth = 112;
 // Entries a world may need by the builders' count: one less than its children
 // for each node on the way down, and the two of an instance's entry.  The rows
-// hold more: a ray that enters an unused slot of a node (k_relocate) pushes
+// hold more: a ray that enters an unused slot of a node (k_place) pushes
 // that too, up to three entries beyond the count in the BLAS and in the TLAS
 // each, since only a node without inner children has unused slots; and one row
 // holds the sentinel.  (A multiple of four, so that the recorded hits stay
@@ -324,7 +324,7 @@ __device__ __forceinline__ NodeAxis nodeAxis(float p, float s, uint32_t lo, uint
 // ulp, 2 u), their product, the padding's and the last sum on M, 1 / d, s / d
 // and the last sum on Q.  The near planes are moved down and the far ones up
 // by 12 u |M| here and by 10 u of the node's size over |d| in the grid itself
-// (k_relocate), which leaves 6 u of both for a primitive's own hit distance,
+// (k_place), which leaves 6 u of both for a primitive's own hit distance,
 // so the closest hit does not depend on the tree.  Neither padding looks
 // further than the node and the ray's origin: culling next to an object does
 // not depend on what else is in the tree, nor on where the origin of the

@@ -255,10 +255,13 @@ struct DPaths
   uint32_t *transQueue; // shadow records that hit only non-opaque surfaces
   uint32_t *neeSampleQueue; // record slots (path * maxRec + sample) to evaluate
   uint32_t *tieQueue; // path slots whose extension hit is re-resolved in FP64
-  // counters of the bounce at hand and of the next one (kCnt*), and of the
-  // pass (kPass*): each bounce has a block of its own in one buffer, cleared
-  // once when the pass begins
-  int32_t *counters, *next, *pass;
+  // Counters of the bounce at hand and of the next one (their first two),
+  // of the bounce's stages (the others), and of the pass (kPass*): each
+  // bounce has a block of its own in one buffer, cleared once when the pass
+  // begins (hpt_begin_pass, atBounce).  With pass == null, `counters` is a
+  // buffer of kNumCounters words that every bounce uses again, with the
+  // hpt_reset_* calls in between (twoQueues).
+  int32_t *counters, *next, *stage, *pass;
   uint32_t *overflow; // traversal scratch row per resident thread: stack overflow, recorded hits
   // transparent hits recorded by the occlusion pass for the records of the
   // transparency queue, by queue slot < transCap: 4 float4 and a count
@@ -309,7 +312,26 @@ constexpr int kPassNrcTrain = 1; // radiance-cache training records
 constexpr int kPassWords = 32;
 // words of the counters of a pass of `bounces` bounces; the last one's
 // shading has a next block too
-constexpr size_t counterWords(int bounces) { return kPassWords + (size_t)(bounces + 1) * kBounceWords; }
+constexpr size_t counterWords(size_t bounces) { return kPassWords + (bounces + 1) * kBounceWords; }
+
+// the counters of bounce b
+inline void atBounce(DPaths &p, size_t b)
+{
+  p.counters = p.stage = p.pass + kPassWords + b * kBounceWords;
+  p.next = p.counters + kBounceWords;
+}
+
+// Counters that every bounce uses again: the pass's, a block for each of the
+// two extension queues and one for the stages.
+constexpr int kNumCounters = kPassWords + 3 * kBounceWords;
+inline DPaths twoQueues(DPaths p, int queue)
+{
+  p.pass = p.counters;
+  p.counters = p.pass + kPassWords + (queue & 1) * kBounceWords;
+  p.next = p.pass + kPassWords + ((queue & 1) ^ 1) * kBounceWords;
+  p.stage = p.pass + kPassWords + 2 * kBounceWords;
+  return p;
+}
 
 // path flags in ld[3]
 constexpr uint32_t FLAG_DEPTH_MASK = 0xffu; // bits 0-7

@@ -42,6 +42,22 @@ def test_module_exports_every_declared_function():
     assert not missing, missing
 
 
+def test_stage_entry_points_stay():
+    """What a caller of the stage kernels was given stays, with its arguments."""
+    text = " ".join(open(os.path.join(ROOT, "include", "ospray_hip", "hip_pt.h")).read().split())
+    text += " ".join(open(os.path.join(ROOT, "include", "ospray_hip", "hip_bvh.h")).read().split())
+    for decl in ("hpt_reset_counters(const HptPaths *P, int keepIndex, hipStream_t s)",
+                 "hpt_reset_extension_counters(const HptPaths *P, int keepIndex, hipStream_t s)",
+                 "hpt_reset_append_counters(const HptPaths *P, int keepIndex, hipStream_t s)",
+                 "hpt_reset_shadow_counters(const HptPaths *P, hipStream_t s)",
+                 "hpt_finish_pass(const HptFrame *F, const HptPaths *P, hipStream_t s)",
+                 "hpt_fb_accumulate(const HptFrame *F, hipStream_t s)",
+                 "hpt_color_convert(const float *color, int npix, int format, void *out, hipStream_t s)",
+                 "hpt_bvh_relocate(void *dst, const void *src, size_t n, int32_t nodeOffset, uint32_t primOffset, "
+                 "hipStream_t s)"):
+        assert "HPT_API hipError_t " + decl + ";" in text, decl
+
+
 def test_module_version_check():
     lib = C.CDLL(os.path.join(K.LIBDIR, "libospray_module_hip.so"), mode=C.RTLD_GLOBAL)
     init = lib.ospray_module_init_hip
