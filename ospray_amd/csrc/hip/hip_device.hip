@@ -2771,7 +2771,7 @@ ManagedObject *HipDevice::renderFrame(ManagedObject *fbo, ManagedObject *ro, Man
       sppPerPass = std::min(sppPerPass, (F.spp + nl - 1) / nl);
       nl = std::min(nl, (F.spp + sppPerPass - 1) / sppPerPass);
     }
-    const int bounces = F.maxDepth + 1;
+    const int bounces = std::min(F.maxDepth, INT32_MAX - 1) + 1;
     PathLane *const frameLane = lane;
     for (int k = nl - 1; k >= 0; k--) {
       lane = k == 0 ? frameLane : &ensureLane(k);

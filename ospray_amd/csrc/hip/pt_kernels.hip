@@ -201,9 +201,9 @@ __device__ __forceinline__ void latchCancel(const DPaths &P)
 // on a frame's first pass the frame's cancellation latch.  Kernels of a
 // bounce then find their counters clear without a launch in between (three
 // resets a bounce were 12 of its 95 us on a 64x64 frame: 613 -> 563 us).
-__global__ __launch_bounds__(256) void k_begin_pass(DPaths P, uint32_t words, int first)
+__global__ __launch_bounds__(256) void k_begin_pass(DPaths P, size_t words, int first)
 {
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < words; i += gridDim.x * blockDim.x)
+  for (size_t i = blockIdx.x * blockDim.x + threadIdx.x; i < words; i += gridDim.x * blockDim.x)
     P.pass[i] = 0;
   if (blockIdx.x == 0 && threadIdx.x == 0 && P.cancelLatch) {
     if (first)
@@ -1745,7 +1745,7 @@ hipError_t hpt_begin_pass(const HptPaths *P, int bounces, int firstPass, hipStre
   const DPaths &p = *reinterpret_cast<const DPaths *>(P);
   if (!p.pass || bounces < 0)
     return hipErrorInvalidValue;
-  const uint32_t words = (uint32_t)counterWords((size_t)bounces);
+  const size_t words = counterWords((size_t)bounces);
   hipLaunchKernelGGL(k_begin_pass, dim3(gridFor(words, 256, 1024)), dim3(256), 0, s, p, words, firstPass);
   return hipGetLastError();
 }

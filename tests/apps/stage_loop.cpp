@@ -154,3 +154,11 @@ extern "C" int stage_loop(const HptScene *S, int w, int h, int spp, int perPass,
   TRY(hipMemcpy(outBytes, bytes, 4 * npix, hipMemcpyDeviceToHost));
   return 0;
 }
+
+// the counters at `pass` as a pass of `bounces` bounces finds them
+extern "C" int begin_pass(int32_t *pass, int bounces)
+{
+  hpt::DPaths p{};
+  p.pass = pass;
+  return (int)hpt_begin_pass(reinterpret_cast<const HptPaths *>(&p), bounces, 1, nullptr);
+}

@@ -26,10 +26,12 @@ def stage_loop(tmp_path_factory):
                     f"-I{ROOT}/ospray_amd/csrc/hip", f"-I{rocm}/include", "-o", so,
                     os.path.join(ROOT, "tests", "apps", "stage_loop.cpp"), f"-L{K.LIBDIR}", "-l:libospray_module_hip.so",
                     f"-Wl,-rpath,{K.LIBDIR}", f"-L{rocm}/lib", "-lamdhip64"], check=True)
-    f = C.CDLL(so).stage_loop
+    lib = C.CDLL(so)
+    lib.begin_pass.argtypes = [C.c_void_p, C.c_int]
+    f = lib.stage_loop
     f.restype = C.c_int
     f.argtypes = [C.c_void_p] + [C.c_int] * 5 + [C.c_float, C.c_void_p, C.c_int, C.c_int, C.c_void_p, C.c_void_p]
-    return f
+    return lib
 
 
 def _scene():
@@ -60,7 +62,7 @@ def test_frame_equals_the_device(hip_device, stage_loop, counters):
     scene = mod.ospHipGetWorldLaunchScene(s.world.h)
     color, words = np.zeros((h, w, 4), np.float32), np.zeros((h, w), np.uint32)
     pos = np.array(sc.camera["position"], np.float32)
-    rc = stage_loop(scene, w, h, spp, 2, depth, sc.camera["fovy"], pos.ctypes.data, counters, 64, color.ctypes.data,
+    rc = stage_loop.stage_loop(scene, w, h, spp, 2, depth, sc.camera["fovy"], pos.ctypes.data, counters, 64, color.ctypes.data,
                     words.ctypes.data)
     assert rc == 0
     assert want[K.OSP_FB_RGBA32F][..., :3].any()
@@ -69,6 +71,26 @@ def test_frame_equals_the_device(hip_device, stage_loop, counters):
     mapped[..., 3] = np.minimum(mapped[..., 3], np.float32(1))
     assert np.array_equal(mapped, want[K.OSP_FB_RGBA32F])
     assert np.array_equal(words.view(np.uint8).reshape(h, w, 4), want[K.OSP_FB_SRGBA])
+
+
+@pytest.mark.parametrize("bounces", [0, 20, 7895200])
+def test_counters_of_any_path_length(hip_device, stage_loop, bounces):
+    """hpt_begin_pass clears hpt_counter_bytes(bounces) bytes, 17 GB (more than
+    2^32 words) of them too."""
+    torch = pytest.importorskip("torch")
+    size = C.CDLL(os.path.join(K.LIBDIR, "libospray_module_hip.so")).hpt_counter_bytes
+    size.restype = C.c_size_t
+    size.argtypes = [C.c_int]
+    words = size(bounces) // 4
+    assert (words > 2 ** 32) == (bounces > 20)
+    t = torch.ones(words + 64, dtype=torch.int32, device="cuda")
+    assert stage_loop.begin_pass(t.data_ptr(), bounces) == 0
+    torch.cuda.synchronize()
+    edge = min(words, 1 << 22)
+    assert not t[:edge].any() and not t[words - edge:words].any()
+    assert t[words:].all()
+    del t
+    torch.cuda.empty_cache()
 
 
 def test_relocated_nodes(hip_device):
