@@ -775,8 +775,8 @@ struct Light : public ManagedObject
 };
 
 // BLAS of one list of geometries (shared by groups with the same list):
-// built on the device or on the host, the build nodes and primitive records
-// in dNodes/dPrims (of a host build from nodes/prims, once a world needs it)
+// built on the device (build nodes and primitive records in dNodes/dPrims) or
+// on the host (nodes/prims)
 struct Blas
 {
   std::vector<hpt::BNode4> nodes;
@@ -799,6 +799,9 @@ struct World : public ManagedObject
   std::vector<Material *> materials; // index order of the material table
   DevBuf dNodes, dPrims, dInstances, dModels, dMaterials, dMedia, dLights, dLightsCDF, dWorldLightsCDF, dGeoCDF;
   DevBuf dVolumes, dVolInsts;
+  // the BLASes, in order, that dNodes and dPrims hold before the TLAS: a
+  // commit that changes none of them (instances moved) writes the TLAS alone
+  std::vector<std::weak_ptr<Blas>> placed;
   hpt::DScene scene{};
   bool built = false;
   int64_t totalNodes = 0, totalPrims = 0;
@@ -2291,29 +2294,54 @@ void World::commit() // World.cpp:70-188 plus the Group BLAS builds (Group.cpp:9
   const size_t totalNodeCount = nNodes + T.nodes.size();
   D.gpu();
   HIP_CHECK(hipStreamSynchronize(D.stream)); // frames in flight read the old arrays
-  dNodes.ensure(sizeof(hpt::DNode4) * totalNodeCount);
-  dPrims.ensure(sizeof(hpt::DPrim) * (nPrims + 1)); // the leaf test reads records in pairs
+  const size_t nodeBytes = sizeof(hpt::DNode4) * totalNodeCount;
+  const size_t primBytes = sizeof(hpt::DPrim) * (nPrims + 1); // the leaf test reads records in pairs
+  bool inPlace = dNodes.ptr && dPrims.ptr && dNodes.bytes >= nodeBytes && dPrims.bytes >= primBytes
+      && placed.size() == uniqueBlas.size();
+  for (size_t k = 0; inPlace && k < uniqueBlas.size(); k++)
+    inPlace = placed[k].lock() == uniqueBlas[k];
+  placed.clear();
+  dNodes.ensure(nodeBytes);
+  dPrims.ensure(primBytes);
   hpt::DNode4 *gNodes = dNodes.as<hpt::DNode4>();
   hpt::DPrim *gPrims = dPrims.as<hpt::DPrim>();
   HIP_CHECK(hipMemsetAsync(gPrims, 0, sizeof(hpt::DPrim), D.stream));
-  for (size_t k = 0; k < uniqueBlas.size(); k++) {
-    Blas &B = *uniqueBlas[k];
-    if (!B.nodes.empty()) { // a host build's first world
-      B.dNodes.upload(B.nodes);
-      B.dPrims.upload(B.prims);
-      std::vector<hpt::BNode4>().swap(B.nodes);
-      std::vector<hpt::DPrim>().swap(B.prims);
+  // host-built nodes pass through a buffer of at most 2^19 of them (64 MiB),
+  // in stream order: a BLAS stays where it was built, and the device holds a
+  // host build once, in the world's layout
+  size_t staged = T.nodes.size();
+  for (size_t k = 0; !inPlace && k < uniqueBlas.size(); k++)
+    staged += uniqueBlas[k]->nodes.size();
+  staged = std::min(staged, (size_t)1 << 19);
+  DevBuf stage;
+  stage.ensure(sizeof(hpt::BNode4) * staged);
+  size_t used = 0;
+  auto placeHost = [&](const std::vector<hpt::BNode4> &nodes, int nodeOff, uint32_t primOff, int32_t unusedRef) {
+    for (size_t i = 0; i < nodes.size();) {
+      if (used == staged)
+        used = 0;
+      const size_t m = std::min(nodes.size() - i, staged - used);
+      hpt::BNode4 *at = stage.as<hpt::BNode4>() + used;
+      HIP_CHECK(hipMemcpyAsync(at, nodes.data() + i, sizeof(hpt::BNode4) * m, hipMemcpyHostToDevice, D.stream));
+      HIP_CHECK(hpt_bvh_place(gNodes + nodeOff + i, at, m, nodeOff, primOff, unusedRef, D.stream));
+      used += m;
+      i += m;
     }
-    HIP_CHECK(hpt_bvh_place(gNodes + blasNodeOff[k], B.dNodes.ptr, B.numNodes, blasNodeOff[k],
-        (uint32_t)blasPrimOff[k], kNoPrim, D.stream));
+  };
+  for (size_t k = 0; !inPlace && k < uniqueBlas.size(); k++) {
+    const Blas &B = *uniqueBlas[k];
+    if (B.onDevice)
+      HIP_CHECK(hpt_bvh_place(gNodes + blasNodeOff[k], B.dNodes.ptr, B.numNodes, blasNodeOff[k],
+          (uint32_t)blasPrimOff[k], kNoPrim, D.stream));
+    else
+      placeHost(B.nodes, blasNodeOff[k], (uint32_t)blasPrimOff[k], kNoPrim);
     if (B.numPrims > 0)
-      HIP_CHECK(hipMemcpyAsync(gPrims + blasPrimOff[k], B.dPrims.ptr, sizeof(hpt::DPrim) * B.numPrims,
-          hipMemcpyDeviceToDevice, D.stream));
+      HIP_CHECK(hipMemcpyAsync(gPrims + blasPrimOff[k], B.onDevice ? B.dPrims.ptr : B.prims.data(),
+          sizeof(hpt::DPrim) * B.numPrims, B.onDevice ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, D.stream));
   }
-  DevBuf tlas;
-  tlas.upload(T.nodes);
-  HIP_CHECK(hpt_bvh_place(gNodes + tlasOff, tlas.ptr, T.nodes.size(), tlasOff, 0, noInstance, D.stream));
+  placeHost(T.nodes, tlasOff, 0, noInstance);
   HIP_CHECK(hipStreamSynchronize(D.stream));
+  placed.assign(uniqueBlas.begin(), uniqueBlas.end());
 
   // lights (PathTracerData.cpp:32-82): [geometry lights, world lights],
   // uniform selection CDFs with and without the geometry lights.  Geometry

@@ -134,3 +134,79 @@ def test_device_bvh_renders_like_host(hip_device):
             _host_bvh(True)
     for a, b in zip(*out):
         assert np.array_equal(a, b)
+
+
+def test_host_build_is_held_once(hip_device):
+    """A world of 2.9M host-built triangles takes the device memory of its
+    nodes (64 B) and primitive records (48 B) and of its geometry, not the
+    builder's nodes (128 B) and a second copy of the records besides; its
+    nodes, more than pass to the device at once, give the device build's hits."""
+    torch = pytest.importorskip("torch")
+    n = 1200
+    gen = np.random.default_rng(11)
+    x = np.linspace(-50, 50, n, dtype=np.float32)
+    v = np.stack([np.tile(x, (n, 1)), gen.uniform(-0.05, 0.05, (n, n)), np.tile(x[:, None], (1, n))], -1)
+    k = np.arange(n * n, dtype=np.uint32).reshape(n, n)
+    a, b, c, d = k[:-1, :-1], k[1:, :-1], k[1:, 1:], k[:-1, 1:]
+    tri = np.stack([np.stack([a, b, c], -1), np.stack([a, c, d], -1)], 2).reshape(-1, 3)
+    sc = scenes.Scene("field", 8, 8, [scenes.Geometry("triangles", vertex=v.reshape(-1, 3).astype(np.float32), index=tri)],
+                      [scenes.Model(0, 0)], [[0]], [scenes.Instance(0)], [{"type": "obj"}], [{"type": "ambient"}],
+                      {"position": (0, 5, -1), "direction": (0, -1, 0.5)}, {"pixelSamples": 1})
+    rays = np.zeros((20000, 8), np.float32)
+    rays[:, :3] = gen.uniform(-40, 40, (20000, 3)) * (1, 0, 1) + (0, 5, 0)
+    rays[:, 3:6] = gen.normal(size=(20000, 3)) * 0.2 + (0, -1, 0)
+    rays[:, 7] = np.inf
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    s = scenes.to_ospray(sc)
+    used = free - torch.cuda.mem_get_info()[0]
+    nodes, prims = A.world_info(s.world)[:2]
+    assert nodes > 1 << 19
+    geometry = v.size * 4 + tri.nbytes
+    assert used <= 64 * nodes + 48 * prims + geometry + (32 << 20), (used, nodes, prims)
+    got = A.trace_rays(s.world, rays)[:2]
+    _host_bvh(False)
+    try:
+        want = A.trace_rays(scenes.to_ospray(sc).world, rays)[:2]
+    finally:
+        _host_bvh(True)
+    assert all(np.array_equal(p, q) for p, q in zip(got, want))
+    assert (got[1][:, 0] == 0).all()
+
+
+@pytest.mark.parametrize("host", [True, False])
+def test_recommitted_worlds(hip_device, host):
+    """A world whose instances move, change order, grow in number or name other
+    groups gives, after each commit, the hits of a world made afresh: what its
+    arrays hold from the commit before is used where it is the same, and only
+    there."""
+    rng = np.random.default_rng(17)
+    geo = [scenes.Geometry("triangles", vertex=rng.uniform(-1, 1, (3 * n, 3)).astype(np.float32),
+                           index=np.arange(3 * n, dtype=np.uint32).reshape(-1, 3)) for n in (40, 90, 25)]
+    sc = scenes.Scene("parts", 8, 8, geo, [scenes.Model(k, 0) for k in range(3)], [[0], [1], [2]],
+                      [scenes.Instance(k) for k in range(3)], [{"type": "obj"}], [{"type": "ambient"}],
+                      {"position": (0, 0, -1), "direction": (0, 0, 1)}, {"pixelSamples": 1})
+    _host_bvh(host)
+    try:
+        s = scenes.to_ospray(sc)
+        groups = [h for h in s.handles if h.type == K.OSP_GROUP]
+        rays = np.zeros((4000, 8), np.float32)
+        rays[:, :3] = rng.uniform(-8, 8, (4000, 3))
+        rays[:, 3:6] = -rays[:, :3] + rng.uniform(-6, 6, (4000, 3))
+        rays[:, 7] = np.inf
+        world, keep = A.new("world"), []
+        for names in ([0, 1], [0, 1], [1, 0], [0, 1] * 40, [0, 1], [2], [0, 1], [2, 1, 0]):
+            insts = []
+            for g in names:
+                x = tuple(np.eye(3).ravel()) + tuple(rng.uniform(-4, 4, 3))
+                insts.append(A.new("instance", params={"group": groups[g], "transform": A.Affine3f(x)}))
+            data = A.object_data(insts, K.OSP_INSTANCE)
+            A.set_params(world.h, {"instance": data})
+            A.commit(world)
+            got = A.trace_rays(world, rays)
+            want = A.trace_rays(A.new("world", params={"instance": data}), rays)
+            assert all(np.array_equal(p, q) for p, q in zip(got[:2], want[:2])) and got[2] == want[2], names
+            assert (got[1][:, 0] != 0xFFFFFFFF).any()
+            keep.append((insts, data))
+    finally:
+        _host_bvh(True)
