@@ -71,6 +71,13 @@ __device__ __forceinline__ float relu(float x)
 __device__ __forceinline__ int rowNeuron(int s) { return (s & 32) + ((s & 12) << 1) + ((s & 16) >> 2) + (s & 3); }
 __device__ __forceinline__ int neuronRow(int n) { return (n & 32) + ((n & 4) << 2) + ((n & 24) >> 1) + (n & 3); }
 
+// x of the lane N further on in the row of 16
+template <int N>
+__device__ __forceinline__ float rotated(float x)
+{
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x120 + N, 0xf, 0xf, false)); // row_ror
+}
+
 // Layers 1..4 of the forward pass in registers.
 // acc[nt][qt]: layer 0's sums in, o[qt]: W4 (16 x 64) x h4; rows 0..2 are
 // the outputs.  wf(layer, nt, kb) loads an A operand (of W4: nt 0, its own
@@ -261,13 +268,15 @@ __global__ __launch_bounds__(256) void k_nrc_train(HptNrc N, const __bf16 *X, co
       *reinterpret_cast<bf16x4 *>(dy + qo * kDyS + 4 * g) = dv;
     }
     __syncthreads();
-    if (threadIdx.x < 16) { // the tile's loss: queries r, r + 16, .. in order, then over r
+    if (threadIdx.x < 16) { // the tile's loss: queries r, r + 16, .. in order, then r + 8, 4, 2, 1
       float loss = 0.f;
       for (int qt = 0; qt < 4; qt++)
         for (int e = 0; e < 3; e++)
           loss += lossTerms[3 * (qt * 16 + r) + e];
-      for (int o2 = 8; o2 > 0; o2 >>= 1)
-        loss += __shfl_xor(loss, o2);
+      loss += rotated<8>(loss);
+      loss += rotated<4>(loss);
+      loss += rotated<2>(loss);
+      loss += rotated<1>(loss);
       if (r == 0)
         N.tileLoss[tile] = loss;
     }
@@ -373,7 +382,7 @@ __global__ __launch_bounds__(256) void k_nrc_init(HptNrc N, uint32_t seed)
 // a group (64 rows each of 256 tiles, a few in flight) a step took 35.2 us,
 // 0.69 TB/s.  Four waves share a group: each has kAdamRows of its rows in
 // flight at once, and they add theirs to the group's sum one after another,
-// which keeps the order and costs four barriers: 7.1 us, 3.3 TB/s (sixteen
+// which keeps the order and costs a barrier each: 6.9 us, 3.5 TB/s (sixteen
 // groups, an order of their own, 6.4).
 constexpr int kAdamGroups = 4, kAdamSegs = 4, kAdamRows = 16;
 __global__ __launch_bounds__(64 * kAdamGroups * kAdamSegs) void k_nrc_adam(HptNrc N, int tiles, float lr, float bc1, float bc2)
@@ -403,8 +412,6 @@ __global__ __launch_bounds__(64 * kAdamGroups * kAdamSegs) void k_nrc_adam(HptNr
     return;
   }
   const int p = blockIdx.x * 64 + col;
-  if (seg == 0)
-    part[grp][col] = 0.f;
   float m0 = 0.f, v0 = 0.f, w0 = 0.f; // on their way beside the rows
   if (wave == 0) {
     m0 = N.adamM[p];
@@ -422,10 +429,11 @@ __global__ __launch_bounds__(64 * kAdamGroups * kAdamSegs) void k_nrc_adam(HptNr
         x[i] = t < tiles ? v : 0.f;
       }
     }
-    for (int s = 0; s < kAdamSegs; s++) {
-      __syncthreads();
+    for (int s = 0; s < kAdamSegs && t0 + s * kAdamGroups * kAdamRows < tiles; s++) {
+      if (t0 + s > 0)
+        __syncthreads();
       if (seg == s) {
-        float gs = part[grp][col];
+        float gs = t0 + s > 0 ? part[grp][col] : 0.f;
 #pragma unroll
         for (int i = 0; i < kAdamRows; i++)
           gs += x[i];
