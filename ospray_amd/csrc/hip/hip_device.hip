@@ -2831,7 +2831,8 @@ ManagedObject *HipDevice::renderFrame(ManagedObject *fbo, ManagedObject *ro, Man
     F.cancelLatch = latch;
     if (nl > 1) {
       if (latch) // before any lane's passes
-        HIP_CHECK(hpt_fill_u32(latch, 1, 0u, stream)); // fork: the other lanes start after the frame's earlier work
+        HIP_CHECK(hpt_fill_u32(latch, 1, 0u, stream));
+      // fork: the other lanes start after the frame's earlier work
       HIP_CHECK(hipEventRecord(laneEvents[0], stream));
       for (int k = 1; k < nl; k++)
         HIP_CHECK(hipStreamWaitEvent(lanes[k]->stream, laneEvents[0], 0));
@@ -2872,10 +2873,11 @@ ManagedObject *HipDevice::renderFrame(ManagedObject *fbo, ManagedObject *ro, Man
         lastBounce = std::min(F.maxDepth, F.nrcBounce + 1);
       // Shadow stages of bounce b on the lane's side stream, beside the
       // extension of bounce b + 1 (they read and write disjoint path state
-      // and counters; the side stream has its own traversal scratch rows).  The shading of bounce b + 1 (and the free-path
-      // sampling, which shares the paths' volume sampler with the
-      // transmittance estimates) waits for bounce b's resolve, so every
-      // contribution is added in the same order as on one stream.
+      // and counters; the side stream has its own traversal scratch rows).
+      // The shading of bounce b + 1 (and the free-path sampling, which shares
+      // the paths' volume sampler with the transmittance estimates) waits for
+      // bounce b's resolve, so every contribution is added in the same order
+      // as on one stream.
       // Below 2^17 paths a pass the events between the streams cost more than
       // the overlap gives (us a frame, two streams / one: 4 k paths 445 / 402,
       // 16 k 509 / 464, 64 k 600 / 580 and 1184 / 1188, 262 k 796 / 814 and

@@ -663,10 +663,11 @@ __global__ __launch_bounds__(256) void k_volume(DScene S, DPaths P, int qin, int
 // path.  At a smooth vertex it stores the NEE vertex record and appends the
 // vertex's light-sample slots to the NEE sample queue; k_nee evaluates them
 // (NextEventEstimation.ispc:25-160).  The loop runs over whole waves so the
-// appends can scan across the wave.  Every instance holds 3 waves per SIMD:
-// the volume instances (whose transmittance walks would take 215
-// registers) spill the registers of their cold branches instead of
-// dropping to 2 waves.
+// appends can scan across the wave.  Every instance holds 3 waves per SIMD
+// (168 registers): the volume instances (whose transmittance walks would take
+// 215) spill the registers of their cold branches, 208 to 224 B a lane,
+// instead of dropping to 2 waves; the surface instance with the cache spills
+// 16 B.
 template <bool VOL, bool NRC>
 __global__ __launch_bounds__(256, 3) void k_shade(DScene S, DFrame F, DPaths P, int qin)
 {

@@ -622,20 +622,6 @@ __device__ __forceinline__ int tracePop(TraceState &s, uint32_t *lds, uint32_t *
   return v;
 }
 
-// Inner nodes of the speculative while-while traversal: a lane that reaches
-// a leaf keeps it aside (post) and goes on with inner nodes until at most
-// as many lanes still look for a leaf as hold one.  Waiting for the last
-// lane ran 10.8 node steps per call with 18.5 of 64 lanes active on the
-// 1080p terrain (88 % of the traversal's instructions), since a lane that
-// meets its second leaf stands still; leaving as soon as half have one
-// trades some fuller leaf rounds for that.  1920x1080, 4 spp: 26.4 ->
-// 24.9 ms (ratios of searching to holding lanes 1/4, 1/2, 2/3, 1, 3/2, 2, 4:
-// 25.2, 24.7, 24.7, 24.8, 25.1, 25.4, 26.6); never later than that, so a
-// wave with few rays goes on as before.  The exit of an instance
-// (its marker) stops a lane too: traceLeaf gives it the world ray back.  A
-// held instance leaf is entered from the world level, with the next world
-// node pushed below the marker.  Lanes with cur == kTraceDone and no held
-// leaf (finished or idle) only take part in the wave vote.
 // the lanes of the wave for which x holds (__ballot takes an int, which
 // costs two more vector instructions)
 __device__ __forceinline__ unsigned long long waveMask(bool x) { return __builtin_amdgcn_ballot_w64(x); }
@@ -644,6 +630,20 @@ __device__ __forceinline__ unsigned long long waveMask(bool x) { return __builti
 // instance
 __device__ __forceinline__ bool traceHolds(const TraceState &s) { return s.post != 0 || s.cur == kMarker; }
 
+// Inner nodes of the speculative while-while traversal: a lane that reaches
+// a leaf keeps it aside (post) and goes on with inner nodes until at most
+// as many lanes still look for a leaf as hold one.  Waiting for the last
+// lane ran 10.8 node steps per call with 18.5 of 64 lanes active on the
+// 1080p terrain (88 % of the traversal's instructions), since a lane that
+// meets its second leaf stands still; leaving as soon as half have one
+// trades some fuller leaf rounds for that.  1920x1080, 4 spp, whole frames:
+// 26.4 -> 23.9 ms.  (Ratios of searching to holding lanes 1/4, 1/2, 2/3, 1,
+// 3/2, 2, 4, without the maps: 25.2, 24.7, 24.7, 24.8, 25.1, 25.4, 26.6.)
+// Never later than that, so a wave with few rays goes on as before.  The exit
+// of an instance (its marker) stops a lane too: traceLeaf gives it the world
+// ray back.  A held instance leaf is entered from the world level, with the
+// next world node pushed below the marker.  Lanes with cur == kTraceDone and
+// no held leaf (finished or idle) only take part in the wave vote.
 template <int MODE, bool STATS>
 __device__ __forceinline__ void traceDescend(
     TraceState &s, const DScene &S, uint32_t *lds, uint32_t *ovf, TraceStats &st)

@@ -42,9 +42,11 @@ struct BNode4
 };
 static_assert(sizeof(BNode4) == 128, "build node size");
 
-// 4-wide BVH node as the traversal reads it.  The traversal waits on its
-// loads more than it computes (63 % of the wave time, VALU issue 58 %), so a
-// node is as few of them as possible: the children's boxes lie on a grid
+// 4-wide BVH node as the traversal reads it.  Its loads bound the traversal:
+// waves wait for half of their time (49 % of k_extend's wave cycles, 47 % of
+// k_shadow's), and a node step with one more 4-byte load from the same node
+// takes the 1080p kernels 13 and 9 % longer, one with twenty more FMAs 2 %.
+// So a node is as few loads as possible: the children's boxes lie on a grid
 // over the node's own box, plane q of an axis at p + q * s, one byte per
 // plane (byte c = child c) and rounded outwards, four 16-byte loads a lane
 // where float boxes take seven, and twice the nodes in a cache.  1080p

@@ -1,12 +1,14 @@
 """How the traversal kernels deal out their queues changes only which rays
 share a wave.  A queue of at least 64 entries per wave of the grid is taken
-in 64-entry batches by whichever wave asks next; a shorter one (the last
-bounces' few paths) is spread as one batch of ceil(n / waves) entries per
-wave.  With one traversal block per CU (512 waves on 256 CUs: queues of
-32,768 rays or more are batched) the 128x72, 4 spp frame's first bounces
-run batched and its later ones spread; with 64 blocks per CU every queue
-is spread.  Frames rendered at 1, 64 and the default number of blocks per
-CU are equal bit for bit, and equal to the oracle."""
+in 64-entry batches by whichever wave asks next; one of at most 4 entries per
+wave is left to whole waves, a ray each; one in between (the last bounces of a
+large frame) is spread as one batch of ceil(n / waves) entries per wave.  With
+one traversal block per CU (512 waves on 256 CUs) the 36,864 rays of the
+128x72, 4 spp frame's first bounce run batched, its later bounces spread and
+its last ones by whole waves; with the default 12 (6,144 waves) the first
+bounces are spread; with 64 every queue is left to whole waves.  Frames
+rendered at 1, 64 and the default number of blocks per CU are equal bit for
+bit, and equal to the oracle."""
 import numpy as np
 import pytest
 
