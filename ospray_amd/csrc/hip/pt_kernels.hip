@@ -1756,23 +1756,26 @@ size_t hpt_counter_bytes(int bounces) { return 4 * counterWords((size_t)(bounces
 void hpt_at_bounce(HptPaths *P, int bounce) { atBounce(*reinterpret_cast<DPaths *>(P), (size_t)bounce); }
 
 namespace {
-// the paths as the kernels of a bounce that reads extension queue `queue` see them
-DPaths pathsAt(const HptPaths *P, int queue)
+// the paths as the kernels of a bounce that reads extension queue `queue` see
+// them: P's own, or made in `two`
+const DPaths &pathsAt(const HptPaths *P, int queue, DPaths &two)
 {
   const DPaths &p = *reinterpret_cast<const DPaths *>(P);
-  return p.pass ? p : twoQueues(p, queue);
+  return p.pass ? p : (two = twoQueues(p, queue));
 }
 hipError_t launchReset(const HptPaths *P, int queue, int32_t *a, int na, int32_t *b, int nb, int32_t *keep, bool poll,
     hipStream_t s)
 {
-  hipLaunchKernelGGL(k_reset, dim3(1), dim3(256), 0, s, pathsAt(P, queue), a, na, b, nb, keep, poll ? 1 : 0);
+  DPaths two;
+  hipLaunchKernelGGL(k_reset, dim3(1), dim3(256), 0, s, pathsAt(P, queue, two), a, na, b, nb, keep, poll ? 1 : 0);
   return hipGetLastError();
 }
 } // namespace
 
 hipError_t hpt_reset_counters(const HptPaths *P, int keepIndex, hipStream_t s)
 {
-  const DPaths p = pathsAt(P, keepIndex < 0 ? 0 : keepIndex);
+  DPaths two;
+  const DPaths &p = pathsAt(P, keepIndex < 0 ? 0 : keepIndex, two);
   if (reinterpret_cast<const DPaths *>(P)->pass)
     return hipErrorInvalidValue;
   if (keepIndex < 0)
@@ -1782,7 +1785,8 @@ hipError_t hpt_reset_counters(const HptPaths *P, int keepIndex, hipStream_t s)
 
 hipError_t hpt_reset_extension_counters(const HptPaths *P, int keepIndex, hipStream_t s)
 {
-  const DPaths p = pathsAt(P, keepIndex);
+  DPaths two;
+  const DPaths &p = pathsAt(P, keepIndex, two);
   if (reinterpret_cast<const DPaths *>(P)->pass)
     return hipErrorInvalidValue;
   return launchReset(P, keepIndex, p.stage + kCntTies, 1, p.stage + kCntFetchExtend, kXcds * kFetchStride,
@@ -1791,7 +1795,8 @@ hipError_t hpt_reset_extension_counters(const HptPaths *P, int keepIndex, hipStr
 
 hipError_t hpt_reset_append_counters(const HptPaths *P, int keepIndex, hipStream_t s)
 {
-  const DPaths p = pathsAt(P, keepIndex);
+  DPaths two;
+  const DPaths &p = pathsAt(P, keepIndex, two);
   if (reinterpret_cast<const DPaths *>(P)->pass)
     return hipErrorInvalidValue;
   return launchReset(P, keepIndex, p.next, 2, nullptr, 0, nullptr, false, s);
@@ -1799,7 +1804,8 @@ hipError_t hpt_reset_append_counters(const HptPaths *P, int keepIndex, hipStream
 
 hipError_t hpt_reset_shadow_counters(const HptPaths *P, hipStream_t s)
 {
-  const DPaths p = pathsAt(P, 0);
+  DPaths two;
+  const DPaths &p = pathsAt(P, 0, two);
   if (reinterpret_cast<const DPaths *>(P)->pass)
     return hipErrorInvalidValue;
   return launchReset(P, 0, p.stage + kCntShadow, 2, p.stage + kCntFetchShadow, kXcds * kFetchStride, nullptr, false, s);
@@ -1824,14 +1830,16 @@ hipError_t hpt_generate(const HptFrame *F, const HptPaths *P, hipStream_t s)
 {
   const DFrame &f = *reinterpret_cast<const DFrame *>(F);
   const size_t n = (size_t)f.passCount * f.numPixPadded;
-  hipLaunchKernelGGL(k_generate, dim3(gridFor(n, 256, 16384)), dim3(256), 0, s, f, pathsAt(P, 0));
+  DPaths two;
+  hipLaunchKernelGGL(k_generate, dim3(gridFor(n, 256, 16384)), dim3(256), 0, s, f, pathsAt(P, 0, two));
   return hipGetLastError();
 }
 
 hipError_t hpt_extend(const HptScene *S, const HptPaths *P, int queue, int residentBlocks, int stats, hipStream_t s)
 {
   const DScene &sc = *reinterpret_cast<const DScene *>(S);
-  const DPaths p = pathsAt(P, queue);
+  DPaths two;
+  const DPaths &p = pathsAt(P, queue, two);
   if (stats)
     hipLaunchKernelGGL(k_extend<true>, dim3(residentBlocks), dim3(kTraceBlock), 0, s, sc, p, queue);
   else
@@ -1842,7 +1850,8 @@ hipError_t hpt_extend(const HptScene *S, const HptPaths *P, int queue, int resid
 hipError_t hpt_ties(const HptScene *S, const HptPaths *P, int residentBlocks, int stats, hipStream_t s)
 {
   const DScene &sc = *reinterpret_cast<const DScene *>(S);
-  const DPaths p = pathsAt(P, 0);
+  DPaths two;
+  const DPaths &p = pathsAt(P, 0, two);
   if (stats)
     hipLaunchKernelGGL(k_ties<true>, dim3(residentBlocks), dim3(kTraceBlock), 0, s, sc, p);
   else
@@ -1854,7 +1863,8 @@ hipError_t hpt_shade(const HptScene *S, const HptFrame *F, const HptPaths *P, in
 {
   const DScene &sc = *reinterpret_cast<const DScene *>(S);
   const DFrame &f = *reinterpret_cast<const DFrame *>(F);
-  const DPaths p = pathsAt(P, queue);
+  DPaths two;
+  const DPaths &p = pathsAt(P, queue, two);
   // the volume variant carries the sampler and transmittance code (more
   // registers), the cache variant the cache records (the caller passes a
   // frame with nrcBounce -1 for the other bounces); surface-only worlds run
@@ -1902,8 +1912,9 @@ hipError_t hpt_nrc_targets(const HptPaths *P, int n, float *target3, hipStream_t
 
 hipError_t hpt_nee(const HptScene *S, const HptFrame *F, const HptPaths *P, int queue, int blocks, hipStream_t s)
 {
+  DPaths two;
   hipLaunchKernelGGL(k_nee, dim3(blocks), dim3(kNeeBlock), 0, s, *reinterpret_cast<const DScene *>(S),
-      *reinterpret_cast<const DFrame *>(F), pathsAt(P, queue), queue);
+      *reinterpret_cast<const DFrame *>(F), pathsAt(P, queue, two), queue);
   return hipGetLastError();
 }
 
@@ -1912,7 +1923,8 @@ hipError_t hpt_shadow(
 {
   const DScene &sc = *reinterpret_cast<const DScene *>(S);
   const DFrame &f = *reinterpret_cast<const DFrame *>(F);
-  const DPaths p = pathsAt(P, 0);
+  DPaths two;
+  const DPaths &p = pathsAt(P, 0, two);
   if (stats) {
     hipLaunchKernelGGL(k_shadow<true>, dim3(residentBlocks), dim3(kTraceBlock), 0, s, sc, f, p);
   } else {
@@ -1926,7 +1938,8 @@ hipError_t hpt_shadow_trans(
 {
   const DScene &sc = *reinterpret_cast<const DScene *>(S);
   const DFrame &f = *reinterpret_cast<const DFrame *>(F);
-  const DPaths p = pathsAt(P, 0);
+  DPaths two;
+  const DPaths &p = pathsAt(P, 0, two);
   if (stats)
     hipLaunchKernelGGL(k_shadow_trans<true>, dim3(residentBlocks), dim3(kTraceBlock), 0, s, sc, f, p);
   else
@@ -1936,8 +1949,9 @@ hipError_t hpt_shadow_trans(
 
 hipError_t hpt_volume(const HptScene *S, const HptPaths *P, int queue, int blocks, int stats, hipStream_t s)
 {
+  DPaths two;
   hipLaunchKernelGGL(k_volume, dim3(blocks), dim3(256), 0, s, *reinterpret_cast<const DScene *>(S),
-      pathsAt(P, queue), queue, stats);
+      pathsAt(P, queue, two), queue, stats);
   return hipGetLastError();
 }
 
@@ -1945,7 +1959,8 @@ hipError_t hpt_resolve(const HptScene *S, const HptFrame *F, const HptPaths *P, 
 {
   const DScene &sc = *reinterpret_cast<const DScene *>(S);
   const DFrame &f = *reinterpret_cast<const DFrame *>(F);
-  const DPaths p = pathsAt(P, queue);
+  DPaths two;
+  const DPaths &p = pathsAt(P, queue, two);
   if (sc.numVolInsts > 0)
     hipLaunchKernelGGL(k_resolve<true>, dim3(blocks), dim3(256), 0, s, sc, f, p, queue);
   else
