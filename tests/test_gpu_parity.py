@@ -319,9 +319,10 @@ def _set_device_params(**kv):
 def test_pass_pipelining_bit_exact(hip_device, lanes, budget_mb):
     # a frame's passes alternate over lanes (the accumulation stays in
     # sample order): every channel equals the one-lane frames and the
-    # oracle; a 1 MB path budget gives one sample per pass, more passes
-    # than lanes
-    sc = scenes.c0(40, 36, spp=5, max_path_length=4)
+    # oracle; the smallest path budget (64 MB, some 120,000 slots) gives one
+    # sample per pass of the larger frame, more passes than lanes
+    w, h = (40, 36) if budget_mb > 64 else (264, 240)
+    sc = scenes.c0(w, h, spp=5, max_path_length=4)
     images = {}
     try:
         for fl in (1, lanes):

@@ -96,21 +96,22 @@ def test_transparency_queue_of_any_length(hip_device, bpc):
 @pytest.mark.parametrize("depths", [(2, 30, 2), (0, 1, 40)])
 def test_counters_follow_the_path_length(hip_device, depths):
     """Each bounce has counters of its own, sized for the longest path so
-    far: frames of growing and shrinking path length, one and several passes
-    a frame, equal the oracle's."""
+    far: frames of growing and shrinking path length, in one pass and in two
+    (the smallest path budget, 64 MB, holds two samples of the larger frame),
+    equal the oracle's."""
     L = K.lib()
     dev = L.ospGetCurrentDevice()
-    for budget in (16384, 64):
+    for budget, w, h in ((16384, 24, 16), (64, 256, 192)):
         A.set_device_param(dev, "pathBudgetMB", budget)
         L.ospDeviceCommit(dev)
         try:
             for d in depths:
-                sc = scenes.c0(24, 16, spp=3, max_path_length=d)
+                sc = scenes.c0(w, h, spp=3, max_path_length=d)
                 s = scenes.to_ospray(sc)
-                fb = A.framebuffer(24, 16, K.OSP_FB_RGBA32F, CH)
+                fb = A.framebuffer(w, h, K.OSP_FB_RGBA32F, CH)
                 A.render(fb, s.renderer, s.camera, s.world)
                 ofb, _, _ = orc.render_scene(sc, frames=1, fmt=K.OSP_FB_RGBA32F, channels=CH)
-                assert np.array_equal(A.map_color(fb, 24, 16, K.OSP_FB_RGBA32F), ofb.channel(K.OSP_FB_COLOR)), (budget, d)
+                assert np.array_equal(A.map_color(fb, w, h, K.OSP_FB_RGBA32F), ofb.channel(K.OSP_FB_COLOR)), (budget, d)
         finally:
             A.set_device_param(dev, "pathBudgetMB", 16384)
             L.ospDeviceCommit(dev)
