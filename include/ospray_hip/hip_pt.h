@@ -34,9 +34,10 @@ typedef struct HptPaths HptPaths; /* wavefront path state, queues and counters *
  * hpt_counter_bytes(bounces) bytes of device memory.  hpt_begin_pass clears
  * them for a pass of `bounces` bounces and polls the frame's cancellation,
  * whose latch firstPass != 0 clears before.  hpt_at_bounce (host only) points
- * P at the counters of bounce b (from 0) for the calls that follow.  Stages of
- * bounce b may run on a second stream beside the extension of bounce b+1:
- * they share no counter. */
+ * P at the counters of bounce b (from 0) for the calls that follow, and leaves
+ * P as it is where P->pass is null or b is negative.  Stages of bounce b may
+ * run on a second stream beside the extension of bounce b+1: they share no
+ * counter. */
 HPT_API size_t hpt_counter_bytes(int bounces);
 HPT_API hipError_t hpt_begin_pass(const HptPaths *P, int bounces, int firstPass, hipStream_t s);
 HPT_API void hpt_at_bounce(HptPaths *P, int bounce);

@@ -1753,7 +1753,12 @@ hipError_t hpt_begin_pass(const HptPaths *P, int bounces, int firstPass, hipStre
 
 size_t hpt_counter_bytes(int bounces) { return 4 * counterWords((size_t)(bounces < 0 ? 0 : bounces)); }
 
-void hpt_at_bounce(HptPaths *P, int bounce) { atBounce(*reinterpret_cast<DPaths *>(P), (size_t)bounce); }
+void hpt_at_bounce(HptPaths *P, int bounce)
+{
+  DPaths &p = *reinterpret_cast<DPaths *>(P);
+  if (p.pass && bounce >= 0)
+    atBounce(p, (size_t)bounce);
+}
 
 namespace {
 // the paths as the kernels of a bounce that reads extension queue `queue` see

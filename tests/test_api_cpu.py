@@ -58,6 +58,21 @@ def test_stage_entry_points_stay():
         assert "HPT_API hipError_t " + decl + ";" in text, decl
 
 
+def test_at_bounce_needs_counters_per_bounce():
+    """hpt_at_bounce returns nothing that could say an error: without P->pass,
+    or before the first bounce, P keeps the counters it has."""
+    lib = C.CDLL(os.path.join(K.LIBDIR, "libospray_module_hip.so"), mode=C.RTLD_GLOBAL)
+    state = (C.c_uint64 * 512)()  # no smaller than the path state
+    lib.hpt_at_bounce(state, 3)
+    assert not any(state)
+    for i in range(len(state)):
+        state[i] = 1 << 40
+    lib.hpt_at_bounce(state, -1)
+    assert all(v == 1 << 40 for v in state)
+    lib.hpt_at_bounce(state, 1)  # the bounce's counters, its stages' and the next bounce's
+    assert sum(v != 1 << 40 for v in state) == 3
+
+
 def test_module_version_check():
     lib = C.CDLL(os.path.join(K.LIBDIR, "libospray_module_hip.so"), mode=C.RTLD_GLOBAL)
     init = lib.ospray_module_init_hip
