@@ -2879,9 +2879,11 @@ ManagedObject *HipDevice::renderFrame(ManagedObject *fbo, ManagedObject *ro, Man
       // bounce b's resolve, so every contribution is added in the same order
       // as on one stream.
       // Below 2^17 paths a pass the events between the streams cost more than
-      // the overlap gives (us a frame, two streams / one: 4 k paths 445 / 402,
-      // 16 k 509 / 464, 64 k 600 / 580 and 1184 / 1188, 262 k 796 / 814 and
-      // 1727 / 1815, volume scenes 16 k 1945 / 1850, 256 k 2766 / 2830).
+      // the overlap gives.  us a frame, two streams / one, of 64 spheres: 4 k
+      // paths 445 / 402, 16 k 509 / 464, 131 k 606 / 558, 262 k 782 / 759,
+      // 524 k 907 / 891, 1 M 1420 / 1452; of a terrain: 64 k 1184 / 1188, 131 k
+      // 1321 / 1303, 262 k 1757 / 1824, 1 M 3117 / 3297, 2 M 7605 / 8095; of a
+      // volume: 16 k 1945 / 1850, 131 k 2207 / 2189, 262 k 2774 / 2836.
       const bool overlap = overlapShadow && nl == 1 && !capturing && !inBatch && F.numFirstLightSamples > 0
           && (size_t)F.passCount * F.numPixPadded >= ((size_t)1 << 17);
       const hipStream_t side = overlap ? ensureSide(*lane) : nullptr;
